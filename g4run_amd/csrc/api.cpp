@@ -473,9 +473,7 @@ extern "C" int g4h_matmul_describe(const g4h_tensor *W, int nb, int path, char *
     if (path == 2) {
         if (!mfma_capable(W)) return fail(G4H_ERR_TYPE, "g4h_matmul_describe: the matrix-core path takes q8_0 / q4_0 / q4_K / q6_K weights and f16 / bf16 rows of whole 16-column steps");
         if (mmk_capable(W->type)) mmk_describe(*W, nb, buf, len);
-        else if (is_float(W->type))
-            snprintf(buf, len, "k_mm_float<%s> grid=%lldx%d block=512 (matrix cores, 32x32 tiles, 8 waves split the columns)",
-                     type_name(W->type), (long long)((W->nrows + 31) / 32), (nb + 31) / 32);
+        else if (is_float(W->type)) mmf_describe(W->type, W->nrows, nb, buf, len);
         else mm_describe(*W, nb, buf, len);
         return G4H_OK;
     }

@@ -9,7 +9,7 @@
 // lanes.  The fp32 order differs from the CPU's 8-lane AVX2 order (within the
 // path's fp32 tolerance) but does not depend on the token count, so a batch
 // gives every token the single-token bits.
-#include <type_traits>
+#include <cstdio>
 
 #include "common.h"
 #include "kernels.h"
@@ -139,111 +139,238 @@ hipError_t launch_gemv_float_x(int wtype, const uint8_t *W, size_t ws, int64_t n
 }
 
 // Prompt batches on the matrix cores (g4h_matmul path 2): Y[t][r] = sum_k
-// W[r][k] a[t][k] for 32-token x 32-row tiles, one v_mfma_f32_32x32x16_f16 /
-// _bf16 per 16 columns.  The operands are the GEMV family's: f16 weights
+// W[r][k] a[t][k], one v_mfma_f32_16x16x32_f16 / _bf16 per 32 columns of a
+// 16-token x 16-row tile.  The operands are the GEMV family's: f16 weights
 // against f16-rounded activations, bf16 weights against bf16-rounded ones
 // (prep_act's AC_F16 / AC_BF16, model.c:163-180), so every product is exact
 // in fp32 (11 x 11 or 8 x 8 significant bits) and only the fp32 order of the
 // sums differs from the CPU's and from the GEMV family's (within the path's
-// tolerance).  The MMF_W waves of a workgroup split the 16-column steps (wave
-// w takes steps w, w + MMF_W, ..., each chained into its accumulator in
-// increasing order) and the waves' tiles are added in wave order through
-// LDS: a token's result does not depend on the batch size.  Operand layout:
-// lane l holds A[l % 32][8 (l / 32) .. + 7] and B[l % 32][8 (l / 32) .. + 7];
-// C[i][j] with j = l % 32 (weight row), i = 8 (r / 4) + 4 (l / 32) + r % 4.
+// tolerance).  A workgroup owns MT x NT such tiles; its MMF_W waves split the
+// 64-column chunks (wave w takes chunks w, w + MMF_W, ..., each chained into
+// its accumulators in increasing order, a last partial chunk included) and
+// the waves' tiles are added in wave order through LDS: a token's result
+// depends neither on the batch size nor on MT and NT.
+//
+// What bounds it: the CU's L1 serves one 64-byte access per clock, and lanes
+// reading different rows are one access each.  An MFMA operand has adjacent
+// lanes in different rows, so loading it straight from memory costs 57
+// accesses per 1 KB instruction (measured).  Here adjacent lanes load adjacent
+// 16 bytes of one row, fp32 activations are rounded on the way, and each wave
+// turns its own chunk into operands through LDS of its own (no barrier), the
+// next chunk's loads in flight meanwhile.  LDS rows of 128 bytes, the 16-byte
+// columns of row r at column ^ (r & 7).  Measured against operands loaded
+// straight from memory for 32 x 32 tiles (fp32 tokens, us): f16 4096 x 4096 at
+// 64 / 201 / 512 tokens 29.4 / 83.0 / 177.9 -> 15.9 / 23.9 / 46.7 (141, 282 and
+// 368 TFLOP/s), f16 256 x 2048 at 64 tokens 13.4 -> 5.6, bf16 2560 x 10240 at
+// 64 / 300 tokens 74.8 / 212.8 -> 33.6 / 51.5.
+// Operand layout: lane l holds A[l % 16][8 (l / 16) .. + 7] and
+// B[l % 16][8 (l / 16) .. + 7]; C[i][j] with j = l % 16 (weight row), i = 4
+// (l / 16) + r (token).
 typedef _Float16 mf_v8h __attribute__((ext_vector_type(8)));
 typedef __bf16 mf_v8bf __attribute__((ext_vector_type(8)));
-typedef float mf_v16f __attribute__((ext_vector_type(16)));
+typedef float mf_v4f __attribute__((ext_vector_type(4)));
 
 constexpr int MMF_W = 8;              // waves per workgroup
 
-// XF: fp32 token rows (row stride `as` bytes) rounded on load with
-// k_act_float's arithmetic; else prepared rows (f16 for F16, bf16-rounded
-// fp32 for BF16)
-template <int WT, bool XF>
-__global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restrict__ W, size_t ws, int64_t nrows, int64_t ncols,
-                                                         const uint8_t *__restrict__ act, size_t as, int M, float *__restrict__ Y) {
-    __shared__ float part[MMF_W - 1][16][64];
-    constexpr bool A32 = XF || WT == BF16;                          // activation rows of fp32
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x) >> 6;
-    const int li = lane & 31, kh = lane >> 5;
-    const int64_t n0 = (int64_t)blockIdx.x * 32;
-    const int m0 = (int)blockIdx.y * 32;
-    const int64_t row = min(n0 + li, nrows - 1);
-    const int tok = min(m0 + li, M - 1);
-    const uint8_t *wr = W + (size_t)row * ws + 16 * kh;
-    const uint8_t *ar = act + (size_t)tok * as + (A32 ? 32 : 16) * kh;
-    const int nk = (int)(ncols >> 4);
-    const int nj = (nk - wave + MMF_W - 1) / MMF_W;                 // this wave's steps (uniform)
-    struct Op {
-        uint4 w, a0, a1;
-    };
-    auto load = [&](int j) __attribute__((always_inline)) -> Op {
-        const size_t sk = (size_t)(wave + MMF_W * j);
-        Op o;
-        o.w = *(const uint4 *)(wr + 32 * sk);
-        o.a0 = *(const uint4 *)(ar + (A32 ? 64 : 32) * sk);
-        if constexpr (A32) o.a1 = *(const uint4 *)(ar + 64 * sk + 16);
-        return o;
-    };
-    mf_v16f acc = {};
-    auto mac = [&](const Op &o) __attribute__((always_inline)) {
-        uint32_t ab[4];
-        if constexpr (A32) {
-            const float v[8] = {__uint_as_float(o.a0.x), __uint_as_float(o.a0.y), __uint_as_float(o.a0.z), __uint_as_float(o.a0.w),
-                                __uint_as_float(o.a1.x), __uint_as_float(o.a1.y), __uint_as_float(o.a1.z), __uint_as_float(o.a1.w)};
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                uint32_t lo, hi;
-                if constexpr (WT == F16) {
-                    lo = f2h(v[2 * k]), hi = f2h(v[2 * k + 1]);
-                } else if constexpr (XF) {
-                    lo = f2bf(v[2 * k]), hi = f2bf(v[2 * k + 1]);
-                } else {                                            // already bf16-rounded: the high halves
-                    lo = __float_as_uint(v[2 * k]) >> 16, hi = __float_as_uint(v[2 * k + 1]) >> 16;
-                }
-                ab[k] = lo | (hi << 16);
-            }
-        } else {
-            ab[0] = o.a0.x, ab[1] = o.a0.y, ab[2] = o.a0.z, ab[3] = o.a0.w;
-        }
-        const uint4 av = make_uint4(ab[0], ab[1], ab[2], ab[3]);
-        if constexpr (WT == F16)
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mf_v8h, av), __builtin_bit_cast(mf_v8h, o.w), acc, 0, 0, 0);
-        else
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mf_v8bf, av), __builtin_bit_cast(mf_v8bf, o.w), acc, 0, 0,
-                                                          0);
-    };
-    // straight-line chunks of steps whose loads all go out first
-    auto chunk = [&](auto Cc, int j0) __attribute__((always_inline)) {
-        constexpr int C = decltype(Cc)::value;
-        Op ops[C];
-#pragma unroll
-        for (int k = 0; k < C; k++) ops[k] = load(j0 + k);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int k = 0; k < C; k++) mac(ops[k]);
-    };
-    int j0 = 0;
-    for (; j0 + 4 <= nj; j0 += 4) chunk(std::integral_constant<int, 4>{}, j0);
-    if (nj - j0 >= 2) chunk(std::integral_constant<int, 2>{}, j0), j0 += 2;
-    if (nj - j0 >= 1) chunk(std::integral_constant<int, 1>{}, j0);
+// two fp32 activations rounded with k_act_float's arithmetic by the packed
+// conversion instructions (round to nearest even; bf16-rounded rows keep their
+// values)
+template <int WT>
+__device__ __forceinline__ uint32_t mmf_round2(uint32_t x, uint32_t y) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    const v2f v = {__uint_as_float(x), __uint_as_float(y)};
+    if constexpr (WT == F16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2h));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2bf));
+}
 
-    if (wave > 0) {
+// A32: activation rows of fp32 (row stride `as` bytes), rounded on the way to
+// LDS; else f16 rows.  Workgroup b runs on XCD b % 8: the token tiles of one
+// row tile go to one XCD, consecutively, and find its weights in that XCD's L2.
+template <int WT, bool A32, int MT, int NT>
+__global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restrict__ W, size_t ws, int64_t nrows, int64_t ncols,
+                                                         const uint8_t *__restrict__ act, size_t as, int M, float *__restrict__ Y,
+                                                         int ntok) {
+    constexpr int AL = A32 ? 4 * MT : 2 * MT, WL = 2 * NT;          // 16-byte loads per lane and chunk
+    // chunks per stage: 40 to 96 registers of loads, at most 16 KB of LDS per wave
+    constexpr int CR = AL + WL >= 12 ? 1 : AL + WL >= 8 ? 2 : 4, CH = CR * (MT + NT) <= 8 ? CR : CR / 2;
+    constexpr int LW = CH * (MT + NT) * 2048;                       // LDS bytes per wave
+    constexpr int PW = MT * NT * 1024;                              // partial tiles per wave
+    __shared__ __align__(16) uint8_t lds[MMF_W * (LW > PW ? LW : PW)];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x) >> 6;
+    const int li = lane & 15, kg = lane >> 4;
+    const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
+    const int64_t n0 = ((int64_t)(l / ntok) * 8 + x) * (16 * NT);
+    const int m0 = (l % ntok) * (16 * MT);
+    if (n0 >= nrows) return;                                        // uniform over the workgroup
+    uint8_t *sl = lds + wave * LW;
+    // 16-byte loads: eight lanes per 128-byte row of W (and of f16
+    // activations), sixteen per 256-byte fp32 row
+    const int wr = lane >> 3, wc = lane & 7, ar = A32 ? lane >> 4 : wr, ac = A32 ? lane & 15 : wc;
+    constexpr int AQ = A32 ? 4 : 8;                                 // activation rows per load
+    const uint8_t *wp[WL], *ap[AL];
 #pragma unroll
-        for (int r = 0; r < 16; r++) part[wave - 1][r][lane] = acc[r];
+    for (int q = 0; q < WL; q++) wp[q] = W + (size_t)min(n0 + 8 * q + wr, nrows - 1) * ws + 16 * wc;
+#pragma unroll
+    for (int q = 0; q < AL; q++) ap[q] = act + (size_t)min(m0 + AQ * q + ar, M - 1) * as + 16 * ac;
+    const int nc = (int)(ncols >> 6);                               // whole chunks
+    const int nj = (nc - wave + MMF_W - 1) / MMF_W;                 // this wave's (uniform)
+    struct Stage {
+        uint4 w[CH][WL], a[CH][AL];
+    };
+    Stage S;
+    auto load = [&](int j0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const size_t k = (size_t)(wave + MMF_W * min(j0 + c, nj - 1));
+#pragma unroll
+            for (int q = 0; q < WL; q++) S.w[c][q] = *(const uint4 *)(wp[q] + 128 * k);
+#pragma unroll
+            for (int q = 0; q < AL; q++) S.a[c][q] = *(const uint4 *)(ap[q] + (A32 ? 256 : 128) * k);
+        }
+    };
+    auto put = [&](int c) __attribute__((always_inline)) {          // chunk c of the stage into LDS
+        uint8_t *la = sl + c * (MT + NT) * 2048, *lw = la + MT * 2048;
+#pragma unroll
+        for (int q = 0; q < WL; q++) *(uint4 *)(lw + (8 * q + wr) * 128 + 16 * (wc ^ wr)) = S.w[c][q];
+#pragma unroll
+        for (int q = 0; q < AL; q++) {
+            const uint4 v = S.a[c][q];
+            const int r = AQ * q + ar;
+            if constexpr (A32)
+                *(uint2 *)(la + r * 128 + 16 * ((ac >> 1) ^ (r & 7)) + 8 * (ac & 1)) =
+                    make_uint2(mmf_round2<WT>(v.x, v.y), mmf_round2<WT>(v.z, v.w));
+            else
+                *(uint4 *)(la + r * 128 + 16 * (ac ^ (r & 7))) = v;
+        }
+    };
+    mf_v4f acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int n = 0; n < NT; n++) acc[m][n] = mf_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    auto mul = [&](int c) __attribute__((always_inline)) {
+        const uint8_t *la = sl + c * (MT + NT) * 2048 + li * 128, *lw = la + MT * 2048;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int o = 16 * ((4 * h + kg) ^ (li & 7));
+            uint4 a[MT], w[NT];
+#pragma unroll
+            for (int m = 0; m < MT; m++) a[m] = *(const uint4 *)(la + 2048 * m + o);
+#pragma unroll
+            for (int n = 0; n < NT; n++) w[n] = *(const uint4 *)(lw + 2048 * n + o);
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    if constexpr (WT == F16)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mf_v8h, a[m]), __builtin_bit_cast(mf_v8h, w[n]),
+                                                                           acc[m][n], 0, 0, 0);
+                    else
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mf_v8bf, a[m]),
+                                                                            __builtin_bit_cast(mf_v8bf, w[n]), acc[m][n], 0, 0, 0);
+                }
+        }
+    };
+    // a wave's LDS accesses complete in order; the empty asms keep the
+    // compiler from moving any access across a hand-over
+    if (nj > 0) {
+        load(0);
+        for (int j0 = 0; j0 < nj; j0 += CH) {
+            const int left = nj - j0;                               // uniform
+#pragma unroll
+            for (int c = 0; c < CH; c++) put(c);
+            asm volatile("" ::: "memory");
+            load(j0 + CH);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int c = 0; c < CH; c++)
+                if (c < left) mul(c);
+            asm volatile("" ::: "memory");
+        }
+    }
+    // a last chunk of ncols % 64 columns, zeros past them
+    if ((ncols & 63) && wave == nc % MMF_W) {                       // uniform
+        const int lw = (int)(ncols & 63) / 8, la = A32 ? 2 * lw : lw;   // 16-byte columns
+        const size_t k = nc;
+        const uint4 z = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < WL; q++) {
+            S.w[0][q] = *(const uint4 *)(wp[q] + 128 * k - 16 * (wc < lw ? 0 : wc));   // past them the chunk's first column
+            if (wc >= lw) S.w[0][q] = z;
+        }
+#pragma unroll
+        for (int q = 0; q < AL; q++) {
+            S.a[0][q] = *(const uint4 *)(ap[q] + (A32 ? 256 : 128) * k - 16 * (ac < la ? 0 : ac));
+            if (ac >= la) S.a[0][q] = z;
+        }
+        put(0);
+        asm volatile("" ::: "memory");
+        mul(0);
     }
     __syncthreads();
-    if (wave > 0) return;
-    const int64_t n = n0 + li;
+    float *part = (float *)lds;                                     // [wave][register][lane]
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        float o = acc[r];
+    for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int w = 1; w < MMF_W; w++) o += part[w - 1][r][lane];
-        const int m = m0 + 8 * (r >> 2) + 4 * kh + (r & 3);
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) part[(wave * MT * NT * 4 + (m * NT + n) * 4 + r) * 64 + lane] = acc[m][n][r];
+    __syncthreads();
+    // the waves' tiles in wave order; wave w stores registers w, w + 8, ..
+    for (int u = wave; u < MT * NT * 4; u += MMF_W) {
+        float o = part[u * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < MMF_W; w++) o += part[(w * MT * NT * 4 + u) * 64 + lane];
+        const int m = m0 + 16 * (u / (4 * NT)) + 4 * kg + (u & 3);
+        const int64_t n = n0 + 16 * ((u >> 2) % NT) + li;
         if (m < M && n < nrows) Y[(size_t)m * nrows + n] = o;
     }
+}
+
+// Tiles of a call: the shape with the least L1 traffic per CU, rounds of
+// workgroups x the bytes a workgroup loads per column (fp32 activation rows 4,
+// f16 rows and weights 2 each).  Measured with fp32 activations (us): f16 4096
+// x 4096 at 64 tokens 2 x 2 15.9, 4 x 1 21.0, 2 x 4 20.2; at 128 tokens 2 x 4
+// 19.0, 4 x 2 22.9; at 201 tokens 4 x 4 25.1, 2 x 4 32.0, 4 x 2 36.2.
+static void mmf_tiles(bool a32, int64_t nrows, int M, int &mt, int &nt, int &ntok, int64_t &grid) {
+    const int tm = (M + 15) / 16;
+    const int64_t tn = (nrows + 15) / 16;
+    int64_t best = INT64_MAX;
+    for (int m = tm > 2 ? 4 : tm; m >= 1; m >>= 1)
+        for (int n = 4; n >= 1; n >>= 1) {
+            const int64_t cost = ((tm + m - 1) / m * ((tn + n - 1) / n) + 255) / 256 * ((a32 ? 2 : 1) * m + n);
+            if (cost < best) best = cost, mt = m, nt = n;
+        }
+    ntok = (tm + mt - 1) / mt;
+    grid = ((tn + nt - 1) / nt + 7) / 8 * 8 * ntok;
+}
+
+void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len) {
+    int mt, nt, ntok;
+    int64_t grid;
+    mmf_tiles(true, nrows, M, mt, nt, ntok, grid);
+    snprintf(buf, len, "k_mm_float<%s,mt=%d,nt=%d> grid=%lld block=%d (matrix cores, 16x16 tiles, %d waves split the columns)",
+             wtype == F16 ? "f16" : "bf16", mt, nt, (long long)grid, 64 * MMF_W, MMF_W);
+}
+
+template <int WT, bool A32>
+static hipError_t mmf_go(const uint8_t *W, size_t ws, int64_t nrows, int64_t ncols, const uint8_t *a, size_t ab, int M, float *Y,
+                         hipStream_t s) {
+    int mt, nt, ntok;
+    int64_t grid;
+    mmf_tiles(A32, nrows, M, mt, nt, ntok, grid);
+    if (grid > 0x7fffffff) return hipErrorInvalidValue;
+#define G4_MMF(MT_, NT_)                                                                                                       \
+    if (mt == MT_ && nt == NT_) {                                                                                              \
+        hipLaunchKernelGGL((k_mm_float<WT, A32, MT_, NT_>), dim3((unsigned)grid), dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, \
+                           M, Y, ntok);                                                                                        \
+        return hipGetLastError();                                                                                              \
+    }
+    G4_MMF(1, 1) G4_MMF(1, 2) G4_MMF(1, 4) G4_MMF(2, 1) G4_MMF(2, 2) G4_MMF(2, 4) G4_MMF(4, 1) G4_MMF(4, 2) G4_MMF(4, 4)
+#undef G4_MMF
+    return hipErrorInvalidValue;
 }
 
 // M tokens of f16 / bf16 weight rows (ws bytes apart, ncols % 16 == 0) on the
@@ -254,17 +381,11 @@ hipError_t launch_mm_float(int wtype, const uint8_t *W, size_t ws, int64_t nrows
     if ((wtype != F16 && wtype != BF16) || ncols % 16 || ws % 16 || (uintptr_t)W % 16 || M < 1 || (x == nullptr) == (act == nullptr))
         return hipErrorInvalidValue;
     if (x ? ((uintptr_t)x % 16 || xs % 4) : ((uintptr_t)act % 16 || as % 16)) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((nrows + 31) / 32), (unsigned)((M + 31) / 32));
     const uint8_t *a = x ? (const uint8_t *)x : act;
     const size_t ab = x ? xs * 4 : as;
-    if (wtype == F16) {
-        if (x) hipLaunchKernelGGL((k_mm_float<F16, true>), grid, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y);
-        else hipLaunchKernelGGL((k_mm_float<F16, false>), grid, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y);
-    } else {
-        if (x) hipLaunchKernelGGL((k_mm_float<BF16, true>), grid, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y);
-        else hipLaunchKernelGGL((k_mm_float<BF16, false>), grid, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y);
-    }
-    return hipGetLastError();
+    // prepared bf16 rows are bf16-rounded fp32: rounding them again keeps them
+    if (wtype == BF16) return mmf_go<BF16, true>(W, ws, nrows, ncols, a, ab, M, Y, s);
+    return x ? mmf_go<F16, true>(W, ws, nrows, ncols, a, ab, M, Y, s) : mmf_go<F16, false>(W, ws, nrows, ncols, a, ab, M, Y, s);
 }
 
 hipError_t launch_act_float(int wtype, const float *x, size_t xs, int64_t ncols, int nb, uint8_t *out, size_t os, hipStream_t s) {

@@ -238,6 +238,7 @@ hipError_t launch_mm_few_ready(const g4h_tensor &W, const FewAct &a, int M, floa
 // weights against GGUF q8_K activation rows at `stride` bytes
 bool mmk_capable(int type);
 void mmk_describe(const g4h_tensor &W, int M, char *buf, size_t len);
+void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len);
 hipError_t launch_matmul_mfma_k(const g4h_tensor &W, const uint8_t *act, size_t stride, int M, float *Y, hipStream_t s);
 
 // k_attn.hip

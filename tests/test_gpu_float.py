@@ -158,3 +158,34 @@ def test_matrix_cores_token_results_independent_of_batch(gpu, oracle, name, wt):
         assert np.array_equal(bits(auto), bits(full[:9]))
     finally:
         t.free()
+
+
+@pytest.mark.parametrize("name,wt", FLOAT)
+@pytest.mark.parametrize("rows,cols", [(4096, 112), (2048, 576), (1000, 96), (257, 1072)])
+def test_matrix_cores_tile_shapes_same_bits(gpu, oracle, name, wt, rows, cols):
+    """k_mm_float's tile shape follows the row and token counts; every shape
+    gives a token the same bits (compared with the largest batch), from fp32
+    and from prepared rows, also with columns that leave a partial 64-column
+    chunk (48, 32 or 16 of them), rows and tokens off the 16-row tiles, and
+    activations that round to subnormal, infinite or zero values."""
+    from g4run_amd import synth
+    w = _weights(wt, rows, cols, seed=rows + cols)
+    x = synth.activations(512, cols, seed=cols)
+    x[3, :6] = [0.0, -0.0, 1e-30, -3e-8, -2.5e-5, 1.00048828125]
+    x[5, 7] = 70000.0                                       # infinite as f16
+    t = gpu.Tensor.from_rows(wt, w, cols)
+    try:
+        act = oracle.prep_act(wt, x)
+        full = gpu_matmul(gpu, t, x=x, nb=512, path=2)
+        ref = oracle_matmul(oracle, wt, w, x[:128])
+        fin = np.isfinite(ref)
+        assert np.array_equal(fin, np.isfinite(full[:128]))
+        assert_close(np.where(fin, full[:128], 0), np.where(fin, ref, 0), f"{name} {rows}x{cols}")
+        shapes = set()
+        for m in (1, 9, 17, 33, 64, 65, 100, 201, 300):
+            shapes.add(gpu.matmul_describe(t, m, 2).split(" ")[0])
+            for part in (gpu_matmul(gpu, t, x=x[:m].copy(), nb=m, path=2), gpu_matmul(gpu, t, act=act[:m].copy(), nb=m, path=2)):
+                assert np.array_equal(bits(part), bits(full[:m])), f"{name} {rows}x{cols} M={m}"
+        assert len(shapes) >= 2, shapes
+    finally:
+        t.free()
