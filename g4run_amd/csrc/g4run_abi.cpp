@@ -276,9 +276,9 @@ extern "C" int g4_sample(g4_sampler *s, float *logits) {
         return -1;
     }
     const int nv = s->n_vocab;
-    const size_t img = al256(sampler_dev_bytes(0) + (size_t)s->n_ban * sizeof(int));
-    const size_t o_l = img, o_o = o_l + al256((size_t)nv * 4);
-    uint8_t *d = stage(o_o + 256);
+    const size_t img = al256(sizeof(SamplerDev) + (size_t)s->n_ban * sizeof(int));
+    const size_t o_l = img, o_o = o_l + al256((size_t)nv * 4), o_g = o_o + 256;
+    uint8_t *d = stage(o_g + SAMPLER_GROUPS * sizeof(uint32_t));
     if (!d) {
         report("g4_sample");
         return -1;
@@ -305,7 +305,7 @@ extern "C" int g4_sample(g4_sampler *s, float *logits) {
     SamplerDev *dS = reinterpret_cast<SamplerDev *>(d);
     int id = -1;
     const bool ok = !g4h_memcpy_h2d(d, h.data(), img, st) && !g4h_memcpy_h2d(d + o_l, logits, (size_t)nv * 4, st) &&
-                    launch_sample(dS, nv, (float *)(d + o_l), (int *)(d + o_o), 0, nullptr, 0, (hipStream_t)st) ==
+                    launch_sample(dS, nv, (float *)(d + o_l), (int *)(d + o_o), 0, nullptr, 0, (uint32_t *)(d + o_g), (hipStream_t)st) ==
                         hipSuccess &&
                     !g4h_memcpy_d2h(logits, d + o_l, (size_t)nv * 4, st) && !g4h_memcpy_d2h(&id, d + o_o, sizeof id, st) &&
                     !g4h_memcpy_d2h(s->rng, dS->rng, sizeof s->rng, st);

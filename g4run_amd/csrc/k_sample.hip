@@ -1,6 +1,18 @@
-// k_sample.hip -- the sampling chain of sampler.c:74-210 on the GPU: one
-// workgroup of 1024 threads draws one id from a logits row resident in HBM,
-// so a decode step can sample without a host round trip.
+// k_sample.hip -- the sampling chain of sampler.c:74-210 on the GPU: one id is
+// drawn from a logits row resident in HBM, so a decode step can sample without
+// a host round trip.
+//
+// Large rows (from GRP_MIN_VOCAB ids) take two launches.  k_sample_groups, a
+// workgroup per 1024 ids, rewrites its ids (bans, n-gram hits, penalties) and
+// writes the largest key of every group of 16 to 256 neighbouring ids.  The
+// drawing workgroup then searches those at most 4096 maxima for a threshold
+// that K1 = k + 1 groups reach: at least K1 elements do, and only the groups
+// that reach it can hold one, so it reads a few thousand elements instead of
+// passing over the row several times from one CU (the row is one CU's 64
+// bytes per clock: 7 us per pass over 262144 logits, of which the one-launch
+// form makes four and more).  Measured on 262144 logits N(0, 3), top-k 40 +
+// top-p 0.95 + repeat penalty: 188.8 us -> 5.6 + 21.7 us.
+// Small rows take one launch, one workgroup of 1024 threads for everything.
 //
 // Stages, in the reference's order, with its arithmetic:
 //   bans -> -inf, no-repeat-ngram hits -> -inf           (sampler.c:78-101)
@@ -45,8 +57,12 @@ constexpr int NT = 1024;            // threads per workgroup
 constexpr int NW = NT / 64;         // waves
 constexpr int CAP = 4096;           // LDS key array (penalty window, sorts)
 constexpr int GT = 1024;            // gathered candidates of the fast path: one per thread
-constexpr int RPT = 32;             // row values per thread held in registers (n_vocab <= RPT * NT)
+constexpr int RPT = 16;             // row values per thread held in registers (n_vocab <= RPT * NT)
 constexpr int KMAX = SAMPLER_TOPK_MAX;
+constexpr int GS_MAX = 256;         // ids per group: one wave's 64 loads of 4
+constexpr int GRP_MIN_VOCAB = 16 * 1024;              // 1024 groups of 16: more than K1 = 513
+constexpr int GRP_MAX_VOCAB = SAMPLER_GROUPS * GS_MAX;
+constexpr int GLIST = 1024;         // groups at or above the threshold, at most
 
 // order-preserving key: larger float <=> larger key (-0 < +0; NaNs at the ends)
 __device__ __forceinline__ uint32_t okey(float v) {
@@ -165,7 +181,7 @@ struct Lds {
     int hi[KMAX];
     int red[NW][16];
     int cred[2][NW][16];                  // per-round wave counts of the threshold search
-    int cnt[16];
+    int glist[GLIST], gn;                 // the groups that reach the threshold
     float bv[NW];
     int bi[NW];
     int suf[64];
@@ -240,13 +256,10 @@ __device__ void heap_replay(const float *L, int nv, int k, Lds &sh) {
     }
 }
 
-template <int REG>
-__global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out, int accept, int *state, int n_ctx) {
-    __shared__ Lds sh;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int nv = S->n_vocab, rn = S->recent_n;
-    const float temp = S->temp, top_p = S->top_p, rp = S->repeat_penalty, fp = S->freq_penalty,
-                pp = S->presence_penalty;
+// The rewrites of sampler.c:78-137 by one workgroup of NT threads.
+__device__ void rewrite(SamplerDev *S, float *L, Lds &sh) {
+    const int t = threadIdx.x, rn = S->recent_n;
+    const float rp = S->repeat_penalty, fp = S->freq_penalty, pp = S->presence_penalty;
     const int rln = S->repeat_last_n, ngram = S->no_repeat_ngram;
 
     // ---- bans and no-repeat-ngram (sampler.c:78-101) ----
@@ -290,10 +303,228 @@ __global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out
         }
         __syncthreads();
     }
+}
 
+// First launch of a large row: the rewrites of sampler.c:78-137 for this
+// workgroup's 1024 ids, then the largest key of each of its groups of GS ids (all
+// ones if one of them is NaN).  Every workgroup walks the ban list, the ring
+// and the penalty window, and keeps the ids of its own slice; the window entry
+// that comes first of its id's entries counts them.
+template <int GS>
+__global__ __launch_bounds__(256) void k_sample_groups(SamplerDev *S, float *L, uint32_t *groups) {
+    __shared__ int win[SAMPLER_RING], suf[64], mod;
+    const int t = threadIdx.x, nv = S->n_vocab, rn = S->recent_n;
+    const float rp = S->repeat_penalty, fp = S->freq_penalty, pp = S->presence_penalty;
+    const int rln = S->repeat_last_n, ngram = S->no_repeat_ngram, nban = S->n_ban;
+    const int lo = blockIdx.x * 1024, hi = min(lo + 1024, nv), i0 = lo + 4 * t;
+    float v[4];
+    auto load = [&] {
+        if (i0 + 3 < nv) f4(*(const float4 *)(L + i0), v);
+        else
+            for (int q = 0; q < 4; q++) v[q] = i0 + q < nv ? L[i0 + q] : -INFINITY;
+    };
+    load();
+    auto mine = [&](int id) { return id >= lo && id < hi; };
+    if (t == 0) mod = 0;
+    __syncthreads();
+    const int *ban = sampler_bans(S);
+    for (int j = t; j < nban; j += 256)
+        if (mine(ban[j])) { L[ban[j]] = -INFINITY; mod = 1; }
+    if (ngram >= 2 && rn >= ngram) {
+        const int m = ngram - 1 < 64 ? ngram - 1 : 64;
+        if (t < m) suf[t] = ring_at(S, rn - m + t);
+        __syncthreads();
+        for (int p = t; p + m < rn; p += 256) {
+            const int id = ring_at(S, p + m);
+            if (!mine(id)) continue;
+            bool hit = true;
+            for (int j = 0; j < m && hit; j++) hit = ring_at(S, p + j) == suf[j];
+            if (hit) { L[id] = -INFINITY; mod = 1; }
+        }
+    }
+    if ((rp != 1.0f || fp != 0 || pp != 0) && rln > 0 && rn > 0) {
+        const int nw = rln < rn ? rln : rn;
+        for (int i = t; i < nw; i += 256) win[i] = ring_at(S, rn - 1 - i);
+        __syncthreads();                                             // the -inf stores above included
+        for (int i = t; i < nw; i += 256) {
+            const int id = win[i];
+            if (!mine(id)) continue;
+            int count = 0, first = nw;
+            for (int j = nw - 1; j >= 0; j--)
+                if (win[j] == id) { count++; first = j; }
+            if (first != i) continue;
+            float l = L[id];
+            if (rp != 1.0f) l = l <= 0 ? l * rp : l / rp;
+            const float fterm = (float)count * fp;
+            l -= fterm + (count > 0 ? pp : 0.0f);
+            L[id] = l;
+            mod = 1;
+        }
+    }
+    __syncthreads();
+    if (mod) load();
+    uint32_t k = 0;
+    bool nan = false;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        nan |= __builtin_isnan(v[q]);
+        if (i0 + q < nv) k = max(k, okey(v[q]));
+    }
+    if (nan) k = 0xffffffffu;
+    k = max(k, partner<1>(k));
+    k = max(k, partner<2>(k));
+    if constexpr (GS >= 64) {
+        k = max(k, partner<4>(k));
+        k = max(k, partner<8>(k));
+    }
+    if constexpr (GS >= 256) {
+        k = max(k, partner<16>(k));
+        k = max(k, partner<32>(k));
+    }
+    if (i0 < nv && (4 * t) % GS == 0) groups[i0 / GS] = k;
+}
+
+// The first index of the row's maximum from its group maxima (wg_first_argmax's
+// rule: -0 equals +0, a row starting with NaN gives 0, other NaNs never win)
+template <int GS>
+__device__ int first_argmax_of_groups(const float *L, int nv, const uint32_t (&gk)[SAMPLER_GROUPS / NT], Lds &sh) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    uint32_t km = 0;
+#pragma unroll
+    for (uint32_t k : gk) km = max(km, k);
+    km = wave_umax(km);
+    if (lane == 0) sh.red[wave][0] = (int)km;
+    if (t == 0) sh.gathered = 0x7fffffff;
+    __syncthreads();
+    km = 0;
+    for (int w = 0; w < NW; w++) km = max(km, (uint32_t)sh.red[w][0]);
+    if (km == 0xffffffffu) return wg_first_argmax(L, nv, sh.bv, sh.bi);   // a NaN somewhere
+    const float best = okey_val(km);
+#pragma unroll
+    for (int q = 0; q < SAMPLER_GROUPS / NT; q++)
+        if (gk[q] && okey_val(gk[q]) == best) atomicMin(&sh.gathered, t + q * NT);
+    __syncthreads();
+    const int base = sh.gathered * GS;
+    __syncthreads();
+    if (t == 0) sh.gathered = 0x7fffffff;
+    __syncthreads();
+    if (t < GS && base + t < nv && L[base + t] == best) atomicMin(&sh.gathered, base + t);
+    __syncthreads();
+    return sh.gathered;
+}
+
+// Gathers every element of the row at or above a threshold that at least K1
+// elements reach into sh.keys (sh.gathered of them): the threshold is one that
+// at least K1 group maxima reach.  lo: the smallest group maximum, kmax the
+// largest.  False (nothing gathered of use) when ties or a row whose largest
+// values crowd into few groups leave more than GT candidates.
+template <int GS>
+__device__ bool gather_from_groups(const float *L, int nv, int ng, const uint32_t (&gk)[SAMPLER_GROUPS / NT], int K1, uint32_t lo,
+                                   uint32_t kmax, Lds &sh) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    constexpr int GPT = SAMPLER_GROUPS / NT;
+    const int most = K1 + K1 / 8 + 16;                               // close enough: a few more groups to read
+    uint64_t hi = (uint64_t)kmax + 1;                                // count(key >= hi) < K1
+    int c_lo = ng;
+    for (int round = 0; c_lo > most; round++) {
+        const uint64_t span = hi - lo;
+        if (span <= 1) break;                                        // equal maxima
+        // 15 thresholds as in the row's search; wave counts by ballots, lane j
+        // keeping threshold j's
+        uint32_t mine = 0, pj = 0;
+#pragma unroll
+        for (int j = 0; j < 15; j++) {
+            const uint32_t p = round == 0 ? (uint32_t)(hi - (span >> (j + 1))) : (uint32_t)(lo + (span * (uint64_t)(j + 1)) / 16);
+            uint32_t c = 0;
+#pragma unroll
+            for (int q = 0; q < GPT; q++) c += __builtin_popcountll(__ballot(gk[q] >= p));
+            mine = (lane & 15) == j ? c : mine;
+            pj = (lane & 15) == j ? p : pj;
+        }
+        int (*cr)[16] = sh.cred[round & 1];
+        if (lane < 16) cr[wave][lane] = (int)mine;
+        __syncthreads();
+        int c = 0;
+#pragma unroll
+        for (int w = 0; w < NW / 4; w++) c += cr[(lane >> 4) + 4 * w][lane & 15];
+        c += partner<16>(c);
+        c += partner<32>(c);
+        // the counts fall with j: the last threshold that K1 groups reach
+        const uint32_t m = (uint32_t)__ballot(c >= K1) & 0x7fffu;    // lanes 0..14
+        const int jb = m ? 31 - __builtin_clz(m) : -1;
+        if (jb >= 0) {
+            const uint32_t p = (uint32_t)__builtin_amdgcn_readlane((int)pj, jb);
+            if (jb < 14) hi = (uint32_t)__builtin_amdgcn_readlane((int)pj, jb + 1);
+            if (p > lo) { lo = p; c_lo = __builtin_amdgcn_readlane(c, jb); }
+        } else {
+            hi = (uint32_t)__builtin_amdgcn_readlane((int)pj, 0);
+        }
+    }
+    if (c_lo > GLIST) return false;
+#pragma unroll
+    for (int q = 0; q < GPT; q++) {
+        const bool on = t + q * NT < ng && gk[q] >= lo;
+        const uint64_t m = __ballot(on);
+        int base = 0;
+        if (lane == 0 && m) base = atomicAdd(&sh.gn, __builtin_popcountll(m));
+        base = __shfl(base, 0, 64);
+        if (on) sh.glist[base + __builtin_popcountll(m & ((1ull << lane) - 1))] = t + q * NT;
+    }
+    __syncthreads();
+    constexpr int LG = GS / 4;                                       // loads of 4 per group
+    const int units = sh.gn * LG;                                    // uniform
+    for (int u0 = 0; u0 < units; u0 += 4 * NT) {
+        float v[4][4];
+        int at[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int u = u0 + q * NT + t;
+            at[q] = u < units ? sh.glist[u / LG] * GS + 4 * (u % LG) : nv;
+            if (at[q] + 3 < nv) f4(*(const float4 *)(L + at[q]), v[q]);
+            else
+                for (int e = 0; e < 4; e++) v[q][e] = at[q] + e < nv ? L[at[q] + e] : 0.0f;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t kk = okey(v[q][e]);
+                const bool keep = at[q] + e < nv && kk >= lo;
+                const uint64_t m = __ballot(keep);
+                if (m == 0) continue;                                // uniform
+                int base = 0;
+                if (lane == 0) base = atomicAdd(&sh.gathered, __builtin_popcountll(m));
+                base = __shfl(base, 0, 64);
+                const int slot = base + __builtin_popcountll(m & ((1ull << lane) - 1));
+                if (keep && slot < GT) sh.keys[slot] = ((uint64_t)kk << 32) | (uint32_t)~(uint32_t)(at[q] + e);
+            }
+    }
+    __syncthreads();
+    return sh.gathered <= GT;
+}
+
+// GS > 0: the second launch of a large row (its ids rewritten, groups holding
+// the largest keys of its groups of GS ids).  GS = 0: the whole chain.
+template <int REG, int GS>
+__global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out, int accept, int *state, int n_ctx,
+                                               const uint32_t *groups) {
+    __shared__ Lds sh;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int nv = S->n_vocab;
+    const float temp = S->temp, top_p = S->top_p;
+    if constexpr (GS == 0) rewrite(S, L, sh);
+    constexpr int GPT = SAMPLER_GROUPS / NT;                         // group maxima per thread
+    const int ng = GS ? (nv + GS - 1) / (GS ? GS : 1) : 0;
+    uint32_t gk[GPT];
+    if constexpr (GS > 0) {
+#pragma unroll
+        for (int q = 0; q < GPT; q++) gk[q] = t + q * NT < ng ? groups[t + q * NT] : 0u;
+    }
     // ---- greedy (140-144) ----
     if (temp <= 0.0f) {
-        const int id = wg_first_argmax(L, nv, sh.bv, sh.bi);
+        int id;
+        if constexpr (GS > 0) id = first_argmax_of_groups<GS>(L, nv, gk, sh);
+        else id = wg_first_argmax(L, nv, sh.bv, sh.bi);
         if (t == 0) {
             if (out) *out = id;
             if (accept) ring_push(S, id);
@@ -345,17 +576,26 @@ __global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out
     // exchanges, the NaN flag by a ballot)
     uint32_t kmax = 0, kmin_c = 0;                 // kmin_c: complement of the smallest key
     int nan = 0;
-    each([&](int, float v) {
-        nan |= __builtin_isnan(v);
-        const uint32_t kk = okey(v);
-        kmax = kk > kmax ? kk : kmax;
-        kmin_c = ~kk > kmin_c ? ~kk : kmin_c;
-    });
+    if constexpr (GS > 0) {
+#pragma unroll
+        for (int q = 0; q < GPT; q++) {
+            kmax = max(kmax, gk[q]);
+            nan |= gk[q] == 0xffffffffu;
+            if (t + q * NT < ng) kmin_c = max(kmin_c, ~gk[q]);
+        }
+    } else {
+        each([&](int, float v) {
+            nan |= __builtin_isnan(v);
+            const uint32_t kk = okey(v);
+            kmax = kk > kmax ? kk : kmax;
+            kmin_c = ~kk > kmin_c ? ~kk : kmin_c;
+        });
+    }
     kmax = wave_umax(kmax);
     kmin_c = wave_umax(kmin_c);
     const bool wnan = __ballot(nan != 0) != 0;
     if (lane == 0) { sh.red[wave][0] = (int)kmax; sh.red[wave][1] = wnan; sh.red[wave][2] = (int)kmin_c; }
-    if (t == 0) { sh.gathered = 0; sh.flag = 0; }
+    if (t == 0) { sh.gathered = 0; sh.gn = 0; sh.flag = 0; }
     __syncthreads();
     kmax = 0;
     kmin_c = 0;
@@ -369,7 +609,17 @@ __global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out
 
     bool slow = nan != 0;
     uint32_t lo = ~kmin_c;                 // count(key >= lo) >= K1: every element
-    if (!slow) {
+    bool whole = true;                     // search the row itself
+    if constexpr (GS > 0) {
+        if (!slow) {
+            whole = !gather_from_groups<GS>(L, nv, ng, gk, K1, lo, kmax, sh);
+            if (whole) lo = 0;             // the smallest key of the groups' maxima is no bound of the row
+            __syncthreads();
+            if (whole && t == 0) sh.gathered = 0;
+            __syncthreads();
+        }
+    }
+    if (!slow && whole) {
         uint64_t hi = (uint64_t)kmax + 1;  // count(key >= hi) < K1
         int c_lo = nv, buf = 0;
         // the 15 counts of keys >= p[j] over the row
@@ -409,7 +659,7 @@ __global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out
         }
     }
 
-    if (!slow) {
+    if (!slow && whole) {
         // gather every element with key >= lo (at most GT) by wave-ballot compaction
         auto gather = [&](int i, float v) {                          // every lane of the wave, each step
             const uint32_t kk = i < nv ? okey(v) : 0u;
@@ -430,6 +680,8 @@ __global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out
             for (int i0 = 0; i0 < nv; i0 += NT) gather(i0 + t, i0 + t < nv ? L[i0 + t] : 0.0f);
         }
         __syncthreads();
+    }
+    if (!slow) {
         const int G = sh.gathered;
         int P = 1;
         while (P < G) P <<= 1;
@@ -573,11 +825,28 @@ __global__ __launch_bounds__(64) void k_sampler_push(SamplerDev *S, const int *i
 
 }  // namespace
 
-hipError_t launch_sample(SamplerDev *S, int n_vocab, float *logits, int *out, int accept, int *state, int n_ctx,
+template <int GS>
+static void sample_large(SamplerDev *S, int n_vocab, float *L, int *out, int accept, int *state, int n_ctx, uint32_t *groups,
                          hipStream_t s) {
-    if (!S || !logits || n_vocab <= 0 || ((uintptr_t)logits & 15)) return hipErrorInvalidValue;
-    if (n_vocab <= RPT * NT) hipLaunchKernelGGL(k_sample<RPT>, dim3(1), dim3(NT), 0, s, S, logits, out, accept, state, n_ctx);
-    else hipLaunchKernelGGL(k_sample<0>, dim3(1), dim3(NT), 0, s, S, logits, out, accept, state, n_ctx);
+    hipLaunchKernelGGL(k_sample_groups<GS>, dim3((unsigned)((n_vocab + 1023) / 1024)), dim3(256), 0, s, S, L, groups);
+    hipLaunchKernelGGL((k_sample<0, GS>), dim3(1), dim3(NT), 0, s, S, L, out, accept, state, n_ctx, groups);
+}
+
+hipError_t launch_sample(SamplerDev *S, int n_vocab, float *logits, int *out, int accept, int *state, int n_ctx,
+                         uint32_t *groups, hipStream_t s) {
+    if (!S || !logits || !groups || n_vocab <= 0 || ((uintptr_t)logits & 15)) return hipErrorInvalidValue;
+    // two launches from GRP_MIN_VOCAB ids, the group size such that at most
+    // SAMPLER_GROUPS maxima come out; beyond them one workgroup reads the row
+    if (n_vocab >= GRP_MIN_VOCAB && n_vocab <= 16 * SAMPLER_GROUPS)
+        sample_large<16>(S, n_vocab, logits, out, accept, state, n_ctx, groups, s);
+    else if (n_vocab >= GRP_MIN_VOCAB && n_vocab <= 64 * SAMPLER_GROUPS)
+        sample_large<64>(S, n_vocab, logits, out, accept, state, n_ctx, groups, s);
+    else if (n_vocab >= GRP_MIN_VOCAB && n_vocab <= GRP_MAX_VOCAB)
+        sample_large<256>(S, n_vocab, logits, out, accept, state, n_ctx, groups, s);
+    else if (n_vocab <= RPT * NT)
+        hipLaunchKernelGGL((k_sample<RPT, 0>), dim3(1), dim3(NT), 0, s, S, logits, out, accept, state, n_ctx, nullptr);
+    else
+        hipLaunchKernelGGL((k_sample<0, 0>), dim3(1), dim3(NT), 0, s, S, logits, out, accept, state, n_ctx, nullptr);
     return hipGetLastError();
 }
 

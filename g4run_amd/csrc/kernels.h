@@ -165,10 +165,11 @@ hipError_t launch_argmax_rows(const float *logits, int n, int nb, int *out, hipS
 constexpr int STATE_CTX_FULL = 1;
 hipError_t launch_argmax_advance(const float *logits, int n, int *state, int n_ctx, hipStream_t s);
 
-// k_sample.hip: the sampling chain of sampler.c:74-210 on one workgroup.
+// k_sample.hip: the sampling chain of sampler.c:74-210.
 // Device image of a sampler: g4_sampler's settings and state (g4run.h:464-482)
 // with a fixed ring of SAMPLER_RING ids (the reference's recent_cap,
-// sampler.c:10) and the ban list after the struct (n_vocab ints).  The
+// sampler.c:10), then the ban list (n_vocab ints) and the group maxima of a
+// draw in progress (SAMPLER_GROUPS words).  The
 // per-id counts the reference keeps in accept are not kept: g4_sample never
 // reads them.
 constexpr int SAMPLER_RING = 4096;
@@ -189,14 +190,21 @@ struct SamplerDev {
     int pad_[3];
     int recent[SAMPLER_RING];
 };
-inline size_t sampler_dev_bytes(int n_vocab) { return sizeof(SamplerDev) + (size_t)n_vocab * sizeof(int); }
+constexpr int SAMPLER_GROUPS = 4096;
 __host__ __device__ inline int *sampler_bans(SamplerDev *S) { return reinterpret_cast<int *>(S + 1); }
+__host__ __device__ inline uint32_t *sampler_groups(SamplerDev *S, int n_vocab) {
+    return reinterpret_cast<uint32_t *>(sampler_bans(S) + (((size_t)n_vocab + 3) & ~(size_t)3));
+}
+inline size_t sampler_dev_bytes(int n_vocab) {
+    return sizeof(SamplerDev) + ((((size_t)n_vocab + 3) & ~(size_t)3) + SAMPLER_GROUPS) * sizeof(int);
+}
 // Draws one id from logits[n_vocab] (rewritten in place as sampler.c does),
 // writes it to *out if out, pushes it into the ring if accept, and if state is
 // given (the model's token, pos, npos, steps, flags) stores it there and
-// advances the position as launch_argmax_advance does.
+// advances the position as launch_argmax_advance does.  groups: SAMPLER_GROUPS
+// words of scratch (sampler_groups of a whole sampler allocation).
 hipError_t launch_sample(SamplerDev *S, int n_vocab, float *logits, int *out, int accept, int *state, int n_ctx,
-                         hipStream_t s);
+                         uint32_t *groups, hipStream_t s);
 // Pushes n ids into the ring in order (sampler.c:37-48).
 hipError_t launch_sampler_push(SamplerDev *S, const int *ids, int n, hipStream_t s);
 

@@ -422,7 +422,8 @@ extern "C" int g4h_forward_state(g4h_model *m, void *stream) {
     }
     M_RC(trace_copy(m->trace ? m->trace + (size_t)c.n_layer * trace_rec : nullptr, TR_X, x, E));
     if (m->sampler)
-        M_HIP(launch_sample(sampler_device(m->sampler), c.n_vocab, m->logits, nullptr, 1, m->state, c.n_ctx, s));
+        M_HIP(launch_sample(sampler_device(m->sampler), c.n_vocab, m->logits, nullptr, 1, m->state, c.n_ctx,
+                            sampler_groups(sampler_device(m->sampler), c.n_vocab), s));
     else
         M_HIP(launch_argmax_advance(m->logits, c.n_vocab, m->state, c.n_ctx, s));
     return G4H_OK;

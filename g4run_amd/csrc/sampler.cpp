@@ -1,8 +1,8 @@
 // sampler.cpp -- host side of the device-resident sampler (include/g4hip.h,
 // the GPU form of g4run.h:464-489 / sampler.c).  The settings, RNG words,
 // ring of recent ids and ban list live in one device allocation laid out as
-// g4::SamplerDev, followed by the ban list (n_vocab ints) and a staging area
-// for the ids of g4h_sampler_accept.
+// g4::SamplerDev, followed by the ban list (n_vocab ints), the group maxima of
+// a draw and a staging area for the ids of g4h_sampler_accept.
 #include "../../include/g4hip.h"
 
 #include <cstring>
@@ -66,7 +66,7 @@ extern "C" int g4h_sampler_create(int n_vocab, const g4h_sampler_params *p, g4h_
         delete s;
         return rc;
     }
-    s->stage = sampler_bans(s->dev) + n_vocab;
+    s->stage = reinterpret_cast<int *>(reinterpret_cast<uint8_t *>(s->dev) + sampler_dev_bytes(n_vocab));
     SamplerDev img;
     std::memset(&img, 0, sizeof img);
     put_params(img, p ? *p : def);
@@ -148,7 +148,7 @@ extern "C" int g4h_sampler_accept(g4h_sampler *s, const int *ids, int n, void *s
 extern "C" int g4h_sample(g4h_sampler *s, float *logits_dev, int *out_dev, int accept, void *stream) {
     if (!s || !logits_dev) return g4h_internal_fail(G4H_ERR_ARG, "g4h_sample: null argument");
     if ((uintptr_t)logits_dev % 16) return g4h_internal_fail(G4H_ERR_ARG, "g4h_sample: logits must be 16-byte aligned");
-    S_HIP(launch_sample(s->dev, s->n_vocab, logits_dev, out_dev, accept, nullptr, 0, (hipStream_t)stream));
+    S_HIP(launch_sample(s->dev, s->n_vocab, logits_dev, out_dev, accept, nullptr, 0, sampler_groups(s->dev, s->n_vocab), (hipStream_t)stream));
     return G4H_OK;
 }
 

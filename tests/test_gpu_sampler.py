@@ -60,6 +60,12 @@ def make_logits(rs, nv, kind):
     elif kind == "flat":                      # > 4096 values within one boundary key
         lg = np.full(nv, 1.0, np.float32)
         lg[rs.integers(0, nv, 30)] = 2.0 + rs.random(30).astype(np.float32)
+    elif kind == "sorted":                    # the largest values all in neighbouring ids
+        lg = np.sort(lg)
+    elif kind == "zeros":                     # -0 and +0 share the maximum
+        lg = -np.abs(lg)
+        lg[rs.integers(0, nv, 3)] = -0.0
+        lg[rs.integers(0, nv, 3)] = 0.0
     return lg
 
 
@@ -193,3 +199,18 @@ def test_sampler_argument_errors(gpu):
                 rope_base=1e6, rms_eps=1e-6)
     with pytest.raises(G.G4HError):
         m.set_sampler(s)                        # vocabulary differs
+
+
+# the two-launch form starts at 16384 ids; 16, 64 and 256 ids per group end at
+# 65536, 262144 and 1048576
+@pytest.mark.parametrize("nv,kind", [(nv, kind) for nv in (16383, 16384, 16387, 65536, 65541, 262146)
+                                     for kind in ("plain", "ties", "nan", "inf", "flat", "sorted", "zeros")] + [(1048577, "plain")])
+def test_row_sizes_and_kinds(gpu, oracle, nv, kind):
+    """Group maxima instead of passes over the row: rows on both sides of each
+    group size, rows off the loads of four, ties, NaNs, equal rows and rows
+    whose candidates crowd into a few groups (which search the row itself),
+    with bans, n-gram hits and repeated ids in the window, drawn and greedy."""
+    rs = np.random.default_rng(nv + len(kind))
+    hist = np.concatenate([rs.integers(0, nv, 60), rs.integers(0, 30, 60)])
+    for p in (dict(BASE, repeat_last_n=100, no_repeat_ngram=2), dict(BASE, top_k=0, no_repeat_ngram=0), dict(BASE, temp=0.0)):
+        run_pair(gpu, oracle, nv, p, rs, kind, 2, bans=[0, 2, nv - 1], hist=hist)
