@@ -558,21 +558,19 @@ static int matmul_impl(const g4h_tensor *W, const float *x, const void *pre, siz
     }
     if (path == 0) path = g4h_matmul_path(W, nb);
     if (path == 2 && mfma_capable(W) && mmk_capable(W->type)) {
-        // K-quants: q8_K activation rows (quantized here from x, or given), read as they are
-        const uint8_t *act = (const uint8_t *)pre;
-        size_t stride = pre_stride;
+        // K-quants: x quantized here into the kernel's own layout, or given q8_K
+        // rows read as they are (no scratch)
         if (x) {
             if ((uintptr_t)x % 4) return fail(G4H_ERR_ARG, "g4h_matmul: x must be 4-byte aligned");
-            stride = g4h_act_stride(W->type, W->ncols);
             void *buf;
-            if (int rc = scr.get(s, stride * nb, &buf)) return rc;
-            const hipError_t e = launch_quantize_q8_K(x, W->ncols, (uint8_t *)buf, stride, W->ncols, nb, s);
-            if (e != hipSuccess) return hip_fail(e, "g4h_matmul: quantize");
-            act = (const uint8_t *)buf;
-        } else {
-            if (int rc = check_act("g4h_matmul", W, pre, pre_stride, nb)) return rc;
-            if (nb == 1) stride = g4h_act_stride(W->type, W->ncols);
+            if (int rc = scr.get(s, g4h_act_stride(W->type, W->ncols) * nb, &buf)) return rc;
+            const hipError_t e = launch_matmul_mfma_kx(*W, x, W->ncols, nb, Y, (uint8_t *)buf, s);
+            if (e != hipSuccess) return hip_fail(e, "g4h_matmul: matrix-core launch");
+            return G4H_OK;
         }
+        if (int rc = check_act("g4h_matmul", W, pre, pre_stride, nb)) return rc;
+        const uint8_t *act = (const uint8_t *)pre;
+        const size_t stride = nb == 1 ? g4h_act_stride(W->type, W->ncols) : pre_stride;
         const hipError_t e = launch_matmul_mfma_k(*W, act, stride, nb, Y, s);
         if (e != hipSuccess) return hip_fail(e, "g4h_matmul: matrix-core launch");
         return G4H_OK;

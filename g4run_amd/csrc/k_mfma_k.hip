@@ -28,9 +28,11 @@
 // contract of g4run.h:148-157 within this family); the fp32 order differs
 // from the CPU dots' within the path's tolerance.
 //
-// Activations are the GGUF q8_K rows themselves (d f32 | 256 int8 | 16 int16
-// bsums, 292 bytes a superblock): a lane's 16-byte operand slices are
-// 4-byte-aligned loads.
+// Two kernels with the same arithmetic and the same bits: k_mmk reads given
+// q8_K rows as they are (d f32 | 256 int8 | 16 int16 bsums, 292 bytes a
+// superblock; a lane's 16-byte operand slices are 4-byte-aligned loads) and
+// needs no scratch; k_mmk_tile takes fp32 tokens through the quantizer launch,
+// which writes them in operand order.
 #include <algorithm>
 #include <cstdio>
 
@@ -276,6 +278,279 @@ __global__ __launch_bounds__(64 * MMK_NW) void k_mmk(g4h_tensor W, const uint8_t
     }
 }
 
+// The same sums from fp32 tokens (the usual call): the quantizer launch writes
+// the activations in operand order (k_quantize_q8_K_tile), so a wave's operand
+// load is 1 KB of adjacent bytes, and each wave owns MT token tiles of its row
+// tile, whose weights it loads in runs of adjacent bytes and turns into
+// operands through LDS of its own (no barrier).  k_mmk's operand loads have
+// adjacent lanes in different rows, one L1 access per lane, and the L1's one
+// access per clock bounds it.  Measured at 4096 x 11008, quantizer included
+// (us, k_mmk / this): q4_K at 9 / 64 / 128 / 509 tokens 20.4 / 25.8 / 45.4 /
+// 165 -> 15.8 / 18.3 / 25.1 / 82.8 (554 TOPS); q6_K at 9 / 64 / 509 tokens 30.3
+// / 38.5 / 250 -> 21.6 / 23.2 / 112; q6_K 2048 x 6144 at 64 26.9 -> 14.3.  What
+// bounds it at 509 tokens: 1.0 GB of operands from L2 and 45 us of VALU issue
+// (the scale multiply-adds), partly overlapped.
+// The waves split the superblocks as k_mmk's do, each superblock's integers
+// and scale products are the same, and the partial tiles are added in the same
+// order: k_mmk's bits.  The next superblock's operands are loaded as the
+// current one's are used up.  q6_K's sub-blocks take the signed q6 - 32
+// directly: the integers of sum q6u q8 - 32 bsum.
+struct Q4KTile {
+    static constexpr int T = Q4_K, WL = 5, ROW = 144, LDSB = 32 * ROW;   // loads per lane, LDS bytes per row and wave
+    struct W {
+        mk_v4i v[WL];
+    };
+    struct Ptr {
+        const uint8_t *p[WL];
+    };
+    struct Head {
+        mk_v4i hdr;
+        uint32_t sc[2], mn[2];
+    };
+    // 9 lanes per row of 144 bytes; past the 288 pieces the last one again
+    static __device__ __forceinline__ void piece(int lane, int i, int &r, int &c) {
+        const int f = min(64 * i + lane, 287);
+        r = f / 9, c = f - 9 * r;
+    }
+    static __device__ __forceinline__ void init(Ptr &P, const g4h_tensor &Wt, int64_t n0, int lane) {
+#pragma unroll
+        for (int i = 0; i < WL; i++) {
+            int r, c;
+            piece(lane, i, r, c);
+            P.p[i] = Wt.qs + (size_t)std::min<int64_t>(n0 + r, Wt.nrows - 1) * Wt.nb * 144 + 16 * c;
+        }
+    }
+    static __device__ __forceinline__ void load(W &w, const Ptr &P, int s) {
+#pragma unroll
+        for (int i = 0; i < WL; i++) w.v[i] = mk_ld(P.p[i] + (size_t)s * 144);
+    }
+    static __device__ __forceinline__ void put(const W &w, uint8_t *lds, int lane) {
+#pragma unroll
+        for (int i = 0; i < WL; i++) {
+            int r, c;
+            piece(lane, i, r, c);
+            *(mk_v4i *)(lds + r * ROW + 16 * c) = w.v[i];
+        }
+    }
+    // the row's 6-bit scales and mins (quants.c:417-423), four to a word
+    static __device__ __forceinline__ Head head(const uint8_t *lds, int li) {
+        Head h;
+        h.hdr = *(const mk_v4i *)(lds + li * ROW);
+        const uint32_t w0 = (uint32_t)h.hdr.y, w1 = (uint32_t)h.hdr.z, w2 = (uint32_t)h.hdr.w;
+        h.sc[0] = w0 & 0x3f3f3f3fu;
+        h.mn[0] = w1 & 0x3f3f3f3fu;
+        h.sc[1] = (w2 & 0x0f0f0f0fu) | ((w0 >> 2) & 0x30303030u);
+        h.mn[1] = ((w2 >> 4) & 0x0f0f0f0fu) | ((w1 >> 2) & 0x30303030u);
+        return h;
+    }
+};
+
+struct Q6KTile {
+    static constexpr int T = Q6_K, WL = 7, QL = 144, QH = 80, LDSB = 32 * (QL + QH);
+    struct W {
+        mk_v4i v[WL];                                                // ql, qh, scales
+        uint16_t d;
+    };
+    struct Ptr {
+        const uint8_t *ql[4], *qh[2], *sc, *dd;
+    };
+    static __device__ __forceinline__ void init(Ptr &P, const g4h_tensor &Wt, int64_t n0, int lane) {
+        auto row = [&](int r) { return (size_t)std::min<int64_t>(n0 + r, Wt.nrows - 1) * Wt.nb; };
+#pragma unroll
+        for (int i = 0; i < 4; i++) P.ql[i] = Wt.qs + row(8 * i + (lane >> 3)) * 128 + 16 * (lane & 7);
+#pragma unroll
+        for (int i = 0; i < 2; i++) P.qh[i] = Wt.ex + row(16 * i + (lane >> 2)) * 64 + 16 * (lane & 3);
+        P.sc = Wt.sc + row(lane & 31) * 16;
+        P.dd = Wt.dd + row(lane & 31) * 2;
+    }
+    static __device__ __forceinline__ void load(W &w, const Ptr &P, int s) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) w.v[i] = mk_ld(P.ql[i] + (size_t)s * 128);
+#pragma unroll
+        for (int i = 0; i < 2; i++) w.v[4 + i] = mk_ld(P.qh[i] + (size_t)s * 64);
+        w.v[6] = mk_ld(P.sc + (size_t)s * 16);
+        w.d = *(const uint16_t *)(P.dd + (size_t)s * 2);
+    }
+    static __device__ __forceinline__ void put(const W &w, uint8_t *lds, int lane) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) *(mk_v4i *)(lds + (8 * i + (lane >> 3)) * QL + 16 * (lane & 7)) = w.v[i];
+#pragma unroll
+        for (int i = 0; i < 2; i++) *(mk_v4i *)(lds + 32 * QL + (16 * i + (lane >> 2)) * QH + 16 * (lane & 3)) = w.v[4 + i];
+    }
+    static __device__ __forceinline__ mk_v4i split(const uint8_t *p) {
+        const mk_v2i a = *(const mk_v2i *)p, b = *(const mk_v2i *)(p + 16);
+        return mk_v4i{a.x, a.y, b.x, b.y};
+    }
+};
+
+// isum += c * i over a result tile, one v_mad_i32_i24 per value: the empty asm
+// keeps the compiler from splitting two of them into two multiplies and a
+// three-operand add
+__device__ __forceinline__ void mk_mad(mk_v16i &isum, int c, const mk_v16i &i) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        int v = __mul24(c, i[r]) + isum[r];
+        asm("" : "+v"(v));
+        isum[r] = v;
+    }
+}
+
+// Workgroup b runs on XCD b % 8: row tiles r with r % 8 == b % 8, the token
+// tiles of a row tile consecutively (as k_mmk).
+template <class S, int MT>
+__global__ __launch_bounds__(64 * MMK_NW) void k_mmk_tile(g4h_tensor W, const uint8_t *__restrict__ act, int M, float *__restrict__ Y,
+                                                          int ntok) {
+    constexpr int PB = MMK_NW * MT * 32 * 33 * 4, WBYTES = MMK_NW * S::LDSB;
+    __shared__ __align__(16) uint8_t lds[PB > WBYTES ? PB : WBYTES];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x) >> 6;
+    const int li = lane & 31, kh = lane >> 5;
+    const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
+    const int64_t n0 = ((int64_t)(l / ntok) * 8 + x) * 32;
+    const int m0 = (l % ntok) * (32 * MT);
+    if (n0 >= W.nrows) return;                                           // uniform over the workgroup
+    const int nb = (int)W.nb;
+    uint8_t *wl = lds + wave * S::LDSB;
+    // activation tiles (a second tile past the last token repeats the first)
+    const uint8_t *ab[MT];
+    int TL[MT], ao[MT], tl[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+        const int t0 = m0 + 32 * m < M ? m0 + 32 * m : m0;
+        TL[m] = min(32, M - t0);
+        ab[m] = act + (size_t)t0 * nb * 292;
+        tl[m] = min(li, TL[m] - 1);
+        ao[m] = (kh * TL[m] + tl[m]) * 16;
+    }
+    typename S::Ptr P;
+    S::init(P, W, n0, lane);
+    typename S::W w;
+    mk_v4i a[MT][8], bs[MT];
+    float d[MT];
+    auto load_a = [&](int m, int j, int s) __attribute__((always_inline)) {
+        a[m][j] = mk_ld(ab[m] + (size_t)s * TL[m] * 292 + 2 * j * TL[m] * 16 + ao[m]);
+    };
+    auto load_s = [&](int m, int s) __attribute__((always_inline)) {
+        const uint8_t *b = ab[m] + (size_t)s * TL[m] * 292;
+        if constexpr (S::T == Q4_K) bs[m] = mk_ld(b + TL[m] * 256 + ao[m]);
+        d[m] = *(const float *)(b + TL[m] * 288 + 4 * tl[m]);
+    };
+    mk_v16f acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++) acc[m] = mk_v16f{};
+    const mk_v16i z = {};
+    if (wave < nb) {
+        S::load(w, P, wave);
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) load_a(m, j, wave);
+            load_s(m, wave);
+        }
+    }
+    for (int s = wave; s < nb; s += MMK_NW) {                            // uniform over the wave
+        const int sn = s + MMK_NW < nb ? s + MMK_NW : s;                 // the next one (the last again at the end)
+        S::put(w, wl, lane);
+        typename S::W wc;                                                // q6_K: scales and d of this superblock
+        if constexpr (S::T == Q6_K) wc.v[6] = w.v[6], wc.d = w.d;
+        asm volatile("" ::: "memory");                                   // a wave's LDS accesses complete in order
+        S::load(w, P, sn);
+        asm volatile("" ::: "memory");
+        mk_v16i isum[MT];
+#pragma unroll
+        for (int m = 0; m < MT; m++) isum[m] = z;
+        if constexpr (S::T == Q4_K) {
+            const auto h = S::head(wl, li);
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                const mk_v4i q = *(const mk_v4i *)(wl + li * S::ROW + 16 + 32 * p + 16 * kh);
+                const mk_v4i lo = q & 0x0F0F0F0F, hi = (q >> 4) & 0x0F0F0F0F;
+                int sc0 = (h.sc[p >> 1] >> (16 * (p & 1))) & 0xff, sc1 = (h.sc[p >> 1] >> (16 * (p & 1) + 8)) & 0xff;
+                asm("" : "+v"(sc0), "+v"(sc1));                          // no byte select inside the multiplies
+#pragma unroll
+                for (int m = 0; m < MT; m++) {
+                    const mk_v16i i0 = mk_mma(a[m][2 * p], lo, z), i1 = mk_mma(a[m][2 * p + 1], hi, z);
+                    load_a(m, 2 * p, sn);
+                    load_a(m, 2 * p + 1, sn);
+                    asm volatile("" ::: "memory");
+                    mk_mad(isum[m], sc0, i0);
+                    mk_mad(isum[m], sc1, i1);
+                }
+            }
+            // weight operand of summ: m of bsums 8 kh .. 8 kh + 7, sub-blocks 4 kh .. 4 kh + 3
+            const uint32_t mn = kh ? h.mn[1] : h.mn[0];
+            mk_v8h mh;
+#pragma unroll
+            for (int t = 0; t < 4; t++) mh[2 * t] = mh[2 * t + 1] = (_Float16)(float)((mn >> (8 * t)) & 0xff);
+            const float dw = h2f((uint16_t)((uint32_t)h.hdr.x & 0xffff)), dm = h2f((uint16_t)((uint32_t)h.hdr.x >> 16));
+            const mk_v32f zf = {};
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                const mk_v16f summ = mk_mma_h(__builtin_bit_cast(mk_v8h, bs[m]), mh);
+                const mk_v32f P2 = __builtin_amdgcn_mfma_f32_32x32x1f32(d[m], kh ? dm : dw, zf, 0, 0, 0);
+                load_s(m, sn);
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    acc[m][r] = __builtin_fmaf(P2[r], (float)isum[m][r], acc[m][r]);
+                    acc[m][r] = __builtin_fmaf(-P2[16 + r], summ[r], acc[m][r]);
+                }
+            }
+        } else {
+            auto scb = [&](int k) { return (int)(int8_t)(((uint32_t)wc.v[6][k >> 2] >> (8 * (k & 3))) & 0xff); };
+#pragma unroll
+            for (int hh = 0; hh < 2; hh++) {
+                const mk_v4i l0 = S::split(wl + li * S::QL + 64 * hh + 8 * kh), l1 = S::split(wl + li * S::QL + 64 * hh + 32 + 8 * kh);
+                const mk_v4i hb = S::split(wl + 32 * S::QL + li * S::QH + 32 * hh + 8 * kh);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const mk_v4i &L = (j & 1) ? l1 : l0;
+                    mk_v4i q = ((L >> (j >= 2 ? 4 : 0)) & 0x0F0F0F0F) | (((hb >> (2 * j)) & 0x03030303) << 4);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) q[e] = (int)(((uint32_t)q[e] + 0x60606060u) ^ 0x80808080u);   // per byte: q - 32
+                    int c0 = scb(8 * hh + 2 * j), c1 = scb(8 * hh + 2 * j + 1);
+                    asm("" : "+v"(c0), "+v"(c1));                        // no byte select inside the multiplies
+#pragma unroll
+                    for (int m = 0; m < MT; m++) {
+                        const mk_v4i &xa = a[m][4 * hh + j];
+                        const mk_v16i i0 = mk_mma16(xa.xy, q.xy, z), i1 = mk_mma16(xa.zw, q.zw, z);
+                        load_a(m, 4 * hh + j, sn);
+                        asm volatile("" ::: "memory");
+                        mk_mad(isum[m], c0, i0);
+                        mk_mad(isum[m], c1, i1);
+                    }
+                }
+            }
+            const mk_v16f zf = {};
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                const mk_v16f P1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kh ? 0.0f : d[m], h2f(wc.d), zf, 0, 0, 0);
+                load_s(m, sn);
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[m][r] = __builtin_fmaf(P1[r], (float)isum[m][r], acc[m][r]);
+            }
+        }
+    }
+    __syncthreads();
+    // C[i][j]: j = lane % 32 (weight row), i = 8 (r / 4) + 4 kh + r % 4 (token)
+    float (*part)[MT * 32][33] = (float (*)[MT * 32][33])lds;
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) part[wave][32 * m + 8 * (r >> 2) + 4 * kh + (r & 3)][li] = acc[m][r];
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < MT * 32 * 32 / (64 * MMK_NW); h++) {
+        const int o = threadIdx.x + 64 * MMK_NW * h, i = o >> 5, j = o & 31;
+        float v = part[0][i][j];
+#pragma unroll
+        for (int k = 1; k < MMK_NW; k++) v += part[k][i][j];
+        const int m = m0 + i;
+        const int64_t n = n0 + j;
+        if (m < M && n < W.nrows) Y[(size_t)m * W.nrows + n] = v;
+    }
+}
+
 bool mmk_capable(int type) { return type == Q4_K || type == Q6_K; }
 
 static void mmk_grid(const g4h_tensor &W, int M, int64_t &grid, int &ntok) {
@@ -294,12 +569,32 @@ hipError_t launch_matmul_mfma_k(const g4h_tensor &W, const uint8_t *act, size_t 
     return hipGetLastError();
 }
 
+// token tiles per wave: two (each weight load and unpack serving 64 tokens)
+// once that still gives every CU a workgroup (q4_K 4096 x 11008, one / two:
+// 64 tokens 18.7 / 25.3 us, 128 tokens 31.1 / 25.9)
+static int mmk_mt(const g4h_tensor &W, int M) { return (W.nrows + 31) / 32 * ((M + 63) / 64) >= 256 ? 2 : 1; }
+
+hipError_t launch_matmul_mfma_kx(const g4h_tensor &W, const float *x, size_t xs, int M, float *Y, uint8_t *ws, hipStream_t s) {
+    if (!mmk_capable(W.type) || M < 1 || !x || !Y || (uintptr_t)ws % 64) return hipErrorInvalidValue;
+    if (hipError_t e = launch_quantize_q8_K_tile(x, xs, ws, W.ncols, M, W.type, s)) return e;
+    const int mt = mmk_mt(W, M), ntok = (M + 32 * mt - 1) / (32 * mt);
+    const int64_t grid = (W.nrows + 255) / 256 * 8 * ntok;
+    if (grid > 0x7fffffff) return hipErrorInvalidValue;
+    const dim3 g((unsigned)grid), b(64 * MMK_NW);
+    if (W.type == Q4_K) {
+        if (mt == 1) hipLaunchKernelGGL((k_mmk_tile<Q4KTile, 1>), g, b, 0, s, W, ws, M, Y, ntok);
+        else hipLaunchKernelGGL((k_mmk_tile<Q4KTile, 2>), g, b, 0, s, W, ws, M, Y, ntok);
+    } else {
+        if (mt == 1) hipLaunchKernelGGL((k_mmk_tile<Q6KTile, 1>), g, b, 0, s, W, ws, M, Y, ntok);
+        else hipLaunchKernelGGL((k_mmk_tile<Q6KTile, 2>), g, b, 0, s, W, ws, M, Y, ntok);
+    }
+    return hipGetLastError();
+}
+
 void mmk_describe(const g4h_tensor &W, int M, char *buf, size_t len) {
-    int64_t grid;
-    int ntok;
-    mmk_grid(W, M, grid, ntok);
-    snprintf(buf, len, "k_mmk<%s> grid=%lld block=%d (int8 MFMA, 32x32 tiles, %d waves split the superblocks)",
-             W.type == Q4_K ? "q4_K" : "q6_K", (long long)grid, 64 * MMK_NW, MMK_NW);
+    const int mt = mmk_mt(W, M), ntok = (M + 32 * mt - 1) / (32 * mt);
+    snprintf(buf, len, "k_mmk_tile<%s,mt=%d> grid=%lld block=%d (int8 MFMA, %dx32 tiles, %d waves split the superblocks)",
+             W.type == Q4_K ? "q4_K" : "q6_K", mt, (long long)((W.nrows + 255) / 256 * 8 * ntok), 64 * MMK_NW, 32 * mt, MMK_NW);
 }
 
 }  // namespace g4

@@ -71,6 +71,45 @@ __global__ __launch_bounds__(256) void k_quantize_q8_K(const float *__restrict__
     }
 }
 
+// The same quants in k_mmk_tile's operand layout: tiles of 32 tokens (the last
+// one TL = rows % 32 wide), per superblock sixteen 16-byte chunks [2 g + kh][TL]
+// -- the lane half kh's quants of the 32-element group g -- then with BS the 16
+// bsums as fp16 [kh][TL][8] (exact: |bsum| <= 2048; without them the place stays
+// unused) and d [TL].  HALVES: kh holds elements 8 kh .. + 7 and 16 + 8 kh .. +
+// 7 of a group (q6_K's sub-blocks of 16), else 16 kh .. + 15.  Consecutive
+// waves take consecutive tokens of one superblock, so their 4-byte stores
+// share lines.
+// QT superblocks per wave (QT consecutive tokens of one superblock index), all
+// of their loads issued first.
+template <bool HALVES, bool BS, int QT>
+__global__ __launch_bounds__(256) void k_quantize_q8_K_tile(const float *__restrict__ x, size_t xs, uint8_t *__restrict__ y, int nb,
+                                                            int rows) {
+    const int nt = (rows + QT - 1) / QT;
+    const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (w >= (int64_t)nt * nb) return;                                   // uniform over the wave
+    const int l = threadIdx.x & 63;
+    const int sb = (int)(w / nt), r0 = QT * (int)(w - (int64_t)sb * nt);
+    float v[QT][4];
+#pragma unroll
+    for (int q = 0; q < QT; q++) {
+        const float *src = x + (size_t)min(r0 + q, rows - 1) * xs + (size_t)sb * 256 + 4 * l;
+        for (int i = 0; i < 4; i++) v[q][i] = src[i];
+    }
+    const int g = l >> 3, e = 4 * (l & 7), k = l >> 2;
+    const int kh = HALVES ? (e >> 3) & 1 : e >> 4, at = HALVES ? (e & 7) + 8 * (e >> 4) : e & 15;
+#pragma unroll
+    for (int q = 0; q < QT; q++) {
+        const int r = r0 + q;
+        if (r >= rows) break;                                            // uniform
+        const Q8KLane o = q8K_wave(v[q]);
+        const int tl = r & 31, TL = min(32, rows - (r & ~31));
+        uint8_t *b = y + ((size_t)(r & ~31) * nb + (size_t)sb * TL) * 292;
+        *(uint32_t *)(b + ((2 * g + kh) * TL + tl) * 16 + at) = o.pk;
+        if (BS && (l & 3) == 0) *(uint16_t *)(b + TL * 256 + ((k >> 3) * TL + tl) * 16 + 2 * (k & 7)) = f2h((float)o.s16);
+        if (l == 0) *(float *)(b + TL * 288 + 4 * tl) = o.d;
+    }
+}
+
 // ------------------------------------------------------------------ q4_0 --
 // 8 lanes per block; lane k < 4 packs elements 4k..4k+3 with 16+4k..16+4k+3.
 __global__ __launch_bounds__(256) void k_quantize_q4_0(const float *__restrict__ x, size_t xs, uint8_t *__restrict__ y,
@@ -312,6 +351,19 @@ hipError_t launch_quantize_q8_0(const float *x, size_t xs, uint8_t *y, size_t ys
 hipError_t launch_quantize_q8_K(const float *x, size_t xs, uint8_t *y, size_t ys, int64_t n, int rows, hipStream_t s) {
     const int nb = (int)(n / 256);
     hipLaunchKernelGGL(k_quantize_q8_K, dim3((unsigned)(((int64_t)rows * nb + 3) / 4)), dim3(256), 0, s, x, xs, y, ys, nb, rows);
+    return hipGetLastError();
+}
+template <int QT>
+static void q8kt_go(const float *x, size_t xs, uint8_t *y, int nb, int rows, int wtype, hipStream_t s) {
+    const dim3 grid((unsigned)(((int64_t)(rows + QT - 1) / QT * nb + 3) / 4));
+    if (wtype == Q6_K) hipLaunchKernelGGL((k_quantize_q8_K_tile<true, false, QT>), grid, dim3(256), 0, s, x, xs, y, nb, rows);
+    else hipLaunchKernelGGL((k_quantize_q8_K_tile<false, true, QT>), grid, dim3(256), 0, s, x, xs, y, nb, rows);
+}
+// four superblocks per wave once that still fills the chip's 8192 waves
+hipError_t launch_quantize_q8_K_tile(const float *x, size_t xs, uint8_t *y, int64_t n, int rows, int wtype, hipStream_t s) {
+    const int nb = (int)(n / 256);
+    if ((int64_t)rows * nb >= 8192) q8kt_go<4>(x, xs, y, nb, rows, wtype, s);
+    else q8kt_go<1>(x, xs, y, nb, rows, wtype, s);
     return hipGetLastError();
 }
 hipError_t launch_quantize_q4_0(const float *x, size_t xs, uint8_t *y, size_t ys, int64_t n, int rows, hipStream_t s) {

@@ -247,6 +247,10 @@ hipError_t launch_mm_few_ready(const g4h_tensor &W, const FewAct &a, int M, floa
 bool mmk_capable(int type);
 void mmk_describe(const g4h_tensor &W, int M, char *buf, size_t len);
 void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len);
+// x fp32 (quantized here into k_mmk_tile's layout, ws: M rows of 292 bytes per
+// superblock, 64-byte aligned): the bits of quantizing to q8_K rows first
+hipError_t launch_matmul_mfma_kx(const g4h_tensor &W, const float *x, size_t xs, int M, float *Y, uint8_t *ws, hipStream_t s);
+hipError_t launch_quantize_q8_K_tile(const float *x, size_t xs, uint8_t *y, int64_t n, int rows, int wtype, hipStream_t s);
 hipError_t launch_matmul_mfma_k(const g4h_tensor &W, const uint8_t *act, size_t stride, int M, float *Y, hipStream_t s);
 
 // k_attn.hip

@@ -228,3 +228,24 @@ def test_kquant_fused_quantizer_equals_prequantized(gpu, oracle, name, qt):
     a = gpu_matmul(gpu, t, x=x, nb=45, path=2)
     b = gpu_matmul(gpu, t, act=oracle.prep_act(qt, x), nb=45, path=2)
     assert np.array_equal(bits(a), bits(b))
+
+
+@pytest.mark.parametrize("name,qt", KQ)
+@pytest.mark.parametrize("rows,cols", [(4100, 768), (4100, 2560), (33, 256)])
+def test_kquant_tile_kernel_equals_given_rows(gpu, oracle, name, qt, rows, cols):
+    """fp32 tokens (k_mmk_tile, quantized in operand order, one or two token
+    tiles per wave) give the bits of the same tokens as q8_K rows (k_mmk), and
+    a token the same bits in any batch: token counts off the 32-token tile,
+    with and without a second tile in the last workgroup, ragged rows, fewer
+    superblocks than waves and a last round that only some waves have."""
+    w, x, t = _setup(gpu, qt, rows, cols, 161, seed=rows + qt)
+    act = oracle.prep_act(qt, x)
+    full = gpu_matmul(gpu, t, x=x, nb=161, path=2)
+    assert_close(full, oracle_matmul(oracle, qt, w, x), f"{name} {rows}x{cols}")
+    for m in (1, 20, 32, 33, 64, 129, 161):
+        a = gpu_matmul(gpu, t, x=x[:m].copy(), nb=m, path=2)
+        b = gpu_matmul(gpu, t, act=act[:m].copy(), nb=m, path=2)
+        assert np.array_equal(bits(a), bits(full[:m])), f"{name} M={m}"
+        assert np.array_equal(bits(b), bits(full[:m])), f"{name} M={m}: given rows"
+    if rows == 4100:
+        assert "mt=2" in gpu.matmul_describe(t, 129, 2) and "mt=1" in gpu.matmul_describe(t, 33, 2)
