@@ -371,19 +371,24 @@ __global__ __launch_bounds__(64 * TM * TN, 2) void k_mm_lds(g4h_tensor W, const 
 
 // Few tokens (M <= 64): 16-row strips.  A workgroup of 4 waves owns 16 weight
 // rows and every token, so each weight byte is read from HBM once per call;
-// there is no LDS staging and no barrier until the final sum.  Wave w takes
-// the blocks of residue pair w (blocks 8 j + 2 w, 8 j + 2 w + 1: a "pair
-// step").  Per pair step and lane: one 16-byte weight load (q8_0; 8 bytes of
-// nibbles for q4_0) covering both blocks of its row (lane groups 0, 1 block
-// 2 p, groups 2, 3 block 2 p + 1), one 2-byte weight scale, one 16-byte
-// activation load per 16-token tile and one 8-byte load of four tiles'
-// activation scales.  A wave keeps the loads of FEW_AHEAD pair steps in
+// there is no barrier until the final sum.  Wave w takes the blocks of residue
+// pair w (blocks 8 j + 2 w, 8 j + 2 w + 1: a "pair step").
+//
+// What bounded it: the L1 serves one 64-byte access per clock, and an MFMA
+// operand loaded straight from memory has adjacent lanes in different rows, an
+// access per lane (400 accesses per pair step of 64 tokens).  So the
+// activations are laid out in operand order, the weights of a pair step are
+// loaded four lanes to a row (q8_0: the two blocks' halves of each plane; q4_0:
+// two pair steps per load) and turned into the operand through LDS of the
+// wave's own, and, for rows of whole 8-block groups (SV), so are the scales of
+// four pair steps at a time (other rows load a 2-byte scale per lane): about
+// 110 accesses per step.  A wave keeps the loads of FEW_AHEAD pair steps in
 // flight: step k + FEW_AHEAD's loads go out before step k multiplies.
-// One v_permlane32_swap per dword pair turns the loaded halves into the
-// operands of the two blocks' int8 MFMAs (lane group g then holds slice
-// sigma(g) of the block: (0, 2, 1, 3) for q8_0, g for q4_0), and the
-// activations are laid out so that each lane's 16 bytes are its slice of both
-// blocks (k_quantize_few).  Per block and 16 x 16 tile: one
+// One v_permlane32_swap per dword pair turns the operand's halves into those
+// of the two blocks' int8 MFMAs (lane group g then holds slice sigma(g) of the
+// block: (0, 2, 1, 3) for q8_0, g for q4_0), and the activations are laid out
+// so that each lane's 16 bytes are its slice of both blocks
+// (k_quantize_planar).  Per block and 16 x 16 tile: one
 // v_mfma_i32_16x16x32_i8 for the exact block sums, one v_mfma_f32_16x16x16_f16
 // for the exact scale product d_a * d_w (one non-zero k per lane group picks
 // the block and tile), and an fma into the tile's accumulator -- the
@@ -391,7 +396,7 @@ __global__ __launch_bounds__(64 * TM * TN, 2) void k_mm_lds(g4h_tensor W, const 
 //
 // Activation layout for M <= 64 (MT 16-token tiles, np = ceil(nb / 2) block
 // pairs, padding tokens and the padding block zero):
-//   qa [np][MT][16 tok][4 slices][2 blocks][8 bytes]
+//   qa [np][MT][4 slices][16 tok][2 blocks][8 bytes]
 //   da [np][16 tok][2 blocks][4 tiles] fp16 (tile slots past MT zero)
 constexpr int MMF_MAXM = 64;
 
@@ -425,14 +430,27 @@ size_t mm_few_bytes(int M, int64_t ncols) {
 // q8_0 4096x4096 at 32 / 64 tokens 12.95 -> 11.79 / 16.36 -> 14.89; q4_0
 // 2560x10240 at 1 token 22.4 -> 18.4; q4_0 20480x2560 at 32 tokens 35.0 ->
 // 25.1; q8_0 2048x2048 at 1 token 9.86 -> 7.58.  A window of 8 steps was
-// slower at 64 tokens (16.0 us).
+// slower at 64 tokens (16.0 us).  Four token tiles keep three steps in flight:
+// 158 registers, three waves per SIMD (four steps: 182, two waves; q4_0
+// 20480x2560 28.1 -> 24.9 us).
+// Coalesced weights and scales and the slice-major activations against the
+// operands straight from memory (same calls, us): q8_0 4096x4096 at 16 / 64
+// tokens 10.7 / 14.6 -> 9.2 / 13.6; q4_0 20480x2560 at 16 / 32 / 64 tokens 22.5
+// / 26.1 / 32.4 -> 15.8 / 18.6 / 24.9; q4_0 2560x10240 19.2 (16) / 27.7 (64) ->
+// 13.8 / 22.4.  At 64 tokens the VALU issue of the epilogues (10.5 us) and the
+// matrix cores (5.3 us) bound the q4_0 20480x2560 call next.
 constexpr int FEW_CHUNK = 16, FEW_AHEAD = 4;
 
-template <int WT, int MT>
+template <int WT, int MT, bool SV>
 __global__ __launch_bounds__(256) void k_mm_few(g4h_tensor W, const int8_t *__restrict__ qa,
                                                 const uint16_t *__restrict__ da, int M, float *__restrict__ Y) {
     using WV = std::conditional_t<WT == Q8_0, v4i, v2i>;
     __shared__ float red[3 * MT * 4 * 64];
+    // a wave's weight operands: q8_0 four lane groups x 16 rows x 16 bytes, q4_0
+    // two steps x four lane groups x 16 rows x 8 bytes (strides off the banks)
+    constexpr int GST = WT == Q8_0 ? 288 : 144, PST = 4 * 144 + 32;
+    constexpr int WLDS = WT == Q8_0 ? 4 * GST : 2 * PST, SLDS = 16 * 80;
+    __shared__ __align__(16) uint8_t wls[4][WLDS], sls[4][SV ? SLDS : 16];
     // the wave index in a scalar register: the first lane's thread index / 64
     // (the compiler folds a readfirstlane of threadIdx.x / 64 itself away and
     // then keeps the value in a vector register).  Every per-step branch and
@@ -440,40 +458,67 @@ __global__ __launch_bounds__(256) void k_mm_few(g4h_tensor W, const int8_t *__re
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t) >> 6;
     const int li = lane & 15, kg = lane >> 4;
+    const int lr = lane >> 2, lq = lane & 3;                                // weight loads: row, quarter
     const int nb = (int)W.nb, np = (nb + 1) >> 1;
     const int nj = (np - wave + 3) >> 2;                                    // this wave's pair steps
-    const int64_t row = min((int64_t)blockIdx.x * 16 + li, W.nrows - 1);
+    const int64_t row = min((int64_t)blockIdx.x * 16 + li, W.nrows - 1), lrow = min((int64_t)blockIdx.x * 16 + lr, W.nrows - 1);
+    uint8_t *wl = wls[wave], *sl_ = sls[wave];
     // the slice of a block this lane group feeds the int8 MFMA after the swap
     const int sl = WT == Q8_0 ? ((kg & 1) << 1) | (kg >> 1) : kg;
     // per-lane 32-bit byte offsets, fixed over the loop; the per-step part is
-    // uniform (the launch keeps the weight planes under 4 GB).  q8_0: lane
-    // group kg takes half kg & 1 of block 2 p + kg / 2 from that half's plane
-    // (common.h); q4_0: bytes 8 kg .. 8 kg + 7 of the pair's 32 nibble bytes.
-    // The weight bytes of an odd last pair's missing block are the next row's
-    // (or, past the last row, the next plane's): loaded, never used.  Its
-    // scale index is clamped to the row.
-    const uint32_t wlane = WT == Q8_0 ? (uint32_t)((uint64_t)row * nb * 16) + 16 * (kg >> 1) + ((kg & 1) ? (uint32_t)(W.ex - W.qs) : 0u)
-                                      : (uint32_t)((uint64_t)row * nb * 16) + 8 * kg;
+    // uniform (the launch keeps the weight planes under 4 GB).  q8_0: quarter
+    // lq is block 2 p + lq % 2's half lq / 2, from that half's plane (common.h);
+    // q4_0: block lq % 2 of step lq / 2.  The weight bytes of an odd last
+    // pair's missing block are the next row's (or, past the last row, the next
+    // plane's): loaded, never used.  Its scale index is clamped to the row.
+    const uint32_t wlane = (uint32_t)((uint64_t)lrow * nb * 16) + 16 * (lq & 1) + (WT == Q8_0 && lq >= 2 ? (uint32_t)(W.ex - W.qs) : 0u);
     const uint32_t slane1 = (uint32_t)((uint64_t)row * nb * 2) + 2 * (kg & 1), slane0 = slane1 - 2 * (kg & 1);
-    const uint32_t alane = li * 64 + 16 * sl, dlane = 8 * (2 * li + (kg & 1));
+    const uint32_t svlane = (uint32_t)((uint64_t)lrow * nb * 2);
+    const uint32_t alane = 16 * li + 256 * sl, dlane = 8 * (2 * li + (kg & 1));
 
     struct Op {
-        WV w;
         v4i a[MT];
         uint64_t d;
         uint32_t s;
+    };
+    constexpr int UW = WT == Q8_0 ? 1 : 2;                                  // steps per weight load
+    // the weights of steps j .. j + UW - 1, and (SV) the scales of steps j ..
+    // j + 3: lane (row, c) the 8 scales of pairs 4 (j + c) .. 4 (j + c) + 3
+    auto load_w = [&](int j) __attribute__((always_inline)) -> v4i {
+        if constexpr (WT == Q8_0) return *(const v4i *)(W.qs + (size_t)min(4 * j + wave, np - 1) * 32 + wlane);
+        const int p0 = min(4 * j + wave, np - 1), p1 = min(4 * j + 4 + wave, np - 1);
+        return *(const v4i *)(W.qs + (lq >= 2 ? p1 : p0) * 32u + wlane);
+    };
+    auto load_sv = [&](int j) __attribute__((always_inline)) -> v4i {
+        return *(const v4i *)(W.sc + (uint32_t)min(j + lq, (np >> 2) - 1) * 16u + svlane);
+    };
+    auto put_w = [&](const v4i &w) __attribute__((always_inline)) {
+        if constexpr (WT == Q8_0) {
+            *(v4i *)(wl + ((lq >> 1) + 2 * (lq & 1)) * GST + lr * 16) = w;
+        } else {
+            uint8_t *p = wl + (lq >> 1) * PST + 2 * (lq & 1) * GST + lr * 8;
+            *(v2i *)p = w.xy;
+            *(v2i *)(p + GST) = w.zw;
+        }
+    };
+    auto put_sv = [&](const v4i &w) __attribute__((always_inline)) { *(v4i *)(sl_ + lr * 80 + lq * 16) = w; };
+    auto get_w = [&](int k) __attribute__((always_inline)) -> WV {          // step k of the chunk
+        if constexpr (WT == Q8_0) return *(const v4i *)(wl + kg * GST + li * 16);
+        else return *(const v2i *)(wl + (k & 1) * PST + kg * GST + li * 8);
     };
     // pair step j of this wave: pair 4 j + wave, clamped to the last pair
     auto load = [&](int j) __attribute__((always_inline)) -> Op {
         const int p = min(4 * j + wave, np - 1);
         Op o;
-        o.w = *(const WV *)(W.qs + (size_t)p * 32 + wlane);
-        o.s = *(const uint16_t *)(W.sc + (size_t)p * 4 + (2 * p + 1 < nb ? slane1 : slane0));
-        // a step past the wave's last, or the missing block of an odd last
-        // pair, gets weight scale 0: its products add +0 to the accumulator,
-        // which never holds -0, so the sums keep their bits
-        const bool live = j < nj, live1 = live && 2 * p + 1 < nb;            // uniform
-        if (!((kg & 1) ? live1 : live)) o.s = 0;
+        if constexpr (!SV) {
+            o.s = *(const uint16_t *)(W.sc + (size_t)p * 4 + (2 * p + 1 < nb ? slane1 : slane0));
+            // the missing block of an odd last pair gets weight scale 0: its
+            // products add +0 to the accumulator, which never holds -0, so the
+            // sums keep their bits
+            if ((kg & 1) && 2 * p + 1 >= nb) o.s = 0;
+        } else {
+            o.s = 0;
+        }
         static_for<0, MT>([&](auto I) { o.a[I.value] = *(const v4i *)(qa + ((size_t)p * MT + I.value) * 1024 + alane); });
         o.d = *(const uint64_t *)((const uint8_t *)da + (size_t)p * 256 + dlane);
         return o;
@@ -483,14 +528,14 @@ __global__ __launch_bounds__(256) void k_mm_few(g4h_tensor W, const int8_t *__re
     for (int tt = 0; tt < MT; tt++) acc[tt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     const v4i zi = {};
     const v4f zf = {};
-    auto mac = [&](const Op &o) __attribute__((always_inline)) {
+    auto mac = [&](const Op &o, const WV &w, uint32_t s) __attribute__((always_inline)) {
         uint32_t x0, x1, y0, y1;
         if constexpr (WT == Q8_0) {
-            x0 = (uint32_t)o.w[0], x1 = (uint32_t)o.w[1], y0 = (uint32_t)o.w[2], y1 = (uint32_t)o.w[3];
+            x0 = (uint32_t)w[0], x1 = (uint32_t)w[1], y0 = (uint32_t)w[2], y1 = (uint32_t)w[3];
         } else {
             // bytes 8 (kg & 1) .. + 7 of a block: low nibbles are slice kg & 1,
             // high nibbles slice 2 + (kg & 1) (quants.c:542-545), each as q - 8
-            const uint32_t u0 = (uint32_t)o.w[0], u1 = (uint32_t)o.w[1];
+            const uint32_t u0 = (uint32_t)w[0], u1 = (uint32_t)w[1];
             x0 = ((u0 & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;
             x1 = ((u1 & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;
             y0 = (((u0 >> 4) & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;
@@ -507,7 +552,7 @@ __global__ __launch_bounds__(256) void k_mm_few(g4h_tensor W, const int8_t *__re
         // (selects, not branches: lane-divergent ifs here split the loop into
         // exec-masked blocks, across which the compiler kept every step's
         // MFMA results live -- 256 registers and more instead of 84 to 166)
-        const _Float16 sw = __builtin_bit_cast(_Float16, (uint16_t)o.s), zh = (_Float16)0.0f;
+        const _Float16 sw = __builtin_bit_cast(_Float16, (uint16_t)s), zh = (_Float16)0.0f;
         const _Float16 sw0 = kg == 0 ? sw : zh, sw1 = kg == 1 ? sw : zh;
         const v4h hw[2][2] = {{v4h{sw0, zh, zh, zh}, v4h{zh, sw0, zh, zh}}, {v4h{sw1, zh, zh, zh}, v4h{zh, sw1, zh, zh}}};
 #pragma unroll
@@ -529,17 +574,42 @@ __global__ __launch_bounds__(256) void k_mm_few(g4h_tensor W, const int8_t *__re
 
     // a chunk of C pair steps from j0; scheduling barriers keep each step's
     // loads where they are issued and one step's multiplies at a time (left
-    // alone the compiler hoists the chunk's MFMAs and runs out of registers)
+    // alone the compiler hoists the chunk's MFMAs and runs out of registers).
+    // Step k + 1's weight operand goes through LDS while step k multiplies (a
+    // wave's LDS accesses complete in order; the empty asms keep the compiler
+    // from moving them).
     auto chunk = [&](auto Cc, int j0) __attribute__((always_inline)) {
-        constexpr int C = decltype(Cc)::value, A = FEW_AHEAD < C ? FEW_AHEAD : C;
+        constexpr int C = decltype(Cc)::value, AH = MT == 4 ? FEW_AHEAD - 1 : FEW_AHEAD, A = AH < C ? AH : C;
         Op ops[C];
-        static_for<0, A>([&](auto I) { ops[I.value] = load(j0 + I.value); });
+        v4i wr[(C + UW - 1) / UW], sv[(C + 3) / 4];
+        WV wo[C];
+        uint32_t so[C];
+        auto fetch = [&](auto I) __attribute__((always_inline)) {
+            constexpr int k = I.value;
+            if constexpr (SV && k % 4 == 0) sv[k / 4] = load_sv(j0 + k);
+            if constexpr (k % UW == 0) wr[k / UW] = load_w(j0 + k);
+            ops[k] = load(j0 + k);
+        };
+        auto turn = [&](auto I) __attribute__((always_inline)) {
+            constexpr int k = I.value;
+            asm volatile("" ::: "memory");
+            if constexpr (SV && k % 4 == 0) put_sv(sv[k / 4]);
+            if constexpr (k % UW == 0) put_w(wr[k / UW]);
+            asm volatile("" ::: "memory");
+            wo[k] = get_w(k);
+            if constexpr (SV) so[k] = *(const uint16_t *)(sl_ + li * 80 + (k & 3) * 16 + 4 * wave + 2 * (kg & 1));
+            else so[k] = ops[k].s;
+            asm volatile("" ::: "memory");
+        };
+        static_for<0, A>([&](auto I) { fetch(I); });
         __builtin_amdgcn_sched_barrier(0);
+        turn(std::integral_constant<int, 0>{});
         static_for<0, C>([&](auto I) {
             constexpr int k = I.value;
-            if constexpr (k + A < C) ops[k + A] = load(j0 + k + A);
+            if constexpr (k + A < C) fetch(std::integral_constant<int, k + A>{});
             __builtin_amdgcn_sched_barrier(0);
-            mac(ops[k]);
+            if constexpr (k + 1 < C) turn(std::integral_constant<int, k + 1>{});
+            mac(ops[k], wo[k], so[k]);
             __builtin_amdgcn_sched_barrier(0);
         });
     };
@@ -724,10 +794,16 @@ hipError_t launch_few_clear(uint8_t *buf, size_t bytes, hipStream_t s) {
 static hipError_t few_go(const g4h_tensor &W, const int8_t *qa, const uint16_t *da, int M, float *Y, hipStream_t s) {
     const int mt = (M + 15) / 16;
     const dim3 grid((unsigned)((W.nrows + 15) / 16));
+    const bool sv = W.nb % 8 == 0;
 #define G4_MF(T)                                                                                                    \
     if (mt == T) {                                                                                                  \
-        if (W.type == Q8_0) hipLaunchKernelGGL((k_mm_few<Q8_0, T>), grid, dim3(256), 0, s, W, qa, da, M, Y);       \
-        else hipLaunchKernelGGL((k_mm_few<Q4_0, T>), grid, dim3(256), 0, s, W, qa, da, M, Y);                    \
+        if (W.type == Q8_0) {                                                                                       \
+            if (sv) hipLaunchKernelGGL((k_mm_few<Q8_0, T, true>), grid, dim3(256), 0, s, W, qa, da, M, Y);          \
+            else hipLaunchKernelGGL((k_mm_few<Q8_0, T, false>), grid, dim3(256), 0, s, W, qa, da, M, Y);            \
+        } else {                                                                                                    \
+            if (sv) hipLaunchKernelGGL((k_mm_few<Q4_0, T, true>), grid, dim3(256), 0, s, W, qa, da, M, Y);          \
+            else hipLaunchKernelGGL((k_mm_few<Q4_0, T, false>), grid, dim3(256), 0, s, W, qa, da, M, Y);            \
+        }                                                                                                           \
         return hipGetLastError();                                                                                   \
     }
     G4_MF(1) G4_MF(2) G4_MF(3) G4_MF(4)

@@ -62,11 +62,12 @@ __device__ __forceinline__ void q8_store4(const float v[4], int gi, bool own, ui
 
 // k_mm_few's operand layout: the byte offset of codes e .. of (block b, token
 // m) with mt 16-token tiles, and the fp16 index of its scale.  Block pairs
-// outermost, then tiles, then the 16 tokens of a tile, each token's 64 bytes
-// holding codes 0-7 of the even block, 0-7 of the odd one, then 8-15, and so
-// on; the scales in 4 tile slots per (pair, token, block).
+// outermost, then tiles, then the four slices of 8 codes, then the 16 tokens of
+// a tile, each token's 16 bytes holding the slice of the even block, then of
+// the odd one (16 lanes' operand is 256 adjacent bytes); the scales in 4 tile
+// slots per (pair, token, block).
 __device__ __forceinline__ size_t few_q(int64_t b, int m, int mt, int e) {
-    return ((((size_t)(b >> 1) * mt + (m >> 4)) * 16 + (m & 15)) * 64) + 16 * (e >> 3) + 8 * (b & 1) + (e & 7);
+    return ((size_t)(b >> 1) * mt + (m >> 4)) * 1024 + 256 * (e >> 3) + 16 * (m & 15) + 8 * (b & 1) + (e & 7);
 }
 __device__ __forceinline__ size_t few_d(int64_t b, int m) { return ((((size_t)(b >> 1) * 16 + (m & 15)) * 2 + (b & 1)) * 4) + (m >> 4); }
 // q8_store4 of token m's row into that layout
