@@ -139,38 +139,43 @@ hipError_t launch_gemv_float_x(int wtype, const uint8_t *W, size_t ws, int64_t n
 }
 
 // Prompt batches on the matrix cores (g4h_matmul path 2): Y[t][r] = sum_k
-// W[r][k] a[t][k], one v_mfma_f32_16x16x32_f16 / _bf16 per 32 columns of a
-// 16-token x 16-row tile.  The operands are the GEMV family's: f16 weights
+// W[r][k] a[t][k], one v_mfma_f32_32x32x16_f16 / _bf16 per 16 columns of a
+// 32-token x 32-row tile.  The operands are the GEMV family's: f16 weights
 // against f16-rounded activations, bf16 weights against bf16-rounded ones
 // (prep_act's AC_F16 / AC_BF16, model.c:163-180), so every product is exact
 // in fp32 (11 x 11 or 8 x 8 significant bits) and only the fp32 order of the
 // sums differs from the CPU's and from the GEMV family's (within the path's
-// tolerance).  A workgroup owns MT x NT such tiles; its MMF_W waves split the
-// 64-column chunks (wave w takes chunks w, w + MMF_W, ..., each chained into
-// its accumulators in increasing order, a last partial chunk included) and
-// the waves' tiles are added in wave order through LDS: a token's result
-// depends neither on the batch size nor on MT and NT.
+// tolerance).  A workgroup owns MR tokens x NR rows; its MMF_W waves split the
+// 16-column steps (wave w takes steps w, w + MMF_W, ..., each chained into its
+// accumulators in increasing order) and the waves' tiles are added in wave
+// order through LDS: a token's result depends neither on the batch size nor on
+// MR and NR (a tile of 16 repeats its rows in the MFMA's other half).
 //
 // What bounds it: the CU's L1 serves one 64-byte access per clock, and lanes
 // reading different rows are one access each.  An MFMA operand has adjacent
 // lanes in different rows, so loading it straight from memory costs 57
-// accesses per 1 KB instruction (measured).  Here adjacent lanes load adjacent
-// 16 bytes of one row, fp32 activations are rounded on the way, and each wave
-// turns its own chunk into operands through LDS of its own (no barrier), the
-// next chunk's loads in flight meanwhile.  LDS rows of 128 bytes, the 16-byte
+// accesses per 1 KB instruction (measured).  Here the workgroup loads chunks
+// of 256 columns, adjacent lanes adjacent 16 bytes of a row, rounds fp32
+// activations on the way into LDS and reads the operands there, the next
+// chunk's loads in flight meanwhile.  LDS rows of 512 bytes, the 16-byte
 // columns of row r at column ^ (r & 7).  Measured against operands loaded
-// straight from memory for 32 x 32 tiles (fp32 tokens, us): f16 4096 x 4096 at
-// 64 / 201 / 512 tokens 29.4 / 83.0 / 177.9 -> 15.9 / 23.9 / 46.7 (141, 282 and
-// 368 TFLOP/s), f16 256 x 2048 at 64 tokens 13.4 -> 5.6, bf16 2560 x 10240 at
-// 64 / 300 tokens 74.8 / 212.8 -> 33.6 / 51.5.
-// Operand layout: lane l holds A[l % 16][8 (l / 16) .. + 7] and
-// B[l % 16][8 (l / 16) .. + 7]; C[i][j] with j = l % 16 (weight row), i = 4
-// (l / 16) + r (token).
+// straight from memory for 32 x 32 tiles, the same bits (fp32 tokens, us): f16
+// 4096 x 4096 at 9 / 64 / 201 / 512 tokens 19.5 / 29.4 / 83.0 / 177.9 -> 10.9 /
+// 16.8 / 25.7 / 55.5 (310 TFLOP/s), f16 256 x 2048 at 64 13.4 -> 5.4, bf16 2560 x
+// 10240 at 64 / 300 tokens 74.8 / 212.8 -> 33.6 / 60.2.  Each wave turning its
+// own 64-column chunks into operands without a barrier was faster at 512
+// tokens (46.7 us), but its other order of the sums moves every 16-bit
+// projection of a model by a last bit.
+// Operand layout: lane l holds A[l % 32][8 (l / 32) .. + 7] and
+// B[l % 32][8 (l / 32) .. + 7]; C[i][j] with j = l % 32 (weight row), i = 8
+// (r / 4) + 4 (l / 32) + r % 4 (token).
 typedef _Float16 mf_v8h __attribute__((ext_vector_type(8)));
 typedef __bf16 mf_v8bf __attribute__((ext_vector_type(8)));
-typedef float mf_v4f __attribute__((ext_vector_type(4)));
+typedef float mf_v16f __attribute__((ext_vector_type(16)));
+typedef uint32_t mf_v4u __attribute__((ext_vector_type(4)));
 
 constexpr int MMF_W = 8;              // waves per workgroup
+constexpr int MMF_KC = 256;           // columns per chunk: two steps per wave
 
 // two fp32 activations rounded with k_act_float's arithmetic by the packed
 // conversion instructions (round to nearest even; bf16-rounded rows keep their
@@ -188,187 +193,175 @@ __device__ __forceinline__ uint32_t mmf_round2(uint32_t x, uint32_t y) {
 // A32: activation rows of fp32 (row stride `as` bytes), rounded on the way to
 // LDS; else f16 rows.  Workgroup b runs on XCD b % 8: the token tiles of one
 // row tile go to one XCD, consecutively, and find its weights in that XCD's L2.
-template <int WT, bool A32, int MT, int NT>
+template <int WT, bool A32, int MR, int NR>
 __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restrict__ W, size_t ws, int64_t nrows, int64_t ncols,
                                                          const uint8_t *__restrict__ act, size_t as, int M, float *__restrict__ Y,
                                                          int ntok) {
-    constexpr int AL = A32 ? 4 * MT : 2 * MT, WL = 2 * NT;          // 16-byte loads per lane and chunk
-    // chunks per stage: 40 to 96 registers of loads, at most 16 KB of LDS per wave
-    constexpr int CR = AL + WL >= 12 ? 1 : AL + WL >= 8 ? 2 : 4, CH = CR * (MT + NT) <= 8 ? CR : CR / 2;
-    constexpr int LW = CH * (MT + NT) * 2048;                       // LDS bytes per wave
-    constexpr int PW = MT * NT * 1024;                              // partial tiles per wave
-    __shared__ __align__(16) uint8_t lds[MMF_W * (LW > PW ? LW : PW)];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x) >> 6;
-    const int li = lane & 15, kg = lane >> 4;
+    constexpr int MT = (MR + 31) / 32, NT = (NR + 31) / 32, NTH = 64 * MMF_W, RB = 2 * MMF_KC;
+    constexpr int AU = A32 ? 64 : 32, AL = MR * AU / NTH, WL = NR * 32 / NTH;   // 16-byte pieces per row, loads per thread
+    static_assert(MR * AU % NTH == 0 && NR * 32 % NTH == 0, "whole loads");
+    constexpr int BUF = (MR + NR) * RB, PART = MMF_W * MT * NT * 4096;
+    __shared__ __align__(16) uint8_t lds[2 * BUF > PART ? 2 * BUF : PART];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t) >> 6;
+    const int li = lane & 31, kh = lane >> 5;
     const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
-    const int64_t n0 = ((int64_t)(l / ntok) * 8 + x) * (16 * NT);
-    const int m0 = (l % ntok) * (16 * MT);
+    const int64_t n0 = ((int64_t)(l / ntok) * 8 + x) * NR;
+    const int m0 = (l % ntok) * MR;
     if (n0 >= nrows) return;                                        // uniform over the workgroup
-    uint8_t *sl = lds + wave * LW;
-    // 16-byte loads: eight lanes per 128-byte row of W (and of f16
-    // activations), sixteen per 256-byte fp32 row
-    const int wr = lane >> 3, wc = lane & 7, ar = A32 ? lane >> 4 : wr, ac = A32 ? lane & 15 : wc;
-    constexpr int AQ = A32 ? 4 : 8;                                 // activation rows per load
+    const int wr = t >> 5, wc = t & 31, ar = A32 ? t >> 6 : wr, ac = A32 ? t & 63 : wc;
+    constexpr int WQ = NTH / 32, AQ = NTH / AU;                     // rows per load of the workgroup
     const uint8_t *wp[WL], *ap[AL];
 #pragma unroll
-    for (int q = 0; q < WL; q++) wp[q] = W + (size_t)min(n0 + 8 * q + wr, nrows - 1) * ws + 16 * wc;
+    for (int q = 0; q < WL; q++) wp[q] = W + (size_t)min(n0 + WQ * q + wr, nrows - 1) * ws;
 #pragma unroll
-    for (int q = 0; q < AL; q++) ap[q] = act + (size_t)min(m0 + AQ * q + ar, M - 1) * as + 16 * ac;
-    const int nc = (int)(ncols >> 6);                               // whole chunks
-    const int nj = (nc - wave + MMF_W - 1) / MMF_W;                 // this wave's (uniform)
+    for (int q = 0; q < AL; q++) ap[q] = act + (size_t)min(m0 + AQ * q + ar, M - 1) * as;
+    const int ns = (int)(ncols >> 4), nc = (ns + 15) >> 4;          // steps, chunks
+    const uint32_t wlast = (uint32_t)ncols * 2 - 16, alast = (uint32_t)ncols * (A32 ? 4 : 2) - 16;
     struct Stage {
-        uint4 w[CH][WL], a[CH][AL];
+        mf_v4u w[WL], a[AL];
     };
-    Stage S;
-    auto load = [&](int j0) __attribute__((always_inline)) {
+    // stages of loads in flight, 48 to 96 registers (64 x 64 workgroups were
+    // slower with two: f16 4096 x 4096 at 512 tokens 55.6 / 58.7 us)
+    constexpr int D = AL + WL >= 12 ? 1 : AL + WL >= 8 ? 2 : 4;
+    Stage st[D];
+    auto load = [&](Stage &S, int c) __attribute__((always_inline)) {   // past the row's end its last piece again, never used
+        const uint32_t wo = min((uint32_t)c * RB + 16 * wc, wlast), ao = min((uint32_t)c * (A32 ? 2 * RB : RB) + 16 * ac, alast);
 #pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const size_t k = (size_t)(wave + MMF_W * min(j0 + c, nj - 1));
+        for (int q = 0; q < WL; q++) S.w[q] = *(const mf_v4u *)(wp[q] + wo);
 #pragma unroll
-            for (int q = 0; q < WL; q++) S.w[c][q] = *(const uint4 *)(wp[q] + 128 * k);
+        for (int q = 0; q < AL; q++) S.a[q] = *(const mf_v4u *)(ap[q] + ao);
+        // the loads go out here: left alone the compiler sinks them to their
+        // use behind the multiplies
+        asm volatile("" ::: "memory");
+    };
+    auto put = [&](const Stage &S, int b) __attribute__((always_inline)) {
+        uint8_t *la = lds + b * BUF, *lw = la + MR * RB;
 #pragma unroll
-            for (int q = 0; q < AL; q++) S.a[c][q] = *(const uint4 *)(ap[q] + (A32 ? 256 : 128) * k);
+        for (int q = 0; q < WL; q++) {
+            const int r = WQ * q + wr;
+            *(mf_v4u *)(lw + r * RB + 16 * (wc ^ (r & 7))) = S.w[q];
         }
-    };
-    auto put = [&](int c) __attribute__((always_inline)) {          // chunk c of the stage into LDS
-        uint8_t *la = sl + c * (MT + NT) * 2048, *lw = la + MT * 2048;
-#pragma unroll
-        for (int q = 0; q < WL; q++) *(uint4 *)(lw + (8 * q + wr) * 128 + 16 * (wc ^ wr)) = S.w[c][q];
 #pragma unroll
         for (int q = 0; q < AL; q++) {
-            const uint4 v = S.a[c][q];
+            const mf_v4u v = S.a[q];
             const int r = AQ * q + ar;
             if constexpr (A32)
-                *(uint2 *)(la + r * 128 + 16 * ((ac >> 1) ^ (r & 7)) + 8 * (ac & 1)) =
+                *(uint2 *)(la + r * RB + 16 * ((ac >> 1) ^ (r & 7)) + 8 * (ac & 1)) =
                     make_uint2(mmf_round2<WT>(v.x, v.y), mmf_round2<WT>(v.z, v.w));
             else
-                *(uint4 *)(la + r * 128 + 16 * (ac ^ (r & 7))) = v;
+                *(mf_v4u *)(la + r * RB + 16 * (ac ^ (r & 7))) = v;
         }
     };
-    mf_v4f acc[MT][NT];
+    mf_v16f acc[MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int n = 0; n < NT; n++) acc[m][n] = mf_v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    auto mul = [&](int c) __attribute__((always_inline)) {
-        const uint8_t *la = sl + c * (MT + NT) * 2048 + li * 128, *lw = la + MT * 2048;
+        for (int n = 0; n < NT; n++) acc[m][n] = mf_v16f{};
+    auto mul = [&](int b, int c) __attribute__((always_inline)) {
+        const uint8_t *la = lds + b * BUF, *lw = la + MR * RB;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const int o = 16 * ((4 * h + kg) ^ (li & 7));
-            uint4 a[MT], w[NT];
+            const int q = wave + MMF_W * h;                         // the chunk's step (uniform)
+            mf_v4u a[MT], w[NT];
 #pragma unroll
-            for (int m = 0; m < MT; m++) a[m] = *(const uint4 *)(la + 2048 * m + o);
+            for (int m = 0; m < MT; m++) {
+                const int r = MR < 32 ? li & (MR - 1) : 32 * m + li;
+                a[m] = *(const mf_v4u *)(la + r * RB + 16 * ((2 * q + kh) ^ (r & 7)));
+            }
 #pragma unroll
-            for (int n = 0; n < NT; n++) w[n] = *(const uint4 *)(lw + 2048 * n + o);
+            for (int n = 0; n < NT; n++) {
+                const int r = NR < 32 ? li & (NR - 1) : 32 * n + li;
+                w[n] = *(const mf_v4u *)(lw + r * RB + 16 * ((2 * q + kh) ^ (r & 7)));
+            }
 #pragma unroll
             for (int m = 0; m < MT; m++)
 #pragma unroll
                 for (int n = 0; n < NT; n++) {
+                    if (16 * c + q >= ns) break;                   // uniform
                     if constexpr (WT == F16)
-                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mf_v8h, a[m]), __builtin_bit_cast(mf_v8h, w[n]),
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mf_v8h, a[m]), __builtin_bit_cast(mf_v8h, w[n]),
                                                                            acc[m][n], 0, 0, 0);
                     else
-                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mf_v8bf, a[m]),
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mf_v8bf, a[m]),
                                                                             __builtin_bit_cast(mf_v8bf, w[n]), acc[m][n], 0, 0, 0);
                 }
         }
     };
-    // a wave's LDS accesses complete in order; the empty asms keep the
-    // compiler from moving any access across a hand-over
-    if (nj > 0) {
-        load(0);
-        for (int j0 = 0; j0 < nj; j0 += CH) {
-            const int left = nj - j0;                               // uniform
+    // chunk c: its stage into one LDS buffer, the stage reloaded D chunks on,
+    // one barrier, the multiplies; the other buffer's readers have passed the
+    // barrier before it.  Every load is issued on every pass, so the memory
+    // counter waits before a store cover only the stage stored.
 #pragma unroll
-            for (int c = 0; c < CH; c++) put(c);
-            asm volatile("" ::: "memory");
-            load(j0 + CH);
-            asm volatile("" ::: "memory");
+    for (int d = 0; d < D; d++) load(st[d], d);
+    for (int c0 = 0; c0 < nc; c0 += D) {                            // uniform
 #pragma unroll
-            for (int c = 0; c < CH; c++)
-                if (c < left) mul(c);
-            asm volatile("" ::: "memory");
+        for (int d = 0; d < D; d++) {
+            if (c0 + d >= nc) break;
+            put(st[d], (c0 + d) & 1);
+            load(st[d], c0 + d + D);
+            lds_barrier();
+            mul((c0 + d) & 1, c0 + d);
         }
-    }
-    // a last chunk of ncols % 64 columns, zeros past them
-    if ((ncols & 63) && wave == nc % MMF_W) {                       // uniform
-        const int lw = (int)(ncols & 63) / 8, la = A32 ? 2 * lw : lw;   // 16-byte columns
-        const size_t k = nc;
-        const uint4 z = make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int q = 0; q < WL; q++) {
-            S.w[0][q] = *(const uint4 *)(wp[q] + 128 * k - 16 * (wc < lw ? 0 : wc));   // past them the chunk's first column
-            if (wc >= lw) S.w[0][q] = z;
-        }
-#pragma unroll
-        for (int q = 0; q < AL; q++) {
-            S.a[0][q] = *(const uint4 *)(ap[q] + (A32 ? 256 : 128) * k - 16 * (ac < la ? 0 : ac));
-            if (ac >= la) S.a[0][q] = z;
-        }
-        put(0);
-        asm volatile("" ::: "memory");
-        mul(0);
     }
     __syncthreads();
-    float *part = (float *)lds;                                     // [wave][register][lane]
+    float *part = (float *)lds;                                     // [wave][tile register][lane]
 #pragma unroll
     for (int m = 0; m < MT; m++)
 #pragma unroll
         for (int n = 0; n < NT; n++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) part[(wave * MT * NT * 4 + (m * NT + n) * 4 + r) * 64 + lane] = acc[m][n][r];
+            for (int r = 0; r < 16; r++) part[((wave * MT * NT + m * NT + n) * 16 + r) * 64 + lane] = acc[m][n][r];
     __syncthreads();
-    // the waves' tiles in wave order; wave w stores registers w, w + 8, ..
-    for (int u = wave; u < MT * NT * 4; u += MMF_W) {
+    // the waves' tiles in wave order; wave w stores tile registers w, w + 8, ..
+    for (int u = wave; u < MT * NT * 16; u += MMF_W) {
         float o = part[u * 64 + lane];
 #pragma unroll
-        for (int w = 1; w < MMF_W; w++) o += part[(w * MT * NT * 4 + u) * 64 + lane];
-        const int m = m0 + 16 * (u / (4 * NT)) + 4 * kg + (u & 3);
-        const int64_t n = n0 + 16 * ((u >> 2) % NT) + li;
-        if (m < M && n < nrows) Y[(size_t)m * nrows + n] = o;
+        for (int w = 1; w < MMF_W; w++) o += part[(w * MT * NT * 16 + u) * 64 + lane];
+        const int r = u & 15, i = 32 * (u / (16 * NT)) + 8 * (r >> 2) + 4 * kh + (r & 3), j = 32 * ((u >> 4) % NT) + li;
+        if (i < MR && j < NR && m0 + i < M && n0 + j < nrows) Y[(size_t)(m0 + i) * nrows + n0 + j] = o;
     }
 }
 
-// Tiles of a call: the shape with the least L1 traffic per CU, rounds of
-// workgroups x the bytes a workgroup loads per column (fp32 activation rows 4,
-// f16 rows and weights 2 each).  Measured with fp32 activations (us): f16 4096
-// x 4096 at 64 tokens 2 x 2 15.9, 4 x 1 21.0, 2 x 4 20.2; at 128 tokens 2 x 4
-// 19.0, 4 x 2 22.9; at 201 tokens 4 x 4 25.1, 2 x 4 32.0, 4 x 2 36.2.
-static void mmf_tiles(bool a32, int64_t nrows, int M, int &mt, int &nt, int &ntok, int64_t &grid) {
-    const int tm = (M + 15) / 16;
-    const int64_t tn = (nrows + 15) / 16;
+// Tokens and rows per workgroup: the shape with the least L1 traffic per CU,
+// rounds of workgroups x the bytes a workgroup loads per column (fp32
+// activation rows 4, f16 rows and weights 2 each).  Measured with fp32
+// activations (us, 64-column chunks): f16 4096 x 4096 at 64 tokens 32 x 32 15.9,
+// 64 x 16 21.0, 32 x 64 20.2; at 128 tokens 32 x 64 19.0, 64 x 32 22.9; at 201
+// tokens 64 x 64 25.1, 32 x 64 32.0, 64 x 32 36.2.
+static void mmf_tiles(bool a32, int64_t nrows, int M, int &mr, int &nr, int &ntok, int64_t &grid) {
     int64_t best = INT64_MAX;
-    for (int m = tm > 2 ? 4 : tm; m >= 1; m >>= 1)
-        for (int n = 4; n >= 1; n >>= 1) {
-            const int64_t cost = ((tm + m - 1) / m * ((tn + n - 1) / n) + 255) / 256 * ((a32 ? 2 : 1) * m + n);
-            if (cost < best) best = cost, mt = m, nt = n;
+    for (int m = M > 32 ? 64 : M > 16 ? 32 : 16; m >= 16; m >>= 1)
+        for (int n = 64; n >= 16; n >>= 1) {
+            const int64_t cost = ((M + m - 1) / m * ((nrows + n - 1) / n) + 255) / 256 * ((a32 ? 2 : 1) * m + n);
+            if (cost < best) best = cost, mr = m, nr = n;
         }
-    ntok = (tm + mt - 1) / mt;
-    grid = ((tn + nt - 1) / nt + 7) / 8 * 8 * ntok;
+    ntok = (M + mr - 1) / mr;
+    grid = ((nrows + nr - 1) / nr + 7) / 8 * 8 * ntok;
 }
 
 void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len) {
-    int mt, nt, ntok;
+    int mr, nr, ntok;
     int64_t grid;
-    mmf_tiles(true, nrows, M, mt, nt, ntok, grid);
-    snprintf(buf, len, "k_mm_float<%s,mt=%d,nt=%d> grid=%lld block=%d (matrix cores, 16x16 tiles, %d waves split the columns)",
-             wtype == F16 ? "f16" : "bf16", mt, nt, (long long)grid, 64 * MMF_W, MMF_W);
+    mmf_tiles(true, nrows, M, mr, nr, ntok, grid);
+    snprintf(buf, len, "k_mm_float<%s,%dx%d> grid=%lld block=%d (matrix cores, %d waves split the columns)",
+             wtype == F16 ? "f16" : "bf16", mr, nr, (long long)grid, 64 * MMF_W, MMF_W);
 }
 
 template <int WT, bool A32>
 static hipError_t mmf_go(const uint8_t *W, size_t ws, int64_t nrows, int64_t ncols, const uint8_t *a, size_t ab, int M, float *Y,
                          hipStream_t s) {
-    int mt, nt, ntok;
+    int mr, nr, ntok;
     int64_t grid;
-    mmf_tiles(A32, nrows, M, mt, nt, ntok, grid);
-    if (grid > 0x7fffffff) return hipErrorInvalidValue;
-#define G4_MMF(MT_, NT_)                                                                                                       \
-    if (mt == MT_ && nt == NT_) {                                                                                              \
-        hipLaunchKernelGGL((k_mm_float<WT, A32, MT_, NT_>), dim3((unsigned)grid), dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, \
+    mmf_tiles(A32, nrows, M, mr, nr, ntok, grid);
+    if (grid > 0x7fffffff || ncols >= (int64_t)1 << 29) return hipErrorInvalidValue;
+#define G4_MMF(MR_, NR_)                                                                                                       \
+    if (mr == MR_ && nr == NR_) {                                                                                              \
+        hipLaunchKernelGGL((k_mm_float<WT, A32, MR_, NR_>), dim3((unsigned)grid), dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, \
                            M, Y, ntok);                                                                                        \
         return hipGetLastError();                                                                                              \
     }
-    G4_MMF(1, 1) G4_MMF(1, 2) G4_MMF(1, 4) G4_MMF(2, 1) G4_MMF(2, 2) G4_MMF(2, 4) G4_MMF(4, 1) G4_MMF(4, 2) G4_MMF(4, 4)
+    G4_MMF(16, 16) G4_MMF(16, 32) G4_MMF(16, 64) G4_MMF(32, 16) G4_MMF(32, 32) G4_MMF(32, 64) G4_MMF(64, 16) G4_MMF(64, 32)
+    G4_MMF(64, 64)
 #undef G4_MMF
     return hipErrorInvalidValue;
 }

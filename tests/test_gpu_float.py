@@ -165,8 +165,9 @@ def test_matrix_cores_token_results_independent_of_batch(gpu, oracle, name, wt):
 def test_matrix_cores_tile_shapes_same_bits(gpu, oracle, name, wt, rows, cols):
     """k_mm_float's tile shape follows the row and token counts; every shape
     gives a token the same bits (compared with the largest batch), from fp32
-    and from prepared rows, also with columns that leave a partial 64-column
-    chunk (48, 32 or 16 of them), rows and tokens off the 16-row tiles, and
+    and from prepared rows, also with columns that leave a partial 256-column
+    chunk (steps that some waves have and others do not), one chunk and an odd
+    number of them, rows and tokens off the 16-row tiles, and
     activations that round to subnormal, infinite or zero values."""
     from g4run_amd import synth
     w = _weights(wt, rows, cols, seed=rows + cols)
