@@ -13,20 +13,18 @@
 // weighted values and the spans added in order -- has the same operands in
 // the same order whatever other tokens share the batch: a token's row has
 // the same bits in any batch, alone included.
-//   scores   grid (KV head x tile, 128-position chunk), 4 waves x 32
-//            positions: S = fp16(q) . K_j (model.c:530-538, no 1/sqrt(d)) as
+//   scores   grid KV head x 128-position chunk x tile, 4 waves x 32
+//            positions: S = K_j . fp16(q) (model.c:530-538, no 1/sqrt(d)) as
 //            one v_mfma_f32_32x32x16_f16 per 16 head elements (exact
 //            products, fp32 sums); per row and chunk the maximum m_c and
 //            l_c = sum expf(s - m_c) over the row's positions, summed in
 //            double.
-//   values   grid (KV head x tile, 256-position span): per row the global
+//   values   grid KV head x 256-position span x tile: per row the global
 //            maximum M and normaliser (sum_c l_c exp(m_c - M) in double) as in
 //            the decode kernels, the weights fp16(expf(s - M) * inv)
 //            (model.c:547-555) into LDS (0 outside a row's positions), then
 //            sum_j w_j V_j on v_mfma_f32_32x32x16_f16 with the positions as
-//            the contraction: lane (c, half) loads V[j][2c], V[j][2c + 1] of
-//            its 8 positions, the even and the odd columns of a 64-column
-//            group being two 32-column tiles.
+//            the contraction, 32 columns per wave.
 //   combine  per (token, head) its spans' partials added in order.
 // With a device position (decode steps replayed from a graph) the grids are
 // sized for the most positions a call can span and the workgroups past the
@@ -102,13 +100,21 @@ __device__ __forceinline__ void amm_view(AmmArgs &c) {
     c.span = c.p0 + c.nb - c.jb;
 }
 
+// Workgroup l of n_kv x n position blocks x ntt token tiles runs on XCD l % 8:
+// the tiles that share a block's K or V rows go to one XCD, consecutively, and
+// find them in its L2.  The grid is padded to whole groups of 8 blocks.
+__device__ __forceinline__ bool amm_block(const AmmArgs &c, int l, int n, int &kvh, int &blk, int &tt) {
+    const int j = l >> 3, pair = (j / c.ntt) * 8 + (l & 7);
+    tt = j % c.ntt;
+    kvh = pair / n;
+    blk = pair - kvh * n;
+    return pair < c.n_kv * n;
+}
+static unsigned amm_blocks(const AmmArgs &c, int n) { return (unsigned)((c.n_kv * n + 7) / 8 * 8) * c.ntt; }
+
 __device__ __forceinline__ am_v8h amm_ld8(const void *p) { return *(const am_v8h *)p; }
 __device__ __forceinline__ am_v16f amm_mma(am_v8h a, am_v8h b, am_v16f c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ const uint8_t *amm_row(const AmmArgs &c, const uint8_t *cache, int j, int kvh, int hd) {
-    const int slot = c.ring ? j % c.ring : j;
-    return cache + ((size_t)slot * c.n_kv + kvh) * hd * 2;
 }
 // tile row i: token b and head h; the row's positions j0 .. p
 template <int GRP>
@@ -120,22 +126,41 @@ __device__ __forceinline__ void amm_rowinfo(const AmmArgs &c, int kvh, int tt, i
     j0 = c.window ? std::max(0, p + 1 - c.window) : 0;
 }
 
+// Scores, transposed: the positions are the MFMA's rows and the tile's 32
+// (token, head) rows its columns, so a lane holds 16 positions of one row and a
+// row's statistics are sums within a lane and one exchange (with the positions
+// across the lanes they were five exchanges for each of 16 rows, most of them
+// of doubles).  A wave's 32 K rows are loaded in runs of adjacent bytes and
+// turned into operands through LDS of its own, 128 head elements at a time: an
+// operand loaded straight from memory has adjacent lanes in different rows, one
+// L1 access each.  64 tokens after 4096 positions, 8 q / 4 kv heads of 256: 17.2
+// -> 10.6 us.
 template <int HD, int GRP>
 __global__ __launch_bounds__(256) void k_amm_scores(AmmArgs c) {
     constexpr int T = 32 / GRP, QS = HD + 8;
+    constexpr int KW = HD < 128 ? HD : 128, KH = HD / KW, LPR = KW / 8, RPL = 64 / LPR, NL = 32 / RPL;   // K: columns at a time, lanes per row
+    constexpr int KS = KW * 2 + 16;                                 // LDS row stride (bytes)
     __shared__ __align__(16) uint16_t qs[32][QS];                   // fp16 queries of the tile
+    __shared__ __align__(16) uint8_t ks[4][32 * KS];
     __shared__ float wm[4][32];
     __shared__ double wl[4][32];
     amm_view(c);
-    const int kvh = blockIdx.x / c.ntt, tt = blockIdx.x % c.ntt, ch = blockIdx.y;
-    if (ch * AMM_CH >= c.span) return;                               // past the call's last position
+    int kvh, tt, ch;
+    if (!amm_block(c, blockIdx.x, c.nch, kvh, ch, tt) || ch * AMM_CH >= c.span) return;   // past the call's last position
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 31, kh = lane >> 5;
-    const int jl = ch * AMM_CH + wave * 32 + li, j = c.jb + jl;    // the lane's position (MFMA column)
-    const int jfirst = c.window ? max(0, c.p0 + 1 - c.window) : 0;
-    const uint8_t *krow = amm_row(c, c.kc, std::min(std::max(j, jfirst), c.jb + c.span - 1), kvh, HD);
-    am_v8h kb[HD / 16];
+    const int jw = ch * AMM_CH + wave * 32;                          // the wave's first position
+    const int jfirst = c.window ? max(0, c.p0 + 1 - c.window) : 0, jlast = c.jb + c.span - 1;
+    // K rows jfirst .. jlast are one contiguous run of slots (at most `ring` of
+    // them, each row stored twice on a ring)
+    const uint8_t *kbase = c.kc + ((size_t)(c.ring ? jfirst % c.ring : jfirst) * c.n_kv + kvh) * HD * 2 + 16 * (lane % LPR);
+    am_v8h kr[KH][NL];
 #pragma unroll
-    for (int s = 0; s < HD / 16; s++) kb[s] = amm_ld8(krow + (16 * s + 8 * kh) * 2);
+    for (int f = 0; f < KH; f++)
+#pragma unroll
+        for (int n = 0; n < NL; n++) {
+            const int j = std::min(std::max(c.jb + jw + RPL * n + lane / LPR, jfirst), jlast);
+            kr[f][n] = amm_ld8(kbase + (size_t)(j - jfirst) * c.n_kv * HD * 2 + f * KW * 2);
+        }
     // the tile's queries: all of a thread's loads issued before any conversion
     constexpr int NQ = 32 * HD / 4 / 256;                           // float4 per thread
     float4 qv[NQ];
@@ -150,215 +175,204 @@ __global__ __launch_bounds__(256) void k_amm_scores(AmmArgs c) {
         const uint32_t lo = f2h(qv[k].x) | ((uint32_t)f2h(qv[k].y) << 16), hi = f2h(qv[k].z) | ((uint32_t)f2h(qv[k].w) << 16);
         *(uint2 *)&qs[i][4 * e4] = make_uint2(lo, hi);
     }
-    __syncthreads();
+    lds_barrier();
     am_v16f acc = {};
+    uint8_t *kl = ks[wave];
 #pragma unroll
-    for (int s = 0; s < HD / 16; s++) acc = amm_mma(amm_ld8(&qs[li][16 * s + 8 * kh]), kb[s], acc);
-    // C[i][li]: rows i = 8 (r / 4) + 4 kh + r % 4
+    for (int f = 0; f < KH; f++) {
+        // a wave's LDS accesses complete in order; the empty asms keep the
+        // compiler from moving them across the hand-over
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int n = 0; n < NL; n++) *(am_v8h *)(kl + (RPL * n + lane / LPR) * KS + 16 * (lane % LPR)) = kr[f][n];
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int s = 0; s < KW / 16; s++)
+            acc = amm_mma(amm_ld8(kl + li * KS + (16 * s + 8 * kh) * 2), amm_ld8(&qs[li][f * KW + 16 * s + 8 * kh]), acc);
+    }
+    // C[i][li]: positions i = 8 (r / 4) + 4 kh + r % 4 of tile row li
+    int b, h, j0, p;
+    amm_rowinfo<GRP>(c, kvh, tt, li, b, h, j0, p);
+    const bool row = b < c.nb;
+    const size_t R = (size_t)(row ? b : 0) * c.n_head + h;
     bool ok[16];
+    float m = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-        const int i = 8 * (r >> 2) + 4 * kh + (r & 3);
-        int b, h, j0, p;
-        amm_rowinfo<GRP>(c, kvh, tt, i, b, h, j0, p);
-        ok[r] = b < c.nb && jl < c.span && j >= j0 && j <= p;
-        if (ok[r]) c.S[((size_t)b * c.n_head + h) * c.nch * AMM_CH + jl] = acc[r];
-        const float m = group_max<32>(ok[r] ? acc[r] : -INFINITY);
-        if (li == 0) wm[wave][i] = m;
+        const int jl = jw + 8 * (r >> 2) + 4 * kh + (r & 3), j = c.jb + jl;
+        ok[r] = row && jl < c.span && j >= j0 && j <= p;
+        m = fmaxf(m, ok[r] ? acc[r] : -INFINITY);
     }
-    __syncthreads();
+    m = fmaxf(m, partner<32>(m));
+    if (kh == 0) wm[wave][li] = m;
+    if (row) {                                                       // positions outside a row's own are never read
+        float *Sr = c.S + R * c.nch * AMM_CH + jw + 4 * kh;
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int i = 8 * (r >> 2) + 4 * kh + (r & 3);
-        // rows 8 (r / 4) .. 8 (r / 4) + 7 hold tokens from (8 (r / 4)) / GRP
-        // on: none of them in the batch (a decode step's later rows) skips
-        // the exps for the whole wave
-        if (tt * T + 8 * (r >> 2) / GRP >= c.nb) continue;           // uniform
-        const float mc = fmaxf(fmaxf(wm[0][i], wm[1][i]), fmaxf(wm[2][i], wm[3][i]));
-        const double l = group_sum_t<32>(ok[r] ? (double)expf(acc[r] - mc) : 0.0);
-        if (li == 0) wl[wave][i] = l;
+        for (int q = 0; q < 4; q++) *(float4 *)(Sr + 8 * q) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
     }
-    __syncthreads();
-    if (t < 32) {
-        int b, h, j0, p;
-        amm_rowinfo<GRP>(c, kvh, tt, t, b, h, j0, p);
-        if (b < c.nb) {
-            const size_t R = (size_t)b * c.n_head + h;
-            c.Mc[R * c.nch + ch] = fmaxf(fmaxf(wm[0][t], wm[1][t]), fmaxf(wm[2][t], wm[3][t]));
-            c.Lc[R * c.nch + ch] = ((wl[0][t] + wl[1][t]) + wl[2][t]) + wl[3][t];
-        }
+    lds_barrier();
+    const float mc = fmaxf(fmaxf(wm[0][li], wm[1][li]), fmaxf(wm[2][li], wm[3][li]));
+    double l = 0.0;
+#pragma unroll
+    for (int r = 0; r < 16; r++) l += ok[r] ? (double)expf(acc[r] - mc) : 0.0;
+    l += partner<32>(l);
+    if (kh == 0) wl[wave][li] = l;
+    lds_barrier();
+    if (t < 32 && row) {
+        c.Mc[R * c.nch + ch] = mc;
+        c.Lc[R * c.nch + ch] = ((wl[0][t] + wl[1][t]) + wl[2][t]) + wl[3][t];
     }
 }
 
-// PF: steps of V loads in flight per wave in the value sums: 8, or for calls
-// of one row tile (decode steps and short verify batches, whose few
-// workgroups are bound by that chain's round trips) 16 at heads up to 256
-// wide, the whole span loaded at the start; the MFMAs and their order are
-// the same either way.  Measured on the 64-token prompt chunk of 26 layers
-// (8 q / 4 KV heads of 256 at position 4096): 3.58 ms with 4 steps, 3.50 with
-// 8, 3.76 with 16.
-template <int HD, int GRP, int PF>
-__global__ __launch_bounds__(256) void k_amm_v(AmmArgs c) {
-    constexpr int WS = AMM_NP + 8;
-    __shared__ __align__(16) uint16_t wsh[32][WS];                  // fp16 weights of the span
-    __shared__ float mx[32], iv[32];
+// Values: 8 waves, each with 4 of the tile's rows for the weights and one of up
+// to 8 units of 32 columns for the sums (heads of 512 take two workgroups, grid
+// y).  Every load goes out at the start -- chunk statistics, scores 16 bytes
+// per lane, V rows in runs of adjacent bytes, 28 loads in all (a wave tracks 63;
+// V loaded as 128 words per lane took 4.3 us to issue), the second half of V
+// once the statistics are done -- so the phases wait on one round trip.  A
+// row's statistics and weights are one wave's, handed over in registers; V
+// passes through LDS of the wave's own 64 positions at a time and is read there
+// transposed (ds_read_b64_tr_b16).  48 KB of LDS and 128 registers: two
+// workgroups per CU.  64 tokens after 4096 positions, 8 q /
+// 4 kv heads of 256: 20.8 -> 15.6 us.
+typedef short am_v4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) am_v4s *am_lds4;
+
+template <int HD, int GRP>
+__global__ __launch_bounds__(512, 4) void k_amm_v(AmmArgs c) {
+    constexpr int NU = HD < 256 ? HD / 32 : 8, ST = AMM_NP / 16, VP = 4, HP = AMM_NP / VP;   // column units, steps, V parts and their positions
+    // fp16 weights of the span, the 16-byte units of row r at unit ^ (r & 7)
+    __shared__ __align__(16) uint8_t wsh[32 * AMM_NP * 2];
+    __shared__ __align__(16) uint8_t vsh[8][HP * 64];               // a wave's part of V: rows of 32 columns
     amm_view(c);
-    const int kvh = blockIdx.x / c.ntt, tt = blockIdx.x % c.ntt, cv = blockIdx.y;
-    if (cv * AMM_NP >= c.span) return;                               // past the call's last position
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 31, kh = lane >> 5;
-    const int jl0 = cv * AMM_NP;
+    int kvh, tt, cv;
+    if (!amm_block(c, blockIdx.x, c.nchv, kvh, cv, tt) || cv * AMM_NP >= c.span) return;   // past the call's last position
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t) >> 6, li = lane & 31, kh = lane >> 5;
+    const int jl0 = cv * AMM_NP, unit = wave + 8 * blockIdx.y;
     const int jfirst = c.window ? max(0, c.p0 + 1 - c.window) : 0, jlast = c.jb + c.span - 1;
-    // the attended positions jfirst .. jlast are at most `ring` apart, so on
-    // a ring (rows stored at j % ring and again at j % ring + ring) they are
-    // one contiguous run of slots from jfirst % ring: one modulo per thread
-    // instead of one per row loaded
-    const uint8_t *vbase = c.vc + ((size_t)(c.ring ? jfirst % c.ring : jfirst) * c.n_kv + kvh) * HD * 2;
-    // lane (c, half)'s V words of step st in column group g (columns 2c,
-    // 2c + 1 of its 8 positions): rows clamped to the positions the batch
-    // attends, so every row loaded holds a stored value
-    auto vword = [&](int g, int st, int k) __attribute__((always_inline)) {
-        const int jb8 = c.jb + jl0 + 16 * st + 8 * kh;
-        return *(const uint32_t *)(vbase + (size_t)(std::min(std::max(jb8 + k, jfirst), jlast) - jfirst) * c.n_kv * HD * 2 +
-                                   (64 * g + 2 * li) * 2);
-    };
-    // one row tile with one column group per wave: every load of the kernel
-    // (this wave's V words, this thread's scores) goes out first, so the
-    // three phases below wait on one round trip instead of three
-    constexpr bool EARLY = PF == 16 && HD <= 256;
-    uint32_t xe[EARLY ? 16 : 1][8];
-    float se[EARLY ? 32 : 1];
-    if constexpr (EARLY) {
-        if (wave < HD / 64) {                                        // uniform
-#pragma unroll
-            for (int q = 0; q < 16; q++)
-#pragma unroll
-                for (int k = 0; k < 8; k++) xe[q][k] = vword(wave, q, k);
-        }
-        const int jl = jl0 + t, j = c.jb + jl;
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
-            int b, h, j0, p;
-            amm_rowinfo<GRP>(c, kvh, tt, i, b, h, j0, p);
-            const bool ok = b < c.nb && jl < c.span && j >= j0 && j <= p;
-            se[i] = ok ? c.S[((size_t)b * c.n_head + h) * c.nch * AMM_CH + jl] : 0.0f;
-        }
-    }
     // 1. per row the global maximum and normaliser over the row's own chunks
-    // (wave w: rows 8 w .. 8 w + 7; lane k: the row's k-th chunk, 64 per
-    // round), the eight rows' loads of a round issued together
+    // (wave w: rows 4 w .. 4 w + 3; lane k: the row's k-th chunk, 64 per round)
+    const int nca = (c.span + AMM_CH - 1) / AMM_CH;                  // >= any row's chunk count
+    int nrc[4], j0r[4], pr[4];
+    size_t base[4];
+    bool rv[4], on[4];
+    float mcv[4];
+    double lcv[4];
+    float4 sv[4];                                                    // the scores of positions 4 lane .. + 3
+    const int jt = jl0 + 4 * lane, jg = c.jb + jt;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        int b, h;
+        amm_rowinfo<GRP>(c, kvh, tt, wave * 4 + k, b, h, j0r[k], pr[k]);
+        rv[k] = b < c.nb;
+        const int clo = rv[k] ? (j0r[k] - c.jb) / AMM_CH : 0;
+        nrc[k] = rv[k] ? (pr[k] - c.jb) / AMM_CH - clo + 1 : 0;
+        base[k] = ((size_t)(rv[k] ? b : 0) * c.n_head + h) * c.nch + clo;
+        on[k] = lane < nrc[k];
+        mcv[k] = on[k] ? c.Mc[base[k] + lane] : -INFINITY;
+        lcv[k] = on[k] ? c.Lc[base[k] + lane] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        // whole chunks of scores are stored for the tile's rows; a span's second
+        // chunk may lie past the last one
+        const bool in = rv[k] && jt < c.nch * AMM_CH;
+        sv[k] = in ? *(const float4 *)(c.S + (base[k] - (rv[k] ? (j0r[k] - c.jb) / AMM_CH : 0)) * AMM_CH + jt) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    // the unit's columns of the span's V rows, 4 lanes to a row, 16 rows per
+    // load.  The attended positions jfirst .. jlast are at most `ring` apart,
+    // so on a ring (rows stored at j % ring and again at j % ring + ring) they
+    // are one contiguous run of slots from jfirst % ring.  Rows are clamped to
+    // them, so every row loaded holds a stored value.
+    am_v8h v[ST];
+    const size_t rstr = (size_t)c.n_kv * HD * 2;
+    const uint8_t *vbase = c.vc + ((size_t)(c.ring ? jfirst % c.ring : jfirst) * c.n_kv + kvh) * HD * 2 + 64 * unit + 16 * (lane & 3);
+    auto load_v = [&](int q) __attribute__((always_inline)) {
+        const int j = std::min(std::max(c.jb + jl0 + 16 * q + (lane >> 2), jfirst), jlast);
+        v[q] = amm_ld8(vbase + (size_t)(j - jfirst) * rstr);
+    };
+    if (wave < NU) {                                                 // uniform
+#pragma unroll
+        for (int q = 0; q < ST / 2; q++) load_v(q);
+    }
+    asm volatile("" ::: "memory");
+    float m[4], inv[4];
     {
-        const int nca = (c.span + AMM_CH - 1) / AMM_CH;              // >= any row's chunk count
-        int clo[8], nrc[8];
-        size_t base[8];
-        bool rv[8];
+        double sum[4];
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            int b, h, j0, p;
-            amm_rowinfo<GRP>(c, kvh, tt, wave * 8 + k, b, h, j0, p);
-            rv[k] = b < c.nb;
-            clo[k] = rv[k] ? (j0 - c.jb) / AMM_CH : 0;
-            nrc[k] = rv[k] ? (p - c.jb) / AMM_CH - clo[k] + 1 : 0;
-            base[k] = ((size_t)(rv[k] ? b : 0) * c.n_head + h) * c.nch + clo[k];
-        }
-        float mcv[8], m[8];
-        double lcv[8], sum[8];
-        bool on[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            on[k] = lane < nrc[k];
-            mcv[k] = on[k] ? c.Mc[base[k] + lane] : -INFINITY;
-            lcv[k] = on[k] ? c.Lc[base[k] + lane] : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < 8; k++) m[k] = group_max<64>(mcv[k]);
+        for (int k = 0; k < 4; k++) m[k] = group_max<64>(mcv[k]);
         for (int c1 = 64; c1 < nca; c1 += 64)
 #pragma unroll
-            for (int k = 0; k < 8; k++) m[k] = fmaxf(m[k], group_max<64>(c1 + lane < nrc[k] ? c.Mc[base[k] + c1 + lane] : -INFINITY));
+            for (int k = 0; k < 4; k++) m[k] = fmaxf(m[k], group_max<64>(c1 + lane < nrc[k] ? c.Mc[base[k] + c1 + lane] : -INFINITY));
 #pragma unroll
-        for (int k = 0; k < 8; k++)                                  // rows outside the batch (uniform) skip the exp
+        for (int k = 0; k < 4; k++)                                  // rows outside the batch (uniform) skip the exp
             sum[k] = rv[k] ? group_sum_t<64>(on[k] ? lcv[k] * exp((double)mcv[k] - (double)m[k]) : 0.0) : 1.0;
         for (int c1 = 64; c1 < nca; c1 += 64)
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
+            for (int k = 0; k < 4; k++) {
                 const bool o = c1 + lane < nrc[k];
                 const float mc = o ? c.Mc[base[k] + c1 + lane] : 0.0f;
                 const double lc = o ? c.Lc[base[k] + c1 + lane] : 0.0;
                 sum[k] += group_sum_t<64>(o ? lc * exp((double)mc - (double)m[k]) : 0.0);
             }
-        if (lane == 0)
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                mx[wave * 8 + k] = m[k];
-                iv[wave * 8 + k] = (float)(1.0 / sum[k]);
-            }
+        for (int k = 0; k < 4; k++) inv[k] = (float)(1.0 / sum[k]);
     }
-    __syncthreads();
-    // 2. the weights (0 outside a row's positions): thread t owns position t
-    // of the span in every row, its score loads issued 16 rows at a time
-    static_assert(AMM_NP == 256, "one position per thread");
+    asm volatile("" ::: "memory");
+    if (wave < NU) {                                                 // the second half, the statistics' registers free
 #pragma unroll
-    for (int i0 = 0; i0 < 32; i0 += 16) {
-        const int jl = jl0 + t, j = c.jb + jl;
-        float sv[16];
-        bool ok[16];
+        for (int q = ST / 2; q < ST; q++) load_v(q);
+    }
+    asm volatile("" ::: "memory");
+    // 2. the weights (0 outside a row's positions)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            int b, h, j0, p;
-            amm_rowinfo<GRP>(c, kvh, tt, i0 + i, b, h, j0, p);
-            ok[i] = b < c.nb && jl < c.span && j >= j0 && j <= p;
-            if constexpr (EARLY) sv[i] = se[i0 + i];
-            else sv[i] = ok[i] ? c.S[((size_t)b * c.n_head + h) * c.nch * AMM_CH + jl] : 0.0f;
+    for (int k = 0; k < 4; k++) {
+        uint2 w = make_uint2(0, 0);
+        if (rv[k]) {                                                 // uniform
+            const float e[4] = {sv[k].x, sv[k].y, sv[k].z, sv[k].w};
+            uint32_t hw[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const bool ok = jt + i < c.span && jg + i >= j0r[k] && jg + i <= pr[k];
+                hw[i] = f2h(ok ? expf(e[i] - m[k]) * inv[k] : 0.0f);
+            }
+            w = make_uint2(hw[0] | (hw[1] << 16), hw[2] | (hw[3] << 16));
         }
+        const int r = wave * 4 + k;
+        *(uint2 *)(wsh + r * (AMM_NP * 2) + 16 * ((lane >> 1) ^ (r & 7)) + 8 * (lane & 1)) = w;
+    }
+    lds_barrier();
+    if (wave >= NU) return;                                          // uniform
+    // 3. sum_j w_j V_j over the span's 16 steps of 16 positions, in step order
+    // (the MFMA's accumulation).  The operand of step q: lane (c, half) holds
+    // column c of positions 8 half .. + 7, two transposed reads in which 16
+    // lanes give 4 rows of 16 columns and get 4 rows of their own column
+    uint8_t *vl = vsh[wave];
+    const int g4 = lane >> 4, i16 = lane & 15;
+    const uint32_t tr = (8 * (g4 >> 1) + (i16 >> 2)) * 64 + 32 * (g4 & 1) + 8 * (i16 & 3);
+    am_v16f acc = {};
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            int b, h, j0, p;
-            amm_rowinfo<GRP>(c, kvh, tt, i0 + i, b, h, j0, p);
-            // a row outside the batch (uniform: a decode step's rows past
-            // its GRP heads) takes weight 0 without the exp
-            wsh[i0 + i][t] = b < c.nb ? f2h(ok[i] ? expf(sv[i] - mx[i0 + i]) * iv[i0 + i] : 0.0f) : (uint16_t)0;
+    for (int f = 0; f < VP; f++) {
+        asm volatile("" ::: "memory");                               // a wave's LDS accesses complete in order
+#pragma unroll
+        for (int q = 0; q < ST / VP; q++) *(am_v8h *)(vl + (16 * q + (lane >> 2)) * 64 + 16 * (lane & 3)) = v[f * (ST / VP) + q];
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int q = 0; q < ST / VP; q++) {
+            const am_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((am_lds4)(vl + tr + 16 * q * 64));
+            const am_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((am_lds4)(vl + tr + (16 * q + 4) * 64));
+            typedef short v8s __attribute__((ext_vector_type(8)));
+            const v8s bv = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            const int un = 2 * (f * (ST / VP) + q) + kh;
+            acc = amm_mma(amm_ld8(wsh + li * (AMM_NP * 2) + 16 * (un ^ (li & 7))), __builtin_bit_cast(am_v8h, bv), acc);
         }
     }
-    __syncthreads();
-    // 3. sum_j w_j V_j over the span's 16 steps of 16 positions, in step
-    // order (the MFMA's accumulation): wave w takes the 64-column groups w,
-    // w + 4, ..; lane (c, half) loads columns 2c, 2c + 1 of its 8 positions
-    // per step (the even and the odd columns two 32-column tiles)
-#pragma unroll 1
-    for (int g = wave; g < HD / 64; g += 4) {
-        const int col = 64 * g + 2 * li;
-        am_v16f ae = {}, ao = {};
-        for (int st0 = 0; st0 < AMM_NP / 16; st0 += PF) {
-            uint32_t x[PF][8];
 #pragma unroll
-            for (int q = 0; q < PF; q++)
-#pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    if constexpr (EARLY) x[q][k] = xe[q][k];                  // loaded at the start (g == wave)
-                    else x[q][k] = vword(g, st0 + q, k);
-                }
-#pragma unroll
-            for (int q = 0; q < PF; q++) {
-                am_v8h be, bo;
-#pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    be[k] = __builtin_bit_cast(_Float16, (uint16_t)(x[q][k] & 0xffff));
-                    bo[k] = __builtin_bit_cast(_Float16, (uint16_t)(x[q][k] >> 16));
-                }
-                const am_v8h a = amm_ld8(&wsh[li][16 * (st0 + q) + 8 * kh]);
-                ae = amm_mma(a, be, ae);
-                ao = amm_mma(a, bo, ao);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int i = 8 * (r >> 2) + 4 * kh + (r & 3);
-            int b, h, j0, p;
-            amm_rowinfo<GRP>(c, kvh, tt, i, b, h, j0, p);
-            if (b < c.nb) {
-                float *dst = c.P + (((size_t)b * c.n_head + h) * c.nchv + cv) * HD;
-                *(float2 *)(dst + col) = make_float2(ae[r], ao[r]);
-            }
-        }
+    for (int r = 0; r < 16; r++) {
+        const int i = 8 * (r >> 2) + 4 * kh + (r & 3);
+        int b, h, j0, p;
+        amm_rowinfo<GRP>(c, kvh, tt, i, b, h, j0, p);
+        if (b < c.nb) c.P[(((size_t)b * c.n_head + h) * c.nchv + cv) * HD + 32 * unit + li] = acc[r];
     }
 }
 
@@ -413,10 +427,8 @@ bool attn_batch_mm_ok(const QkvArgs &a) {
 
 template <int HD, int GRP>
 static void amm_go(const AmmArgs &c, hipStream_t s) {
-    hipLaunchKernelGGL((k_amm_scores<HD, GRP>), dim3(c.n_kv * c.ntt, c.nch), dim3(256), 0, s, c);
-    constexpr int PF1 = HD == 512 ? 8 : 16;                          // 16 steps of 512-wide rows spill
-    if (c.ntt == 1) hipLaunchKernelGGL((k_amm_v<HD, GRP, PF1>), dim3(c.n_kv * c.ntt, c.nchv), dim3(256), 0, s, c);
-    else hipLaunchKernelGGL((k_amm_v<HD, GRP, 8>), dim3(c.n_kv * c.ntt, c.nchv), dim3(256), 0, s, c);
+    hipLaunchKernelGGL((k_amm_scores<HD, GRP>), dim3(amm_blocks(c, c.nch)), dim3(256), 0, s, c);
+    hipLaunchKernelGGL((k_amm_v<HD, GRP>), dim3(amm_blocks(c, c.nchv), HD == 512 ? 2 : 1), dim3(512), 0, s, c);
     hipLaunchKernelGGL(k_amm_combine<HD>, dim3(c.n_head, c.nb), dim3(256), 0, s, c);
 }
 
