@@ -488,6 +488,10 @@ extern "C" int g4h_matmul_describe(const g4h_tensor *W, int nb, int path, char *
     const int chunk = gemv_chunk_at(*W, nb, 0);
     int launches = 0;
     for (int done = 0; done < nb; launches++) done += gemv_chunk_at(*W, nb, done);
+    if (mmg_fits(*W, nb)) {
+        mmg_describe(*W, nb, buf, len);
+        return G4H_OK;
+    }
     const bool xq = x_fused(*W, nb);
     gemv_launch_shape(*W, &lpr, &upl, &wpg, &grid, chunk, xq);
     upl = gemv_upl_final(W->type, W->nb, chunk, lpr, upl);
@@ -666,6 +670,12 @@ static int matmul_impl(const g4h_tensor *W, const float *x, const void *pre, siz
         stride = g4h_act_stride(W->type, W->ncols);
         void *buf;
         if (int rc = scr.get(s, stride * nb, &buf)) return rc;
+        if (mmg_fits(*W, nb)) {
+            // same bits as the chunks below (given rows take those)
+            const hipError_t e = launch_matmul_mfma_gx(*W, x, W->ncols, nb, Y, (uint8_t *)buf, s);
+            if (e != hipSuccess) return hip_fail(e, "g4h_matmul: matrix-core launch");
+            return G4H_OK;
+        }
         const hipError_t e = g4h_act_type(W->type) == Q8_0
                                  ? launch_quantize_q8_0(x, W->ncols, (uint8_t *)buf, stride, W->ncols, nb, s)
                                  : launch_quantize_q8_K(x, W->ncols, (uint8_t *)buf, stride, W->ncols, nb, s);

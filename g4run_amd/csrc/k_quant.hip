@@ -75,13 +75,14 @@ __global__ __launch_bounds__(256) void k_quantize_q8_K(const float *__restrict__
 // one TL = rows % 32 wide), per superblock sixteen 16-byte chunks [2 g + kh][TL]
 // -- the lane half kh's quants of the 32-element group g -- then with BS the 16
 // bsums as fp16 [kh][TL][8] (exact: |bsum| <= 2048; without them the place stays
-// unused) and d [TL].  HALVES: kh holds elements 8 kh .. + 7 and 16 + 8 kh .. +
-// 7 of a group (q6_K's sub-blocks of 16), else 16 kh .. + 15.  Consecutive
-// waves take consecutive tokens of one superblock, so their 4-byte stores
-// share lines.
+// unused) and d [TL].  LAY 0: kh holds elements 16 kh .. + 15 of group g; 1: 8 kh
+// .. + 7 and 16 + 8 kh .. + 7 (q6_K's sub-blocks of 16); 2 (k_mmg's units of
+// 16-byte quant runs): g = 2 (2 h + k) + f, and kh holds elements 128 h + 32 j +
+// 16 k + 8 kh .. + 7 of j = 2 f and 2 f + 1.  Consecutive waves take consecutive
+// tokens of one superblock, so their 4-byte stores share lines.
 // QT superblocks per wave (QT consecutive tokens of one superblock index), all
 // of their loads issued first.
-template <bool HALVES, bool BS, int QT>
+template <int LAY, bool BS, int QT>
 __global__ __launch_bounds__(256) void k_quantize_q8_K_tile(const float *__restrict__ x, size_t xs, uint8_t *__restrict__ y, int nb,
                                                             int rows) {
     const int nt = (rows + QT - 1) / QT;
@@ -95,8 +96,9 @@ __global__ __launch_bounds__(256) void k_quantize_q8_K_tile(const float *__restr
         const float *src = x + (size_t)min(r0 + q, rows - 1) * xs + (size_t)sb * 256 + 4 * l;
         for (int i = 0; i < 4; i++) v[q][i] = src[i];
     }
-    const int g = l >> 3, e = 4 * (l & 7), k = l >> 2;
-    const int kh = HALVES ? (e >> 3) & 1 : e >> 4, at = HALVES ? (e & 7) + 8 * (e >> 4) : e & 15;
+    const int e = 4 * (l & 7), k = l >> 2;
+    const int g = LAY == 2 ? 2 * (2 * (l >> 5) + (e >> 4)) + ((l >> 4) & 1) : l >> 3;
+    const int kh = LAY ? (e >> 3) & 1 : e >> 4, at = LAY == 2 ? (e & 7) + (l & 8) : LAY ? (e & 7) + 8 * (e >> 4) : e & 15;
 #pragma unroll
     for (int q = 0; q < QT; q++) {
         const int r = r0 + q;
@@ -356,8 +358,10 @@ hipError_t launch_quantize_q8_K(const float *x, size_t xs, uint8_t *y, size_t ys
 template <int QT>
 static void q8kt_go(const float *x, size_t xs, uint8_t *y, int nb, int rows, int wtype, hipStream_t s) {
     const dim3 grid((unsigned)(((int64_t)(rows + QT - 1) / QT * nb + 3) / 4));
-    if (wtype == Q6_K) hipLaunchKernelGGL((k_quantize_q8_K_tile<true, false, QT>), grid, dim3(256), 0, s, x, xs, y, nb, rows);
-    else hipLaunchKernelGGL((k_quantize_q8_K_tile<false, true, QT>), grid, dim3(256), 0, s, x, xs, y, nb, rows);
+    if (wtype == Q6_K) hipLaunchKernelGGL((k_quantize_q8_K_tile<1, false, QT>), grid, dim3(256), 0, s, x, xs, y, nb, rows);
+    else if (wtype == Q3_K || wtype == TQ2_0) hipLaunchKernelGGL((k_quantize_q8_K_tile<2, false, QT>), grid, dim3(256), 0, s, x, xs, y, nb, rows);
+    else if (wtype == Q2_K) hipLaunchKernelGGL((k_quantize_q8_K_tile<2, true, QT>), grid, dim3(256), 0, s, x, xs, y, nb, rows);
+    else hipLaunchKernelGGL((k_quantize_q8_K_tile<0, true, QT>), grid, dim3(256), 0, s, x, xs, y, nb, rows);
 }
 // four superblocks per wave once that still fills the chip's 8192 waves
 hipError_t launch_quantize_q8_K_tile(const float *x, size_t xs, uint8_t *y, int64_t n, int rows, int wtype, hipStream_t s) {

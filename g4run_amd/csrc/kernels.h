@@ -251,6 +251,11 @@ void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len);
 // superblock, 64-byte aligned): the bits of quantizing to q8_K rows first
 hipError_t launch_matmul_mfma_kx(const g4h_tensor &W, const float *x, size_t xs, int M, float *Y, uint8_t *ws, hipStream_t s);
 hipError_t launch_quantize_q8_K_tile(const float *x, size_t xs, uint8_t *y, int64_t n, int rows, int wtype, hipStream_t s);
+// k_mfma_g.hip: batches of 9 tokens and more over q5_K / q3_K / q2_K / tq2_0
+// weights on the matrix cores, with the GEMV family's bits (ws as above)
+bool mmg_fits(const g4h_tensor &W, int M);
+void mmg_describe(const g4h_tensor &W, int M, char *buf, size_t len);
+hipError_t launch_matmul_mfma_gx(const g4h_tensor &W, const float *x, size_t xs, int M, float *Y, uint8_t *ws, hipStream_t s);
 hipError_t launch_matmul_mfma_k(const g4h_tensor &W, const uint8_t *act, size_t stride, int M, float *Y, hipStream_t s);
 
 // k_attn.hip

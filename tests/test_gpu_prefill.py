@@ -249,3 +249,27 @@ def test_kquant_tile_kernel_equals_given_rows(gpu, oracle, name, qt, rows, cols)
         assert np.array_equal(bits(b), bits(full[:m])), f"{name} M={m}: given rows"
     if rows == 4100:
         assert "mt=2" in gpu.matmul_describe(t, 129, 2) and "mt=1" in gpu.matmul_describe(t, 33, 2)
+
+
+@pytest.mark.parametrize("name,qt", [("q5_K", 13), ("q3_K", 11), ("q2_K", 10), ("tq2_0", 35)])
+@pytest.mark.parametrize("rows,cols", [(100, 256), (257, 2048), (33, 2304), (260, 4096), (64, 4352), (520, 11008)])
+def test_gemv_order_tiles_equal_gemv(gpu, oracle, name, qt, rows, cols):
+    """fp32 tokens from 9 on (k_mmg, matrix cores) give the GEMV kernels' bits
+    (the same tokens as q8_K rows): 16, 32 and 64 lanes per row, superblock
+    classes that have none, one or several superblocks, ragged rows and tokens
+    off the 32-token tile; and a token the same bits alone."""
+    w, x, t = _setup(gpu, qt, rows, cols, 70, seed=rows + qt)
+    x[1] *= 8192.0
+    x[2, :] = 0.0
+    x[3, ::2] = -x[3, ::2] * 1e-6
+    act = oracle.prep_act(qt, x)
+    assert gpu.matmul_describe(t, 9, 0).startswith("k_mmg") and gpu.matmul_describe(t, 8, 0).startswith("k_gemv")
+    full = gpu_matmul(gpu, t, act=act, nb=70, path=1)
+    # a token scaled by 2^13 has every product and sum scaled by 2^13 (no rounding
+    # changes), so the absolute part of the bound scales with it
+    s = np.ones((70, 1), np.float32)
+    s[1] = 1.0 / 8192.0
+    assert_close(full * s, oracle_matmul(oracle, qt, w, x) * s, f"{name} {rows}x{cols}")
+    for m in (1, 9, 31, 32, 33, 64, 70):
+        a = gpu_matmul(gpu, t, x=x[:m].copy(), nb=m, path=0)
+        assert np.array_equal(bits(a), bits(full[:m])), f"{name} {rows}x{cols} M={m}"
