@@ -299,7 +299,12 @@ __global__ __launch_bounds__(NC < 8 ? 256 : 512) void k_mmg(g4h_tensor W, const 
     }
 }
 
-// the GEMV shapes it reproduces: 16, 32 or 64 lanes per row
+// the GEMV shapes it reproduces: 16, 32 or 64 lanes per row.  From 9 tokens,
+// where the GEMV takes a second launch (up to 8 it takes one, two at wide
+// rows): faster at every size there, the smallest included (GEMV chunks / this,
+// us, 9 tokens: q5_K 256 x 256 11.9 / 7.5, 256 x 2048 14.6 / 8.3, 256 x 11008
+// 49.2 / 19.2, 1024 x 4096 15.4 / 9.9; tq2_0 256 x 256 12.3 / 8.4, 1024 x 4096
+// 15.2 / 8.3)
 static int mmg_classes(const g4h_tensor &W) {
     int lpr, upl;
     gemv_shape(W.type, W.nb, &lpr, &upl);
