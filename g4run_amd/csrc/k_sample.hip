@@ -308,61 +308,67 @@ __device__ void rewrite(SamplerDev *S, float *L, Lds &sh) {
 // First launch of a large row: the rewrites of sampler.c:78-137 for this
 // workgroup's 1024 ids, then the largest key of each of its groups of GS ids (all
 // ones if one of them is NaN).  Every workgroup walks the ban list, the ring
-// and the penalty window, and keeps the ids of its own slice; the window entry
-// that comes first of its id's entries counts them.
+// and the penalty window, 2048 entries per round of loads, and marks the ids of
+// its own slice in LDS: a bit for a ban or an n-gram hit, a count of the window's
+// entries.  A thread then rewrites its four ids in registers.  The counts are
+// linear in the window (counting each entry by a walk over the window was
+// quadratic: with 4096 entries over 32768 ids a draw and a copy of its row took
+// 2234 us, 108 with the one-launch form's sort, 30 with this).
 template <int GS>
 __global__ __launch_bounds__(256) void k_sample_groups(SamplerDev *S, float *L, uint32_t *groups) {
-    __shared__ int win[SAMPLER_RING], suf[64], mod;
+    __shared__ __align__(16) int cnt[1024];
+    __shared__ uint32_t out[32];
+    __shared__ int suf[64];
     const int t = threadIdx.x, nv = S->n_vocab, rn = S->recent_n;
     const float rp = S->repeat_penalty, fp = S->freq_penalty, pp = S->presence_penalty;
-    const int rln = S->repeat_last_n, ngram = S->no_repeat_ngram, nban = S->n_ban;
+    const int rln = S->repeat_last_n, ngram = S->no_repeat_ngram;
     const int lo = blockIdx.x * 1024, hi = min(lo + 1024, nv), i0 = lo + 4 * t;
     float v[4];
-    auto load = [&] {
-        if (i0 + 3 < nv) f4(*(const float4 *)(L + i0), v);
-        else
-            for (int q = 0; q < 4; q++) v[q] = i0 + q < nv ? L[i0 + q] : -INFINITY;
-    };
-    load();
-    auto mine = [&](int id) { return id >= lo && id < hi; };
-    if (t == 0) mod = 0;
+    if (i0 + 3 < nv) f4(*(const float4 *)(L + i0), v);
+    else
+        for (int q = 0; q < 4; q++) v[q] = i0 + q < nv ? L[i0 + q] : -INFINITY;
+    const int m = ngram >= 2 && rn >= ngram ? (ngram - 1 < 64 ? ngram - 1 : 64) : 0;   // uniform
+    *(int4 *)&cnt[4 * t] = make_int4(0, 0, 0, 0);
+    if (t < 32) out[t] = 0;
+    if (t < m) suf[t] = ring_at(S, rn - m + t);
     __syncthreads();
+    // f(i, id) for every i < n whose id lies in the slice
+    auto walk = [&](int n, auto &&id_at, auto &&f) {
+        for (int j0 = t; j0 < n; j0 += 8 * 256) {
+            int id[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) id[q] = j0 + 256 * q < n ? id_at(j0 + 256 * q) : -1;
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                if (id[q] >= lo && id[q] < hi) f(j0 + 256 * q, id[q] - lo);
+        }
+    };
     const int *ban = sampler_bans(S);
-    for (int j = t; j < nban; j += 256)
-        if (mine(ban[j])) { L[ban[j]] = -INFINITY; mod = 1; }
-    if (ngram >= 2 && rn >= ngram) {
-        const int m = ngram - 1 < 64 ? ngram - 1 : 64;
-        if (t < m) suf[t] = ring_at(S, rn - m + t);
-        __syncthreads();
-        for (int p = t; p + m < rn; p += 256) {
-            const int id = ring_at(S, p + m);
-            if (!mine(id)) continue;
+    walk(S->n_ban, [&](int j) { return ban[j]; }, [&](int, int e) { atomicOr(&out[e >> 5], 1u << (e & 31)); });
+    if (m)
+        walk(rn - m, [&](int p) { return ring_at(S, p + m); }, [&](int p, int e) {
             bool hit = true;
             for (int j = 0; j < m && hit; j++) hit = ring_at(S, p + j) == suf[j];
-            if (hit) { L[id] = -INFINITY; mod = 1; }
-        }
-    }
-    if ((rp != 1.0f || fp != 0 || pp != 0) && rln > 0 && rn > 0) {
-        const int nw = rln < rn ? rln : rn;
-        for (int i = t; i < nw; i += 256) win[i] = ring_at(S, rn - 1 - i);
-        __syncthreads();                                             // the -inf stores above included
-        for (int i = t; i < nw; i += 256) {
-            const int id = win[i];
-            if (!mine(id)) continue;
-            int count = 0, first = nw;
-            for (int j = nw - 1; j >= 0; j--)
-                if (win[j] == id) { count++; first = j; }
-            if (first != i) continue;
-            float l = L[id];
-            if (rp != 1.0f) l = l <= 0 ? l * rp : l / rp;
-            const float fterm = (float)count * fp;
-            l -= fterm + (count > 0 ? pp : 0.0f);
-            L[id] = l;
-            mod = 1;
-        }
-    }
+            if (hit) atomicOr(&out[e >> 5], 1u << (e & 31));
+        });
+    if ((rp != 1.0f || fp != 0 || pp != 0) && rln > 0)
+        walk(min(rln, rn), [&](int i) { return ring_at(S, rn - 1 - i); }, [&](int, int e) { atomicAdd(&cnt[e], 1); });
     __syncthreads();
-    if (mod) load();
+    const uint32_t bits = out[t >> 3] >> (4 * (t & 7));
+    const int4 c4 = *(const int4 *)&cnt[4 * t];
+    const int c[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        if (bits >> q & 1) v[q] = -INFINITY;
+        if (c[q] > 0) {
+            float l = v[q];
+            if (rp != 1.0f) l = l <= 0 ? l * rp : l / rp;
+            const float fterm = (float)c[q] * fp;
+            l -= fterm + pp;
+            v[q] = l;
+        }
+        if ((bits >> q & 1) || c[q] > 0) L[i0 + q] = v[q];
+    }
     uint32_t k = 0;
     bool nan = false;
 #pragma unroll

@@ -214,3 +214,51 @@ def test_row_sizes_and_kinds(gpu, oracle, nv, kind):
     hist = np.concatenate([rs.integers(0, nv, 60), rs.integers(0, 30, 60)])
     for p in (dict(BASE, repeat_last_n=100, no_repeat_ngram=2), dict(BASE, top_k=0, no_repeat_ngram=0), dict(BASE, temp=0.0)):
         run_pair(gpu, oracle, nv, p, rs, kind, 2, bans=[0, 2, nv - 1], hist=hist)
+
+
+# the two-launch form's walks take 2048 entries per round: windows, n-gram
+# histories and ban lists beyond one round, the ring wrapped
+@pytest.mark.parametrize("nv", [16384, 32768, 262144])
+@pytest.mark.parametrize("ids", [20, 1024, None])
+def test_long_windows_of_large_rows(gpu, oracle, nv, ids):
+    rs = np.random.default_rng(nv + (ids or 0))
+    hist = rs.integers(0, ids or nv, 4500)
+    p = dict(BASE, repeat_last_n=5000, repeat_penalty=1.3, freq_penalty=0.2, no_repeat_ngram=4 if ids == 20 else 2)
+    run_pair(gpu, oracle, nv, p, rs, "plain", 3, bans=rs.permutation(nv)[:2100] if ids is None else [], hist=hist)
+
+
+def draw_us(G, nv, row, hist, **params):
+    """Best time of one draw, replayed from a graph."""
+    s = G.Sampler(nv, **dict(BASE, **params))
+    s.accept(np.asarray(hist, np.int32))
+    fresh, buf, out, st = G.Buffer.from_array(row), G.Buffer(nv * 4), G.Buffer(4), G.Stream()
+
+    def draws():
+        for _ in range(4):
+            G.check(G.lib().g4h_memcpy_d2d(buf.ptr, fresh.ptr, nv * 4, st.ptr))
+            s.sample(buf, out, accept=False, stream=st.ptr)
+
+    G.synchronize()
+    draws()
+    st.synchronize()
+    graph, best = G.Graph(st.ptr, draws), float("inf")
+    for _ in range(6):
+        a, b = G.Event(), G.Event()
+        a.record(st.ptr)
+        graph.launch(st.ptr)
+        b.record(st.ptr)
+        st.synchronize()
+        best = min(best, a.elapsed_ms(b) * 250)
+    return best
+
+
+@pytest.mark.parametrize("ids", [1, 500, None])
+def test_draw_time_is_linear_in_the_window(gpu, ids):
+    """A window of the whole ring costs a few times a short one's draw, not its
+    square (about 1.2 times measured; a walk over the window per entry was 90)."""
+    nv = 32768
+    rs = np.random.default_rng(3)
+    row = make_logits(rs, nv, "plain")
+    hist = rs.integers(0, ids or nv, 4096)
+    short, full = (draw_us(gpu, nv, row, hist, repeat_last_n=n, no_repeat_ngram=0) for n in (1, 4096))
+    assert full < 4 * short, f"{full:.1f} us against {short:.1f} us"
