@@ -185,7 +185,7 @@ struct Lds {
     float bv[NW];
     int bi[NW];
     int suf[64];
-    int flag, n_keep, gathered, id;
+    int flag, n_keep, gathered, above, id;
     double dsum;
 };
 
@@ -208,51 +208,76 @@ __device__ __forceinline__ void wg_counts15(int c[15], Lds &sh, int buf) {
     }
 }
 
+// ids base .. base + 63 of heap_replay, lane i holding id base + i's value
+__device__ __forceinline__ void heap_chunk(float l, int base, int nv, int k, Lds &sh, int &hn, float &root) {
+    const int lane = threadIdx.x & 63, i = base + lane;
+    uint64_t m = __ballot(i < nv && (hn < k || l > root));
+    while (m) {
+        const int j = __builtin_ctzll(m);
+        m &= m - 1;
+        const float v = __shfl(l, j, 64);
+        const int id = base + j;
+        if (hn < k) {
+            int p = hn++;
+            if (lane == 0) { sh.hv[p] = v; sh.hi[p] = id; }
+            while (p > 0) {
+                const int up = (p - 1) / 2;
+                const float a = sh.hv[p], b = sh.hv[up];
+                if (!(a < b)) break;
+                const int ia = sh.hi[p], ib = sh.hi[up];
+                if (lane == 0) { sh.hv[up] = a; sh.hi[up] = ia; sh.hv[p] = b; sh.hi[p] = ib; }
+                p = up;
+            }
+        } else if (v > sh.hv[0]) {
+            if (lane == 0) { sh.hv[0] = v; sh.hi[0] = id; }
+            int p = 0;
+            for (;;) {
+                const int a = 2 * p + 1, b = 2 * p + 2;
+                int lo = p;
+                if (a < k && sh.hv[a] < sh.hv[lo]) lo = a;
+                if (b < k && sh.hv[b] < sh.hv[lo]) lo = b;
+                if (lo == p) break;
+                const float x = sh.hv[lo], y = sh.hv[p];
+                const int ix = sh.hi[lo], iy = sh.hi[p];
+                if (lane == 0) { sh.hv[lo] = y; sh.hi[lo] = iy; sh.hv[p] = x; sh.hi[p] = ix; }
+                p = lo;
+            }
+        }
+        root = sh.hv[0];
+    }
+}
+
 // The reference's heap over ids 0..nv-1 (sampler.c:149-168) on wave 0;
 // lane 0 writes the heap, every lane reads it.  Ids whose value cannot enter
 // (the heap is full and the value is not above its root, which only grows)
-// are skipped 64 at a time.
+// are skipped 1024 or 64 at a time.  The row comes 1024 ids per round trip, the
+// next ones in flight meanwhile: the groups launch leaves it in the other XCDs'
+// L2, and 64 ids per round trip made a replay 1.1 to 1.3 times the one-launch
+// form's (a row of 262144 with ties, its draw and a copy of it: 1093 us there,
+// 1453 after the groups launch, 692 now).
 __device__ void heap_replay(const float *L, int nv, int k, Lds &sh) {
+    constexpr int NC = 16;                                           // chunks of 64 ids per round trip
     const int lane = threadIdx.x & 63;
+    float *stage = reinterpret_cast<float *>(sh.keys);               // each lane's own values of the chunks
     int hn = 0;
-    float root = 0.0f;
-    for (int base = 0; base < nv; base += 64) {
-        const int i = base + lane;
-        const float l = i < nv ? L[i] : 0.0f;
-        uint64_t m = __ballot(i < nv && (hn < k || l > root));
-        while (m) {
-            const int j = __builtin_ctzll(m);
-            m &= m - 1;
-            const float v = __shfl(l, j, 64);
-            const int id = base + j;
-            if (hn < k) {
-                int p = hn++;
-                if (lane == 0) { sh.hv[p] = v; sh.hi[p] = id; }
-                while (p > 0) {
-                    const int up = (p - 1) / 2;
-                    const float a = sh.hv[p], b = sh.hv[up];
-                    if (!(a < b)) break;
-                    const int ia = sh.hi[p], ib = sh.hi[up];
-                    if (lane == 0) { sh.hv[up] = a; sh.hi[up] = ia; sh.hv[p] = b; sh.hi[p] = ib; }
-                    p = up;
-                }
-            } else if (v > sh.hv[0]) {
-                if (lane == 0) { sh.hv[0] = v; sh.hi[0] = id; }
-                int p = 0;
-                for (;;) {
-                    const int a = 2 * p + 1, b = 2 * p + 2;
-                    int lo = p;
-                    if (a < k && sh.hv[a] < sh.hv[lo]) lo = a;
-                    if (b < k && sh.hv[b] < sh.hv[lo]) lo = b;
-                    if (lo == p) break;
-                    const float x = sh.hv[lo], y = sh.hv[p];
-                    const int ix = sh.hi[lo], iy = sh.hi[p];
-                    if (lane == 0) { sh.hv[lo] = y; sh.hi[lo] = iy; sh.hv[p] = x; sh.hi[p] = ix; }
-                    p = lo;
-                }
-            }
-            root = sh.hv[0];
+    float root = 0.0f, cur[NC], nxt[NC];
+    auto load = [&](float (&b)[NC], int first) {
+#pragma unroll
+        for (int q = 0; q < NC; q++) b[q] = first + 64 * q + lane < nv ? L[first + 64 * q + lane] : 0.0f;
+    };
+    load(cur, 0);
+    for (int first = 0; first < nv; first += 64 * NC) {
+        load(nxt, first + 64 * NC);
+        bool any = hn < k;
+#pragma unroll
+        for (int q = 0; q < NC; q++) any |= first + 64 * q + lane < nv && cur[q] > root;
+        if (__ballot(any)) {                                         // uniform
+#pragma unroll
+            for (int q = 0; q < NC; q++) stage[64 * q + lane] = cur[q];
+            for (int q = 0; q < NC && first + 64 * q < nv; q++) heap_chunk(stage[64 * q + lane], first + 64 * q, nv, k, sh, hn, root);
         }
+#pragma unroll
+        for (int q = 0; q < NC; q++) cur[q] = nxt[q];
     }
 }
 
@@ -422,11 +447,12 @@ __device__ int first_argmax_of_groups(const float *L, int nv, const uint32_t (&g
 // Gathers every element of the row at or above a threshold that at least K1
 // elements reach into sh.keys (sh.gathered of them): the threshold is one that
 // at least K1 group maxima reach.  lo: the smallest group maximum, kmax the
-// largest.  False (nothing gathered of use) when ties or a row whose largest
-// values crowd into few groups leave more than GT candidates.
+// largest; lo becomes the threshold.  False (nothing gathered of use) when ties
+// or a row whose largest values crowd into few groups leave more than GT
+// elements at or above it; slow when more than GT elements share the boundary key.
 template <int GS>
-__device__ bool gather_from_groups(const float *L, int nv, int ng, const uint32_t (&gk)[SAMPLER_GROUPS / NT], int K1, uint32_t lo,
-                                   uint32_t kmax, Lds &sh) {
+__device__ bool gather_from_groups(const float *L, int nv, int ng, const uint32_t (&gk)[SAMPLER_GROUPS / NT], int K1, uint32_t &lo,
+                                   uint32_t kmax, bool &slow, Lds &sh) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     constexpr int GPT = SAMPLER_GROUPS / NT;
     const int most = K1 + K1 / 8 + 16;                               // close enough: a few more groups to read
@@ -466,7 +492,11 @@ __device__ bool gather_from_groups(const float *L, int nv, int ng, const uint32_
             hi = (uint32_t)__builtin_amdgcn_readlane((int)pj, 0);
         }
     }
-    if (c_lo > GLIST) return false;
+    // more than GLIST groups share the maximum lo: the fewer than K1 groups above
+    // it either hold K1 larger elements or lo is the boundary key
+    static_assert(GLIST >= GT, "more than GT elements");
+    const bool tied = c_lo > GLIST;
+    if (tied) lo++;
 #pragma unroll
     for (int q = 0; q < GPT; q++) {
         const bool on = t + q * NT < ng && gk[q] >= lo;
@@ -479,6 +509,7 @@ __device__ bool gather_from_groups(const float *L, int nv, int ng, const uint32_
     __syncthreads();
     constexpr int LG = GS / 4;                                       // loads of 4 per group
     const int units = sh.gn * LG;                                    // uniform
+    int above = 0;
     for (int u0 = 0; u0 < units; u0 += 4 * NT) {
         float v[4][4];
         int at[4];
@@ -498,6 +529,7 @@ __device__ bool gather_from_groups(const float *L, int nv, int ng, const uint32_
                 const bool keep = at[q] + e < nv && kk >= lo;
                 const uint64_t m = __ballot(keep);
                 if (m == 0) continue;                                // uniform
+                above += __builtin_popcountll(__ballot(keep && kk > lo));
                 int base = 0;
                 if (lane == 0) base = atomicAdd(&sh.gathered, __builtin_popcountll(m));
                 base = __shfl(base, 0, 64);
@@ -505,7 +537,9 @@ __device__ bool gather_from_groups(const float *L, int nv, int ng, const uint32_
                 if (keep && slot < GT) sh.keys[slot] = ((uint64_t)kk << 32) | (uint32_t)~(uint32_t)(at[q] + e);
             }
     }
+    if (lane == 0 && above) atomicAdd(&sh.above, above);
     __syncthreads();
+    slow = tied ? sh.gathered < K1 : sh.gathered > GT && sh.above < K1;
     return sh.gathered <= GT;
 }
 
@@ -601,7 +635,7 @@ __global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out
     kmin_c = wave_umax(kmin_c);
     const bool wnan = __ballot(nan != 0) != 0;
     if (lane == 0) { sh.red[wave][0] = (int)kmax; sh.red[wave][1] = wnan; sh.red[wave][2] = (int)kmin_c; }
-    if (t == 0) { sh.gathered = 0; sh.gn = 0; sh.flag = 0; }
+    if (t == 0) { sh.gathered = 0; sh.above = 0; sh.gn = 0; sh.flag = 0; }
     __syncthreads();
     kmax = 0;
     kmin_c = 0;
@@ -618,8 +652,9 @@ __global__ __launch_bounds__(NT) void k_sample(SamplerDev *S, float *L, int *out
     bool whole = true;                     // search the row itself
     if constexpr (GS > 0) {
         if (!slow) {
-            whole = !gather_from_groups<GS>(L, nv, ng, gk, K1, lo, kmax, sh);
-            if (whole) lo = 0;             // the smallest key of the groups' maxima is no bound of the row
+            // the threshold left in lo is the bracket's lower end either way:
+            // K1 elements reach it, and with `whole` more than GT do
+            whole = !gather_from_groups<GS>(L, nv, ng, gk, K1, lo, kmax, slow, sh);
             __syncthreads();
             if (whole && t == 0) sh.gathered = 0;
             __syncthreads();

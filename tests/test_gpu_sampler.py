@@ -62,6 +62,14 @@ def make_logits(rs, nv, kind):
         lg[rs.integers(0, nv, 30)] = 2.0 + rs.random(30).astype(np.float32)
     elif kind == "sorted":                    # the largest values all in neighbouring ids
         lg = np.sort(lg)
+    elif kind == "masked":                    # fewer finite values than top-k
+        keep = rs.permutation(nv)[:10]
+        lg, all_ = np.full(nv, -np.inf, np.float32), lg
+        lg[keep] = all_[keep]
+    elif kind in ("crowd", "crowds"):         # equal values, larger ones next to each other
+        n = 150 if kind == "crowd" else 2000
+        lg = np.full(nv, 1.0, np.float32)
+        lg[5000:5000 + n] = 2.0 + rs.permutation(n).astype(np.float32) / n
     elif kind == "zeros":                     # -0 and +0 share the maximum
         lg = -np.abs(lg)
         lg[rs.integers(0, nv, 3)] = -0.0
@@ -262,3 +270,26 @@ def test_draw_time_is_linear_in_the_window(gpu, ids):
     hist = rs.integers(0, ids or nv, 4096)
     short, full = (draw_us(gpu, nv, row, hist, repeat_last_n=n, no_repeat_ngram=0) for n in (1, 4096))
     assert full < 4 * short, f"{full:.1f} us against {short:.1f} us"
+
+
+@pytest.mark.parametrize("nv", [16384, 16387, 65541, 262146])
+@pytest.mark.parametrize("kind", ["masked", "crowd", "crowds"])
+def test_groups_that_share_their_maximum(gpu, oracle, nv, kind):
+    """Most groups share one maximum: the larger elements are fewer than k (ties
+    decide), k to 1024 in few groups, or more than the draw gathers."""
+    rs = np.random.default_rng(nv)
+    for top_k in (40, 511):
+        slow = run_pair(gpu, oracle, nv, dict(BASE, top_k=top_k), rs, kind, 2, bans=[1], hist=rs.integers(0, nv, 40))
+        if kind == "masked" or (kind == "crowd" and top_k == 511):
+            assert slow == 2                  # decided by the heap
+
+
+@pytest.mark.parametrize("kind", ["ties", "masked"])
+def test_tied_rows_cost_no_more_in_two_launches(gpu, kind):
+    """1048576 ids are the largest row of two launches, one id more takes one
+    launch (the group maxima added 34 % to a row with ties)."""
+    us = []
+    for nv in (1048576, 1048577):
+        rs = np.random.default_rng(4)
+        us.append(draw_us(gpu, nv, make_logits(rs, nv, kind), rs.integers(0, nv, 40), no_repeat_ngram=0))
+    assert us[0] < 1.15 * us[1], f"{us[0]:.1f} us against {us[1]:.1f} us"
