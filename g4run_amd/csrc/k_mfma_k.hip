@@ -570,9 +570,12 @@ hipError_t launch_matmul_mfma_k(const g4h_tensor &W, const uint8_t *act, size_t 
 }
 
 // token tiles per wave: two (each weight load and unpack serving 64 tokens)
-// once that still gives every CU a workgroup (q4_K 4096 x 11008, one / two:
-// 64 tokens 18.7 / 25.3 us, 128 tokens 31.1 / 25.9)
-static int mmk_mt(const g4h_tensor &W, int M) { return (W.nrows + 31) / 32 * ((M + 63) / 64) >= 256 ? 2 : 1; }
+// once there are two and that still gives every CU a workgroup.  Measured (us,
+// one / two): q4_K 4096 x 11008 at 64 tokens 18.7 / 25.3, at 128 31.1 / 25.9;
+// q4_K 8192 x 4096 at 33 tokens 14.8 / 12.6.  Up to 32 tokens the second tile is
+// all padding: q4_K 10240 x 4096 at 9 tokens 13.9 / 18.9, q6_K 20480 x 4096 at
+// 32 30.5 / 40.8.
+static int mmk_mt(const g4h_tensor &W, int M) { return M > 32 && (W.nrows + 31) / 32 * ((M + 63) / 64) >= 256 ? 2 : 1; }
 
 hipError_t launch_matmul_mfma_kx(const g4h_tensor &W, const float *x, size_t xs, int M, float *Y, uint8_t *ws, hipStream_t s) {
     if (!mmk_capable(W.type) || M < 1 || !x || !Y || (uintptr_t)ws % 64) return hipErrorInvalidValue;

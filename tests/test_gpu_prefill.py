@@ -251,6 +251,19 @@ def test_kquant_tile_kernel_equals_given_rows(gpu, oracle, name, qt, rows, cols)
         assert "mt=2" in gpu.matmul_describe(t, 129, 2) and "mt=1" in gpu.matmul_describe(t, 33, 2)
 
 
+@pytest.mark.parametrize("name,qt", [("q4_K", 12), ("q6_K", 14)])
+def test_kquant_tile_count_follows_the_tokens(gpu, oracle, name, qt):
+    """A wave takes a second token tile only where there is one: many rows with up
+    to 32 tokens ran one all of padding; the bits are the given rows' either way."""
+    w, x, t = _setup(gpu, qt, 8200, 512, 65, seed=qt)
+    act = oracle.prep_act(qt, x)
+    for m in (9, 32, 33, 64, 65):
+        assert ("mt=2" in gpu.matmul_describe(t, m, 2)) == (m > 32)
+        a = gpu_matmul(gpu, t, x=x[:m].copy(), nb=m, path=2)
+        b = gpu_matmul(gpu, t, act=act[:m].copy(), nb=m, path=2)
+        assert np.array_equal(bits(a), bits(b)), f"{name} M={m}"
+
+
 @pytest.mark.parametrize("name,qt", [("q5_K", 13), ("q3_K", 11), ("q2_K", 10), ("tq2_0", 35)])
 @pytest.mark.parametrize("rows,cols", [(100, 256), (257, 2048), (33, 2304), (260, 4096), (64, 4352), (520, 11008)])
 def test_gemv_order_tiles_equal_gemv(gpu, oracle, name, qt, rows, cols):
