@@ -577,8 +577,24 @@ hipError_t launch_matmul_mfma_k(const g4h_tensor &W, const uint8_t *act, size_t 
 // 32 30.5 / 40.8.
 static int mmk_mt(const g4h_tensor &W, int M) { return M > 32 && (W.nrows + 31) / 32 * ((M + 63) / 64) >= 256 ? 2 : 1; }
 
+// fp32 tokens that k_mmk takes all the same, quantized to rows: q6_K rows of one
+// superblock, where one wave of eight works and the time is its longest chain,
+// shorter by the LDS pass in k_mmk.  Up to 64 tokens, or while every CU has at
+// most one workgroup (us, k_mmk / k_mmk_tile: 4096 x 256 at 9 / 64 tokens 6.8 / 7.1,
+// 7.2 / 7.4; 20480 x 256 at 9 11.4 / 12.4; 256 x 256 at 512 7.2 / 7.4); past both
+// the loads decide (4096 x 256 at 100 tokens 9.8 / 9.0).  q4_K is faster in
+// k_mmk_tile everywhere.
+static bool mmk_from_rows(const g4h_tensor &W, int M) {
+    return W.type == Q6_K && W.nb == 1 && (M <= 64 || (W.nrows + 31) / 32 * ((M + 31) / 32) <= 256);
+}
+
 hipError_t launch_matmul_mfma_kx(const g4h_tensor &W, const float *x, size_t xs, int M, float *Y, uint8_t *ws, hipStream_t s) {
     if (!mmk_capable(W.type) || M < 1 || !x || !Y || (uintptr_t)ws % 64) return hipErrorInvalidValue;
+    if (mmk_from_rows(W, M)) {
+        const size_t stride = 292;                                   // one superblock
+        if (hipError_t e = launch_quantize_q8_K(x, xs, ws, stride, W.ncols, M, s)) return e;
+        return launch_matmul_mfma_k(W, ws, stride, M, Y, s);
+    }
     if (hipError_t e = launch_quantize_q8_K_tile(x, xs, ws, W.ncols, M, W.type, s)) return e;
     const int mt = mmk_mt(W, M), ntok = (M + 32 * mt - 1) / (32 * mt);
     const int64_t grid = (W.nrows + 255) / 256 * 8 * ntok;
@@ -595,9 +611,18 @@ hipError_t launch_matmul_mfma_kx(const g4h_tensor &W, const float *x, size_t xs,
 }
 
 void mmk_describe(const g4h_tensor &W, int M, char *buf, size_t len) {
+    const char *type = W.type == Q4_K ? "q4_K" : "q6_K";
+    if (mmk_from_rows(W, M)) {
+        int64_t grid;
+        int ntok;
+        mmk_grid(W, M, grid, ntok);
+        snprintf(buf, len, "k_mmk<%s> grid=%lld block=%d (int8 MFMA, 32x32 tiles, %d waves split the superblocks; fp32 x quantized to rows)", type,
+                 (long long)grid, 64 * MMK_NW, MMK_NW);
+        return;
+    }
     const int mt = mmk_mt(W, M), ntok = (M + 32 * mt - 1) / (32 * mt);
-    snprintf(buf, len, "k_mmk_tile<%s,mt=%d> grid=%lld block=%d (int8 MFMA, %dx32 tiles, %d waves split the superblocks)",
-             W.type == Q4_K ? "q4_K" : "q6_K", mt, (long long)((W.nrows + 255) / 256 * 8 * ntok), 64 * MMK_NW, 32 * mt, MMK_NW);
+    snprintf(buf, len, "k_mmk_tile<%s,mt=%d> grid=%lld block=%d (int8 MFMA, %dx32 tiles, %d waves split the superblocks; given rows take k_mmk)",
+             type, mt, (long long)((W.nrows + 255) / 256 * 8 * ntok), 64 * MMK_NW, 32 * mt, MMK_NW);
 }
 
 }  // namespace g4

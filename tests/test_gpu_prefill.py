@@ -264,6 +264,18 @@ def test_kquant_tile_count_follows_the_tokens(gpu, oracle, name, qt):
         assert np.array_equal(bits(a), bits(b)), f"{name} M={m}"
 
 
+@pytest.mark.parametrize("name,qt,rows,m,kernel", [("q6_K", 14, 4200, 64, "k_mmk<"), ("q6_K", 14, 4200, 65, "k_mmk_tile<"),
+                                                   ("q6_K", 14, 300, 65, "k_mmk<"), ("q4_K", 12, 300, 64, "k_mmk_tile<")])
+def test_one_superblock_rows(gpu, oracle, name, qt, rows, m, kernel):
+    """256 columns: q6_K takes k_mmk up to 64 tokens, or one workgroup per CU; the
+    bits are the given rows'."""
+    w, x, t = _setup(gpu, qt, rows, 256, m, seed=m)
+    assert gpu.matmul_describe(t, m, 2).startswith(kernel)
+    a = gpu_matmul(gpu, t, x=x, nb=m, path=2)
+    assert np.array_equal(bits(a), bits(gpu_matmul(gpu, t, act=oracle.prep_act(qt, x), nb=m, path=2)))
+    assert_close(a, oracle_matmul(oracle, qt, w, x), f"{name} M={m}")
+
+
 @pytest.mark.parametrize("name,qt", [("q5_K", 13), ("q3_K", 11), ("q2_K", 10), ("tq2_0", 35)])
 @pytest.mark.parametrize("rows,cols", [(100, 256), (257, 2048), (33, 2304), (260, 4096), (64, 4352), (520, 11008)])
 def test_gemv_order_tiles_equal_gemv(gpu, oracle, name, qt, rows, cols):
