@@ -190,10 +190,13 @@ __device__ __forceinline__ uint32_t mmf_round2(uint32_t x, uint32_t y) {
     else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2bf));
 }
 
+// ONE: rows of one chunk (up to 256 columns), which is loaded once and takes one
+// buffer; the loop's loads ahead would all be of the last piece again (us, loop /
+// this: f16 65536 x 256 at 9 / 17 / 80 tokens 14.5 / 16.4 / 40.3 -> 8.1 / 10.3 / 37.3).
 // A32: activation rows of fp32 (row stride `as` bytes), rounded on the way to
 // LDS; else f16 rows.  Workgroup b runs on XCD b % 8: the token tiles of one
 // row tile go to one XCD, consecutively, and find its weights in that XCD's L2.
-template <int WT, bool A32, int MR, int NR>
+template <int WT, bool A32, bool ONE, int MR, int NR>
 __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restrict__ W, size_t ws, int64_t nrows, int64_t ncols,
                                                          const uint8_t *__restrict__ act, size_t as, int M, float *__restrict__ Y,
                                                          int ntok) {
@@ -201,7 +204,8 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
     constexpr int AU = A32 ? 64 : 32, AL = MR * AU / NTH, WL = NR * 32 / NTH;   // 16-byte pieces per row, loads per thread
     static_assert(MR * AU % NTH == 0 && NR * 32 % NTH == 0, "whole loads");
     constexpr int BUF = (MR + NR) * RB, PART = MMF_W * MT * NT * 4096;
-    __shared__ __align__(16) uint8_t lds[2 * BUF > PART ? 2 * BUF : PART];
+    constexpr int STAGED = ONE ? BUF : 2 * BUF;
+    __shared__ __align__(16) uint8_t lds[STAGED > PART ? STAGED : PART];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t) >> 6;
     const int li = lane & 31, kh = lane >> 5;
     const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
@@ -222,7 +226,7 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
     };
     // stages of loads in flight, 48 to 96 registers (64 x 64 workgroups were
     // slower with two: f16 4096 x 4096 at 512 tokens 55.6 / 58.7 us)
-    constexpr int D = AL + WL >= 12 ? 1 : AL + WL >= 8 ? 2 : 4;
+    constexpr int D = ONE || AL + WL >= 12 ? 1 : AL + WL >= 8 ? 2 : 4;
     Stage st[D];
     auto load = [&](Stage &S, int c) __attribute__((always_inline)) {   // past the row's end its last piece again, never used
         const uint32_t wo = min((uint32_t)c * RB + 16 * wc, wlast), ao = min((uint32_t)c * (A32 ? 2 * RB : RB) + 16 * ac, alast);
@@ -293,14 +297,20 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
     // counter waits before a store cover only the stage stored.
 #pragma unroll
     for (int d = 0; d < D; d++) load(st[d], d);
-    for (int c0 = 0; c0 < nc; c0 += D) {                            // uniform
+    if constexpr (ONE) {
+        put(st[0], 0);
+        lds_barrier();
+        mul(0, 0);
+    } else {
+        for (int c0 = 0; c0 < nc; c0 += D) {                        // uniform
 #pragma unroll
-        for (int d = 0; d < D; d++) {
-            if (c0 + d >= nc) break;
-            put(st[d], (c0 + d) & 1);
-            load(st[d], c0 + d + D);
-            lds_barrier();
-            mul((c0 + d) & 1, c0 + d);
+            for (int d = 0; d < D; d++) {
+                if (c0 + d >= nc) break;
+                put(st[d], (c0 + d) & 1);
+                load(st[d], c0 + d + D);
+                lds_barrier();
+                mul((c0 + d) & 1, c0 + d);
+            }
         }
     }
     __syncthreads();
@@ -325,13 +335,16 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
 // Tokens and rows per workgroup: the shape with the least L1 traffic per CU,
 // rounds of workgroups x the bytes a workgroup loads per column (fp32
 // activation rows 4, f16 rows and weights 2 each).  Measured with fp32
-// activations (us, 64-column chunks): f16 4096 x 4096 at 64 tokens 32 x 32 15.9,
-// 64 x 16 21.0, 32 x 64 20.2; at 128 tokens 32 x 64 19.0, 64 x 32 22.9; at 201
-// tokens 64 x 64 25.1, 32 x 64 32.0, 64 x 32 36.2.
+// activations (us): f16 4096 x 4096 at 64 tokens 32 x 32 16.1, 64 x 32 21.3, 64 x 64
+// 25.3; at 200 tokens 64 x 64 26.4, 64 x 32 38.5; 10240 x 4096 at 9 tokens 16 x 64
+// 18.3, 16 x 32 23.7.  Past one 16 x 64 workgroup per CU, 16 x 32 keeps more loads in
+// flight instead: 20480 x 1040 at 9 tokens 16.1 / 12.3, 65536 x 1040 37.3 / 29.6.
+// Shapes that this never finds best are not built (fp32: fewer rows than tokens).
 static void mmf_tiles(bool a32, int64_t nrows, int M, int &mr, int &nr, int &ntok, int64_t &grid) {
     int64_t best = INT64_MAX;
     for (int m = M > 32 ? 64 : M > 16 ? 32 : 16; m >= 16; m >>= 1)
-        for (int n = 64; n >= 16; n >>= 1) {
+        for (int n = 64; n >= (a32 ? m : std::max(16, m / 2)); n >>= 1) {
+            if (m == 16 && n == 64 && nrows > 256 * 64) continue;   // 16 x 32 above
             const int64_t cost = ((M + m - 1) / m * ((nrows + n - 1) / n) + 255) / 256 * ((a32 ? 2 : 1) * m + n);
             if (cost < best) best = cost, mr = m, nr = n;
         }
@@ -340,11 +353,12 @@ static void mmf_tiles(bool a32, int64_t nrows, int M, int &mr, int &nr, int &nto
 }
 
 void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len) {
-    int mr, nr, ntok;
-    int64_t grid;
+    int mr, nr, ntok, pm, pn;
+    int64_t grid, pgrid;
+    mmf_tiles(wtype != F16, nrows, M, pm, pn, ntok, pgrid);
     mmf_tiles(true, nrows, M, mr, nr, ntok, grid);
-    snprintf(buf, len, "k_mm_float<%s,%dx%d> grid=%lld block=%d (matrix cores, %d waves split the columns)",
-             wtype == F16 ? "f16" : "bf16", mr, nr, (long long)grid, 64 * MMF_W, MMF_W);
+    snprintf(buf, len, "k_mm_float<%s,%dx%d> grid=%lld block=%d (matrix cores, %d waves split the columns; given rows %dx%d)",
+             wtype == F16 ? "f16" : "bf16", mr, nr, (long long)grid, 64 * MMF_W, MMF_W, pm, pn);
 }
 
 template <int WT, bool A32>
@@ -355,13 +369,14 @@ static hipError_t mmf_go(const uint8_t *W, size_t ws, int64_t nrows, int64_t nco
     mmf_tiles(A32, nrows, M, mr, nr, ntok, grid);
     if (grid > 0x7fffffff || ncols >= (int64_t)1 << 29) return hipErrorInvalidValue;
 #define G4_MMF(MR_, NR_)                                                                                                       \
-    if (mr == MR_ && nr == NR_) {                                                                                              \
-        hipLaunchKernelGGL((k_mm_float<WT, A32, MR_, NR_>), dim3((unsigned)grid), dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, \
-                           M, Y, ntok);                                                                                        \
-        return hipGetLastError();                                                                                              \
-    }
-    G4_MMF(16, 16) G4_MMF(16, 32) G4_MMF(16, 64) G4_MMF(32, 16) G4_MMF(32, 32) G4_MMF(32, 64) G4_MMF(64, 16) G4_MMF(64, 32)
-    G4_MMF(64, 64)
+    if constexpr (!A32 || NR_ >= MR_)                                                                                          \
+        if (mr == MR_ && nr == NR_) {                                                                                          \
+            const dim3 g((unsigned)grid), t(64 * MMF_W);                                                                       \
+            if (ncols <= MMF_KC) hipLaunchKernelGGL((k_mm_float<WT, A32, true, MR_, NR_>), g, t, 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok); \
+            else hipLaunchKernelGGL((k_mm_float<WT, A32, false, MR_, NR_>), g, t, 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok); \
+            return hipGetLastError();                                                                                          \
+        }
+    G4_MMF(16, 16) G4_MMF(16, 32) G4_MMF(16, 64) G4_MMF(32, 16) G4_MMF(32, 32) G4_MMF(32, 64) G4_MMF(64, 32) G4_MMF(64, 64)
 #undef G4_MMF
     return hipErrorInvalidValue;
 }

@@ -190,3 +190,57 @@ def test_matrix_cores_tile_shapes_same_bits(gpu, oracle, name, wt, rows, cols):
         assert len(shapes) >= 2, shapes
     finally:
         t.free()
+
+
+# every tile shape the dispatch takes: from fp32 tokens (bf16: from prepared rows
+# too), and from prepared f16 rows
+@pytest.mark.parametrize("name,wt", FLOAT)
+@pytest.mark.parametrize("cols", [112, 256, 576, 1072])
+@pytest.mark.parametrize("rows,m,shape,given", [(100, 9, "16x16", "16x16"), (8190, 13, "16x32", "16x32"), (16000, 16, "16x64", "16x64"),
+                                                (16500, 16, "16x32", "16x32"), (2040, 33, "16x32", "32x16"),
+                                                (8190, 30, "32x32", "32x32"), (16000, 31, "32x64", "32x64"), (4090, 100, "32x64", "64x32"),
+                                                (16000, 64, "64x64", "64x64")])
+def test_every_tile_shape(gpu, oracle, name, wt, cols, rows, m, shape, given):
+    """Rows of one 256-column chunk (with and without a remainder), of an odd and
+    an even number of chunks; the first and last weight rows give the bits of
+    the same rows as a small matrix (16 x 16 or 16 x 32 tiles), whose values
+    are within tolerance of the oracle's dots."""
+    from g4run_amd import synth
+    w = _weights(wt, rows, cols, seed=rows + cols)
+    x = synth.activations(m, cols, seed=cols + m)
+    act = oracle.prep_act(wt, x)
+    pick = np.r_[0:48, rows - 48:rows]
+    t, ts = gpu.Tensor.from_rows(wt, w, cols), gpu.Tensor.from_rows(wt, w[pick].copy(), cols)
+    try:
+        d = gpu.matmul_describe(t, m, 2)
+        assert f",{shape}>" in d and d.endswith(f"given rows {given if wt == 1 else shape})"), d
+        small = gpu_matmul(gpu, ts, x=x, nb=m, path=2)
+        assert_close(small, oracle_matmul(oracle, wt, w[pick].copy(), x), f"{name} {rows}x{cols}")
+        for y in (gpu_matmul(gpu, t, x=x, nb=m, path=2), gpu_matmul(gpu, t, act=act, nb=m, path=2)):
+            assert np.array_equal(bits(np.ascontiguousarray(y[:, pick])), bits(small)), f"{name} {rows}x{cols} M={m}"
+    finally:
+        t.free()
+        ts.free()
+
+
+def test_one_chunk_rows_cost_less_than_two(gpu):
+    """A row of 256 columns is one chunk and is loaded once: its batch takes well
+    under the time of 1024 columns (about 0.28 of it; 0.44 with the loop's loads
+    ahead and 16 x 64 tiles)."""
+    us = []
+    for cols in (256, 1024):
+        t = gpu.Tensor.from_rows(1, np.tile(_weights(1, 64, cols, seed=1), (1024, 1)), cols)
+        x, y, st = gpu.Buffer.from_array(np.ones((9, cols), np.float32)), gpu.Buffer(9 * 65536 * 4), gpu.Stream()
+        gpu.matmul(t, y, nb=9, x=x, path=2, stream=st.ptr)
+        st.synchronize()
+        g, best = gpu.Graph(st.ptr, lambda: [gpu.matmul(t, y, nb=9, x=x, path=2, stream=st.ptr) for _ in range(8)]), float("inf")
+        for _ in range(6):
+            a, b = gpu.Event(), gpu.Event()
+            a.record(st.ptr)
+            g.launch(st.ptr)
+            b.record(st.ptr)
+            st.synchronize()
+            best = min(best, a.elapsed_ms(b) * 125)
+        us.append(best)
+        t.free()
+    assert us[0] < 0.4 * us[1], us
