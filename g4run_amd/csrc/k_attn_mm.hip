@@ -100,17 +100,29 @@ __device__ __forceinline__ void amm_view(AmmArgs &c) {
     c.span = c.p0 + c.nb - c.jb;
 }
 
-// Workgroup l of n_kv x n position blocks x ntt token tiles runs on XCD l % 8:
-// the tiles that share a block's K or V rows go to one XCD, consecutively, and
-// find them in its L2.  The grid is padded to whole groups of 8 blocks.
-__device__ __forceinline__ bool amm_block(const AmmArgs &c, int l, int n, int &kvh, int &blk, int &tt) {
-    const int j = l >> 3, pair = (j / c.ntt) * 8 + (l & 7);
-    tt = j % c.ntt;
+// Workgroup l of a call's n_kv x n position blocks x ntt token tiles runs on XCD
+// l % 8.  The tiles that share a block's K or V rows are neighbours on one XCD
+// and find them in its L2: each XCD takes an eighth of the tiles, whatever the
+// number of blocks.  (With whole blocks dealt to the XCDs in turn, two blocks of
+// one KV head kept six XCDs idle: 256 tokens at position 0, 8 q / 1 kv heads of
+// 512, 42.6 us, now 23.6; 64 tokens at position 4096, 8 q / 4 kv heads of 128, 26.6
+// and 23.7.)  From AMM_ROUNDS tiles whole rounds of 8 blocks are dealt so all the
+// same and an eighth of the rest to each: the XCDs then read neighbouring rows at
+// any one time (256 tokens at position 16000, 32 q / 4 kv heads of 256, 1005 us
+// against 1044).  n counts the blocks up to the call's last position; the grid may
+// be sized for more.
+constexpr int AMM_ROUNDS = 4096;
+__device__ __forceinline__ bool amm_block(const AmmArgs &c, int l, int size, int &kvh, int &blk, int &tt) {
+    const int n = (c.span + size - 1) / size, pairs = c.n_kv * n, total = pairs * c.ntt;
+    const int rounds = total >= AMM_ROUNDS ? pairs >> 3 : 0, whole = rounds * c.ntt, left = total - 8 * whole, per = (left + 7) >> 3;
+    const int x = l & 7, i = l >> 3, item = i < whole ? i : x * per + i - whole, p = item / c.ntt;
+    const int pair = i < whole ? p * 8 + x : 8 * rounds + p;
+    tt = item - p * c.ntt;
     kvh = pair / n;
     blk = pair - kvh * n;
-    return pair < c.n_kv * n;
+    return i < whole || (i - whole < per && item < left);
 }
-static unsigned amm_blocks(const AmmArgs &c, int n) { return (unsigned)((c.n_kv * n + 7) / 8 * 8) * c.ntt; }
+static unsigned amm_blocks(const AmmArgs &c, int n) { return (unsigned)((c.n_kv * n * c.ntt + 7) / 8 * 8); }
 
 __device__ __forceinline__ am_v8h amm_ld8(const void *p) { return *(const am_v8h *)p; }
 __device__ __forceinline__ am_v16f amm_mma(am_v8h a, am_v8h b, am_v16f c) {
@@ -146,7 +158,7 @@ __global__ __launch_bounds__(256) void k_amm_scores(AmmArgs c) {
     __shared__ double wl[4][32];
     amm_view(c);
     int kvh, tt, ch;
-    if (!amm_block(c, blockIdx.x, c.nch, kvh, ch, tt) || ch * AMM_CH >= c.span) return;   // past the call's last position
+    if (!amm_block(c, blockIdx.x, AMM_CH, kvh, ch, tt)) return;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 31, kh = lane >> 5;
     const int jw = ch * AMM_CH + wave * 32;                          // the wave's first position
     const int jfirst = c.window ? max(0, c.p0 + 1 - c.window) : 0, jlast = c.jb + c.span - 1;
@@ -246,7 +258,7 @@ __global__ __launch_bounds__(512, 4) void k_amm_v(AmmArgs c) {
     __shared__ __align__(16) uint8_t vsh[8][HP * 64];               // a wave's part of V: rows of 32 columns
     amm_view(c);
     int kvh, tt, cv;
-    if (!amm_block(c, blockIdx.x, c.nchv, kvh, cv, tt) || cv * AMM_NP >= c.span) return;   // past the call's last position
+    if (!amm_block(c, blockIdx.x, AMM_NP, kvh, cv, tt)) return;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t) >> 6, li = lane & 31, kh = lane >> 5;
     const int jl0 = cv * AMM_NP, unit = wave + 8 * blockIdx.y;
     const int jfirst = c.window ? max(0, c.p0 + 1 - c.window) : 0, jlast = c.jb + c.span - 1;

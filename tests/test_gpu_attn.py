@@ -572,3 +572,53 @@ def test_prefill_matrix_cores_errors(gpu):
     with pytest.raises(G.G4HError) as e:                              # a batch longer than the ring allows
         G.attn_prefill_mm(b, b, b, G.F16, 8, 1, 256, 10, 70, b, window=512, ring=576)
     assert e.value.status == G.ERR_ARG
+
+
+# position blocks x token tiles dealt to the 8 XCDs: fewer than 8 blocks, whole
+# and broken eighths, and calls of 4096 tiles and more (whole rounds of blocks
+# and a rest: scores at the first such case, values too at the second)
+@pytest.mark.parametrize("n_kv,grp,hd,pos0,nb", [(1, 8, 512, 0, 256), (1, 8, 256, 0, 9), (3, 2, 64, 1000, 33), (1, 1, 128, 1030, 70),
+                                                 (4, 8, 64, 1900, 250), (4, 8, 64, 4000, 256)])
+def test_prefill_matrix_cores_blocks_and_tiles(gpu, n_kv, grp, hd, pos0, nb):
+    """Every (block, tile) pair is taken once: the rows equal those of the same
+    tokens in batches of up to 7."""
+    G, H = gpu, n_kv * grp
+    rs = np.random.default_rng(hd + nb)
+    k, v = (G.Buffer.from_array(rs.standard_normal((pos0 + nb, n_kv, hd)).astype(np.float16)) for _ in range(2))
+    q = (rs.standard_normal((nb, H, hd)) * 2 / np.sqrt(hd)).astype(np.float32)
+
+    def rows(b0, cnt):
+        out = G.Buffer.from_array(np.full((cnt, H, hd), np.nan, np.float32))
+        G.attn_prefill_mm(G.Buffer.from_array(np.ascontiguousarray(q[b0:b0 + cnt])), k, v, G.F16, H, n_kv, hd, pos0 + b0, cnt, out)
+        G.synchronize()
+        return out.download(np.float32, (cnt, H, hd))
+
+    full = rows(0, nb)
+    assert np.isfinite(full).all()
+    for b0 in {0, (nb - 7) // 2, nb - 7}:
+        assert np.array_equal(full[b0:b0 + 7].view(np.uint32), rows(b0, 7).view(np.uint32)), f"token {b0}"
+
+
+def test_prefill_matrix_cores_few_blocks_fill_the_chip(gpu):
+    """256 tokens at position 0 are a few position blocks of one KV head: about
+    half the time of the same tokens at position 1000 (0.76 when whole blocks
+    went to one XCD each)."""
+    G, us = gpu, []
+    for pos0 in (0, 1000):
+        c = G.Buffer.from_array(np.ones((pos0 + 256, 1, 512), np.float16))
+        q, out = G.Buffer.from_array(np.ones((256, 8, 512), np.float32)), G.Buffer(256 * 8 * 512 * 4)
+        ws, st = G.Buffer(G.attn_prefill_workspace_bytes(8, 512, pos0, 256)), G.Stream()
+        run = lambda: G.attn_prefill_mm(q, c, c, G.F16, 8, 1, 512, pos0, 256, out, ws=ws, stream=st.ptr)  # noqa: E731
+        G.synchronize()
+        run()
+        st.synchronize()
+        g, best = G.Graph(st.ptr, lambda: [run() for _ in range(8)]), float("inf")
+        for _ in range(6):
+            a, b = G.Event(), G.Event()
+            a.record(st.ptr)
+            g.launch(st.ptr)
+            b.record(st.ptr)
+            st.synchronize()
+            best = min(best, a.elapsed_ms(b) * 125)
+        us.append(best)
+    assert us[0] < 0.64 * us[1], us
