@@ -122,7 +122,7 @@ __device__ __forceinline__ bool amm_block(const AmmArgs &c, int l, int size, int
     blk = pair - kvh * n;
     return i < whole || (i - whole < per && item < left);
 }
-static unsigned amm_blocks(const AmmArgs &c, int n) { return (unsigned)((c.n_kv * n * c.ntt + 7) / 8 * 8); }
+static int64_t amm_blocks(const AmmArgs &c, int n) { return ((int64_t)c.n_kv * n * c.ntt + 7) / 8 * 8; }
 
 __device__ __forceinline__ am_v8h amm_ld8(const void *p) { return *(const am_v8h *)p; }
 __device__ __forceinline__ am_v16f amm_mma(am_v8h a, am_v8h b, am_v16f c) {
@@ -439,8 +439,8 @@ bool attn_batch_mm_ok(const QkvArgs &a) {
 
 template <int HD, int GRP>
 static void amm_go(const AmmArgs &c, hipStream_t s) {
-    hipLaunchKernelGGL((k_amm_scores<HD, GRP>), dim3(amm_blocks(c, c.nch)), dim3(256), 0, s, c);
-    hipLaunchKernelGGL((k_amm_v<HD, GRP>), dim3(amm_blocks(c, c.nchv), HD == 512 ? 2 : 1), dim3(512), 0, s, c);
+    hipLaunchKernelGGL((k_amm_scores<HD, GRP>), dim3((unsigned)amm_blocks(c, c.nch)), dim3(256), 0, s, c);
+    hipLaunchKernelGGL((k_amm_v<HD, GRP>), dim3((unsigned)amm_blocks(c, c.nchv), HD == 512 ? 2 : 1), dim3(512), 0, s, c);
     hipLaunchKernelGGL(k_amm_combine<HD>, dim3(c.n_head, c.nb), dim3(256), 0, s, c);
 }
 
@@ -480,7 +480,7 @@ hipError_t launch_attn_batch_mm(const float *q, const QkvArgs &a, int npos0, int
     const int grp = a.n_head / a.n_kv;
     c.ntt = (nb + 32 / grp - 1) / (32 / grp);
     const AmmWs w = amm_ws(a.n_head, a.hd, nb, span);
-    if (ws_bytes < w.total || (size_t)c.n_kv * c.ntt > 0x7fffffff) return hipErrorInvalidValue;
+    if (ws_bytes < w.total || amm_blocks(c, c.nch) > max_grid(256) || amm_blocks(c, c.nchv) > max_grid(512)) return hipErrorInvalidValue;
     c.S = (float *)(ws + w.S);
     c.Mc = (float *)(ws + w.Mc);
     c.Lc = (double *)(ws + w.Lc);

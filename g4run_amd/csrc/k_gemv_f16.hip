@@ -351,14 +351,24 @@ static void mmf_tiles(bool a32, int64_t nrows, int M, int &mr, int &nr, int &nto
     ntok = (M + mr - 1) / mr;
     grid = ((nrows + nr - 1) / nr + 7) / 8 * 8 * ntok;
 }
+// token tiles of one launch (all of them, but for outputs of 2^33 values and more)
+static int mmf_tok(int64_t grid, int ntok) { return (int)std::min<int64_t>(ntok, max_grid(64 * MMF_W) / (grid / ntok)); }
 
 void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len) {
     int mr, nr, ntok, pm, pn;
     int64_t grid, pgrid;
     mmf_tiles(wtype != F16, nrows, M, pm, pn, ntok, pgrid);
     mmf_tiles(true, nrows, M, mr, nr, ntok, grid);
-    snprintf(buf, len, "k_mm_float<%s,%dx%d> grid=%lld block=%d (matrix cores, %d waves split the columns; given rows %dx%d)",
-             wtype == F16 ? "f16" : "bf16", mr, nr, (long long)grid, 64 * MMF_W, MMF_W, pm, pn);
+    const int nt = mmf_tok(grid, ntok);
+    snprintf(buf, len, "k_mm_float<%s,%dx%d> grid=%lld block=%d (x%d launches; matrix cores, %d waves split the columns; given rows %dx%d)",
+             wtype == F16 ? "f16" : "bf16", mr, nr, (long long)(grid / ntok * nt), 64 * MMF_W, nt ? (ntok + nt - 1) / nt : 0, MMF_W, pm, pn);
+}
+
+template <int WT, bool A32, int MR, int NR>
+static void mmf_run(dim3 g, const uint8_t *W, size_t ws, int64_t nrows, int64_t ncols, const uint8_t *a, size_t ab, int M, float *Y, int ntok,
+                    hipStream_t s) {
+    if (ncols <= MMF_KC) hipLaunchKernelGGL((k_mm_float<WT, A32, true, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
+    else hipLaunchKernelGGL((k_mm_float<WT, A32, false, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
 }
 
 template <int WT, bool A32>
@@ -367,18 +377,21 @@ static hipError_t mmf_go(const uint8_t *W, size_t ws, int64_t nrows, int64_t nco
     int mr, nr, ntok;
     int64_t grid;
     mmf_tiles(A32, nrows, M, mr, nr, ntok, grid);
-    if (grid > 0x7fffffff || ncols >= (int64_t)1 << 29) return hipErrorInvalidValue;
-#define G4_MMF(MR_, NR_)                                                                                                       \
-    if constexpr (!A32 || NR_ >= MR_)                                                                                          \
-        if (mr == MR_ && nr == NR_) {                                                                                          \
-            const dim3 g((unsigned)grid), t(64 * MMF_W);                                                                       \
-            if (ncols <= MMF_KC) hipLaunchKernelGGL((k_mm_float<WT, A32, true, MR_, NR_>), g, t, 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok); \
-            else hipLaunchKernelGGL((k_mm_float<WT, A32, false, MR_, NR_>), g, t, 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok); \
-            return hipGetLastError();                                                                                          \
-        }
-    G4_MMF(16, 16) G4_MMF(16, 32) G4_MMF(16, 64) G4_MMF(32, 16) G4_MMF(32, 32) G4_MMF(32, 64) G4_MMF(64, 32) G4_MMF(64, 64)
+    const int nt = mmf_tok(grid, ntok);
+    if (nt < 1 || ncols >= MMF_MAX_COLS) return hipErrorInvalidValue;
+    for (int64_t m0 = 0; m0 < M; m0 += (int64_t)nt * mr) {          // one launch as a rule
+        const int m = (int)std::min<int64_t>(M - m0, (int64_t)nt * mr), n = (m + mr - 1) / mr;
+        const dim3 g((unsigned)(grid / ntok * n));
+        bool run = false;
+#define G4_MMF(MR_, NR_)                                                                                          \
+        if constexpr (!A32 || NR_ >= MR_)                                                                         \
+            if (mr == MR_ && nr == NR_) mmf_run<WT, A32, MR_, NR_>(g, W, ws, nrows, ncols, a + m0 * ab, ab, m, Y + m0 * nrows, n, s), run = true;
+        G4_MMF(16, 16) G4_MMF(16, 32) G4_MMF(16, 64) G4_MMF(32, 16) G4_MMF(32, 32) G4_MMF(32, 64) G4_MMF(64, 32) G4_MMF(64, 64)
 #undef G4_MMF
-    return hipErrorInvalidValue;
+        if (!run) return hipErrorInvalidValue;
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 // M tokens of f16 / bf16 weight rows (ws bytes apart, ncols % 16 == 0) on the

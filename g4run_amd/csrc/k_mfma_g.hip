@@ -310,18 +310,29 @@ static int mmg_classes(const g4h_tensor &W) {
     gemv_shape(W.type, W.nb, &lpr, &upl);
     return lpr == 16 || lpr == 32 || lpr == 64 ? lpr / 4 : 0;
 }
+// token tiles of one launch (all of them, but for outputs of 2^33 values and more)
+static int mmg_tok(const g4h_tensor &W, int M) {
+    return (int)std::min<int64_t>((M + 31) / 32, max_grid(mmg_classes(W) < 8 ? 256 : 512) / ((W.nrows + 255) / 256 * 8));
+}
 bool mmg_fits(const g4h_tensor &W, int M) {
     if (W.type != Q5_K && W.type != Q3_K && W.type != Q2_K && W.type != TQ2_0) return false;
-    return M > 8 && mmg_classes(W) && (W.nrows + 255) / 256 * 8 * ((M + 31) / 32) <= 0x7fffffff;
+    return M > 8 && mmg_classes(W) && mmg_tok(W, M) > 0;
 }
 
 template <int T>
-static void mmg_go(const g4h_tensor &W, const uint8_t *ws, int M, float *Y, int nc, hipStream_t s) {
-    const int ntok = (M + 31) / 32;
-    const dim3 g((unsigned)((W.nrows + 255) / 256 * 8 * ntok));
-    if (nc == 4) hipLaunchKernelGGL((k_mmg<T, 4>), g, dim3(256), 0, s, W, ws, M, Y, ntok);
-    else if (nc == 8) hipLaunchKernelGGL((k_mmg<T, 8>), g, dim3(512), 0, s, W, ws, M, Y, ntok);
-    else hipLaunchKernelGGL((k_mmg<T, 16>), g, dim3(512), 0, s, W, ws, M, Y, ntok);
+static hipError_t mmg_go(const g4h_tensor &W, const uint8_t *ws, int M, float *Y, int nc, hipStream_t s) {
+    const int nt = mmg_tok(W, M);
+    for (int64_t m0 = 0; m0 < M; m0 += (int64_t)nt * 32) {              // one launch as a rule
+        const int m = (int)std::min<int64_t>(M - m0, (int64_t)nt * 32), ntok = (m + 31) / 32;
+        const dim3 g((unsigned)((W.nrows + 255) / 256 * 8 * ntok));
+        const uint8_t *a = ws + (size_t)m0 * W.nb * 292;
+        float *y = Y + (size_t)m0 * W.nrows;
+        if (nc == 4) hipLaunchKernelGGL((k_mmg<T, 4>), g, dim3(256), 0, s, W, a, m, y, ntok);
+        else if (nc == 8) hipLaunchKernelGGL((k_mmg<T, 8>), g, dim3(512), 0, s, W, a, m, y, ntok);
+        else hipLaunchKernelGGL((k_mmg<T, 16>), g, dim3(512), 0, s, W, a, m, y, ntok);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_matmul_mfma_gx(const g4h_tensor &W, const float *x, size_t xs, int M, float *Y, uint8_t *ws, hipStream_t s) {
@@ -329,19 +340,18 @@ hipError_t launch_matmul_mfma_gx(const g4h_tensor &W, const float *x, size_t xs,
     if (hipError_t e = launch_quantize_q8_K_tile(x, xs, ws, W.ncols, M, W.type, s)) return e;
     const int nc = mmg_classes(W);
     switch (W.type) {
-    case Q5_K: mmg_go<Q5_K>(W, ws, M, Y, nc, s); break;
-    case Q3_K: mmg_go<Q3_K>(W, ws, M, Y, nc, s); break;
-    case Q2_K: mmg_go<Q2_K>(W, ws, M, Y, nc, s); break;
-    default: mmg_go<TQ2_0>(W, ws, M, Y, nc, s); break;
+    case Q5_K: return mmg_go<Q5_K>(W, ws, M, Y, nc, s);
+    case Q3_K: return mmg_go<Q3_K>(W, ws, M, Y, nc, s);
+    case Q2_K: return mmg_go<Q2_K>(W, ws, M, Y, nc, s);
+    default: return mmg_go<TQ2_0>(W, ws, M, Y, nc, s);
     }
-    return hipGetLastError();
 }
 
 void mmg_describe(const g4h_tensor &W, int M, char *buf, size_t len) {
-    const int nc = mmg_classes(W);
-    snprintf(buf, len, "k_mmg<%s,classes=%d> grid=%lld block=%d (int8 MFMA in the GEMV's order, fp32 x; given rows take the GEMV chunks)",
+    const int nc = mmg_classes(W), nt = mmg_tok(W, M);
+    snprintf(buf, len, "k_mmg<%s,classes=%d> grid=%lld block=%d (x%d launches; int8 MFMA in the GEMV's order, fp32 x; given rows take the GEMV chunks)",
              W.type == Q5_K ? "q5_K" : W.type == Q3_K ? "q3_K" : W.type == Q2_K ? "q2_K" : "tq2_0", nc,
-             (long long)((W.nrows + 255) / 256 * 8 * ((M + 31) / 32)), nc < 8 ? 256 : 512);
+             (long long)((W.nrows + 255) / 256 * 8 * nt), nc < 8 ? 256 : 512, ((M + 31) / 32 + nt - 1) / nt);
 }
 
 }  // namespace g4

@@ -7,6 +7,8 @@ The per-block integer sums come out of one int8 MFMA per block and are exact
 by construction; the fp32 results must be within |gpu - cpu| <= 1e-5 +
 1e-3*|cpu| of the oracle (the fp32 order differs from the CPU's 8-lane one).
 """
+import re
+
 import numpy as np
 import pytest
 
@@ -298,3 +300,37 @@ def test_gemv_order_tiles_equal_gemv(gpu, oracle, name, qt, rows, cols):
     for m in (1, 9, 31, 32, 33, 64, 70):
         a = gpu_matmul(gpu, t, x=x[:m].copy(), nb=m, path=0)
         assert np.array_equal(bits(a), bits(full[:m])), f"{name} {rows}x{cols} M={m}"
+
+
+@pytest.mark.parametrize("qt", [13, 35, 1, 30])
+@pytest.mark.parametrize("rows,m", [(262144, 32800), (262144, 200000), (1 << 20, 60000)])
+def test_launches_stay_below_the_grid_limit(gpu, qt, rows, m):
+    """HIP takes gridDim * blockDim below 2^32: outputs of 2^33 values (q5_K and the
+    like) or 2^35 (f16 / bf16) and more run as several launches."""
+    t = gpu.Tensor(qt, 2304 if qt in (13, 35) else 256, rows)
+    d = gpu.matmul_describe(t, m, 0)
+    grid, block, n = (int(v) for v in re.search(r"grid=(\d+) block=(\d+) \(x(\d+) launches", d).groups())
+    assert d.startswith("k_mmg<" if qt in (13, 35) else "k_mm_float<")
+    assert grid * block < 1 << 32 and grid * n * (32 * 32 if qt in (13, 35) else 64 * 64) >= rows * m, d
+
+
+def test_batch_of_two_launches(gpu):
+    """An output past one launch's grid: tokens of the first launch, on both sides
+    of the cut, and of the last, ragged tile have the bits of a small batch."""
+    from g4run_amd import synth
+    rows, m, cols = 262144, 32799, 2304
+    w = synth.weights(35, 4096, cols, seed=1)
+    t, small = gpu.Tensor.from_rows(35, np.tile(w, (rows // 4096, 1)), cols), gpu.Tensor.from_rows(35, w, cols)
+    x = np.tile(synth.activations(33, cols, seed=2), (m // 33 + 1, 1))[:m]
+    d = gpu.matmul_describe(t, m, 0)
+    grid, n = (int(v) for v in re.search(r"grid=(\d+) .*\(x(\d+) launches", d).groups())
+    cut = grid // (rows // 32) * 32
+    assert n == 2 and 0 < cut < m
+    Y = gpu.Buffer(m * rows * 4)
+    gpu.matmul(t, Y, nb=m, x=gpu.Buffer.from_array(x))
+    gpu.synchronize()
+    for b in (0, 31, cut - 1, cut, m - 1):
+        y = Y.download(np.float32, (rows,), offset=b * rows * 4)
+        ref = gpu_matmul(gpu, small, x=np.ascontiguousarray(np.tile(x[b], (9, 1))), nb=9)[0]
+        assert np.array_equal(bits(y.reshape(-1, 4096)), np.tile(bits(ref), (rows // 4096, 1))), f"token {b}"
+    Y.free()
