@@ -48,6 +48,11 @@ typedef _Float16 mg_v8h __attribute__((ext_vector_type(8)));
 typedef unsigned short mg_v2u __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ mg_v4i mg_ld(const uint8_t *p) { return *(const mg_v4i *)p; }
+// activations: the ragged last tile of the layout is 4-byte aligned (one global
+// load all the same)
+typedef int mg_v4i4 __attribute__((ext_vector_type(4), aligned(4)));
+static_assert(alignof(mg_v4i4) == 4, "superblocks of TL * 292 bytes");
+__device__ __forceinline__ mg_v4i mg_ld_act(const uint8_t *p) { return *(const mg_v4i4 *)p; }
 __device__ __forceinline__ mg_v16i mg_mma(mg_v4i a, mg_v4i b, mg_v16i c) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ uint32_t mg_pkmul(uint32_t a, uint32_t b) {   // 16-bit halves, modulo 2^16
     return __builtin_bit_cast(uint32_t, (mg_v2u)(__builtin_bit_cast(mg_v2u, a) * __builtin_bit_cast(mg_v2u, b)));
@@ -143,10 +148,10 @@ __global__ __launch_bounds__(NC < 8 ? 256 : 512) void k_mmg(g4h_tensor W, const 
     float d;
     const mg_v16i z = {};
     const mg_v16f zf = {};
-    auto load_a = [&](int j, int s) __attribute__((always_inline)) { a[j] = mg_ld(ab + (size_t)s * TL * 292 + 2 * j * TL * 16 + ao); };
+    auto load_a = [&](int j, int s) __attribute__((always_inline)) { a[j] = mg_ld_act(ab + (size_t)s * TL * 292 + 2 * j * TL * 16 + ao); };
     auto load_s = [&](int s) __attribute__((always_inline)) {
         const uint8_t *b = ab + (size_t)s * TL * 292;
-        if constexpr (MINS) bs = mg_ld(b + TL * 256 + ao);
+        if constexpr (MINS) bs = mg_ld_act(b + TL * 256 + ao);
         d = *(const float *)(b + TL * 288 + 4 * tl);
     };
     if (wave * CPW < nb) {

@@ -51,6 +51,12 @@ typedef _Float16 mk_v8h __attribute__((ext_vector_type(8)));
 constexpr int MMK_NW = 8;             // waves per workgroup, splitting the superblocks of one 32 x 32 tile
 
 __device__ __forceinline__ mk_v4i mk_ld(const uint8_t *p) { return *(const mk_v4i *)p; }
+// activations: given q8_K rows, and the ragged last tile of the operand layout,
+// are 4-byte aligned (one global load all the same)
+typedef int mk_v4i4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef int mk_v2i4 __attribute__((ext_vector_type(2), aligned(4)));
+static_assert(alignof(mk_v4i4) == 4 && alignof(mk_v2i4) == 4, "superblocks of 292 bytes");
+__device__ __forceinline__ mk_v4i mk_ld_act(const uint8_t *p) { return *(const mk_v4i4 *)p; }
 __device__ __forceinline__ mk_v16i mk_mma(mk_v4i a, mk_v4i b, mk_v16i c) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ mk_v16i mk_mma16(mk_v2i a, mk_v2i b, mk_v16i c) {
     return __builtin_amdgcn_mfma_i32_32x32x16_i8(__builtin_bit_cast(long, a), __builtin_bit_cast(long, b), c, 0, 0, 0);
@@ -68,8 +74,8 @@ struct MkAct {
 };
 __device__ __forceinline__ void mk_load_act(MkAct &a, const uint8_t *ab, int kh) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) a.q[j] = mk_ld(ab + 4 + 32 * j + 16 * kh);
-    a.bs = mk_ld(ab + 260 + 16 * kh);
+    for (int j = 0; j < 8; j++) a.q[j] = mk_ld_act(ab + 4 + 32 * j + 16 * kh);
+    a.bs = mk_ld_act(ab + 260 + 16 * kh);
     a.d = *(const float *)ab;
 }
 // the 8 int16 bsums as fp16 (exact: |bsum| <= 16 * 128)
@@ -172,8 +178,11 @@ struct Q6KSb {
     }
     static __device__ __forceinline__ void load_act(MkAct &a, const uint8_t *ab, int kh) {
 #pragma unroll
-        for (int g = 0; g < 8; g++) a.q[g] = ld_split(ab + 4 + 32 * g + 8 * kh);
-        a.bs = mk_ld(ab + 260 + 16 * kh);
+        for (int g = 0; g < 8; g++) {
+            const mk_v2i lo = *(const mk_v2i4 *)(ab + 4 + 32 * g + 8 * kh), hi = *(const mk_v2i4 *)(ab + 20 + 32 * g + 8 * kh);
+            a.q[g] = mk_v4i{lo.x, lo.y, hi.x, hi.y};
+        }
+        a.bs = mk_ld_act(ab + 260 + 16 * kh);
         a.d = *(const float *)ab;
     }
     static __device__ __forceinline__ void mul(const W &w, const MkAct &a, int kh, mk_v16f &acc) {
@@ -427,11 +436,11 @@ __global__ __launch_bounds__(64 * MMK_NW) void k_mmk_tile(g4h_tensor W, const ui
     mk_v4i a[MT][8], bs[MT];
     float d[MT];
     auto load_a = [&](int m, int j, int s) __attribute__((always_inline)) {
-        a[m][j] = mk_ld(ab[m] + (size_t)s * TL[m] * 292 + 2 * j * TL[m] * 16 + ao[m]);
+        a[m][j] = mk_ld_act(ab[m] + (size_t)s * TL[m] * 292 + 2 * j * TL[m] * 16 + ao[m]);
     };
     auto load_s = [&](int m, int s) __attribute__((always_inline)) {
         const uint8_t *b = ab[m] + (size_t)s * TL[m] * 292;
-        if constexpr (S::T == Q4_K) bs[m] = mk_ld(b + TL[m] * 256 + ao[m]);
+        if constexpr (S::T == Q4_K) bs[m] = mk_ld_act(b + TL[m] * 256 + ao[m]);
         d[m] = *(const float *)(b + TL[m] * 288 + 4 * tl[m]);
     };
     mk_v16f acc[MT];

@@ -75,7 +75,8 @@ __global__ __launch_bounds__(256) void k_quantize_q8_K(const float *__restrict__
 // one TL = rows % 32 wide), per superblock sixteen 16-byte chunks [2 g + kh][TL]
 // -- the lane half kh's quants of the 32-element group g -- then with BS the 16
 // bsums as fp16 [kh][TL][8] (exact: |bsum| <= 2048; without them the place stays
-// unused) and d [TL].  LAY 0: kh holds elements 16 kh .. + 15 of group g; 1: 8 kh
+// unused) and d [TL]; a tile of 32 has its chunks 64-byte aligned, the last one
+// 4-byte aligned.  LAY 0: kh holds elements 16 kh .. + 15 of group g; 1: 8 kh
 // .. + 7 and 16 + 8 kh .. + 7 (q6_K's sub-blocks of 16); 2 (k_mmg's units of
 // 16-byte quant runs): g = 2 (2 h + k) + f, and kh holds elements 128 h + 32 j +
 // 16 k + 8 kh .. + 7 of j = 2 f and 2 f + 1.  Consecutive waves take consecutive
