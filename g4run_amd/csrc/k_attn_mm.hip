@@ -18,7 +18,8 @@
 //            one v_mfma_f32_32x32x16_f16 per 16 head elements (exact
 //            products, fp32 sums); per row and chunk the maximum m_c and
 //            l_c = sum expf(s - m_c) over the row's positions, summed in
-//            double.
+//            double: 16 per lane in order, the two lanes of a row, then the
+//            waves in order.
 //   values   grid KV head x 256-position span x tile: per row the global
 //            maximum M and normaliser (sum_c l_c exp(m_c - M) in double) as in
 //            the decode kernels, the weights fp16(expf(s - M) * inv)
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(256) void k_amm_scores(AmmArgs c) {
     }
     m = fmaxf(m, partner<32>(m));
     if (kh == 0) wm[wave][li] = m;
-    if (row) {                                                       // positions outside a row's own are never read
+    if (row) {                                                       // whole chunks; k_amm_v gives positions outside a row's own weight 0
         float *Sr = c.S + R * c.nch * AMM_CH + jw + 4 * kh;
 #pragma unroll
         for (int q = 0; q < 4; q++) *(float4 *)(Sr + 8 * q) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
@@ -238,10 +239,12 @@ __global__ __launch_bounds__(256) void k_amm_scores(AmmArgs c) {
 
 // Values: 8 waves, each with 4 of the tile's rows for the weights and one of up
 // to 8 units of 32 columns for the sums (heads of 512 take two workgroups, grid
-// y).  Every load goes out at the start -- chunk statistics, scores 16 bytes
-// per lane, V rows in runs of adjacent bytes, 28 loads in all (a wave tracks 63;
-// V loaded as 128 words per lane took 4.3 us to issue), the second half of V
-// once the statistics are done -- so the phases wait on one round trip.  A
+// y).  Chunk statistics, scores (16 bytes per lane) and half of the V rows (in
+// runs of adjacent bytes) are loaded at the start, 20 loads in all (V as 128
+// words per lane took 4.3 us to issue); the other half of V goes out once the
+// statistics' registers are free and is in flight while the weights are formed.
+// Scores of a chunk past the call's last one are not loaded; scores that a
+// loaded chunk holds outside a row's positions are dropped.  A
 // row's statistics and weights are one wave's, handed over in registers; V
 // passes through LDS of the wave's own 64 positions at a time and is read there
 // transposed (ds_read_b64_tr_b16).  48 KB of LDS and 128 registers: two

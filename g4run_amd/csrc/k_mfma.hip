@@ -383,7 +383,8 @@ __global__ __launch_bounds__(64 * TM * TN, 2) void k_mm_lds(g4h_tensor W, const 
 // wave's own, and, for rows of whole 8-block groups (SV), so are the scales of
 // four pair steps at a time (other rows load a 2-byte scale per lane): about
 // 110 accesses per step.  A wave keeps the loads of FEW_AHEAD pair steps in
-// flight: step k + FEW_AHEAD's loads go out before step k multiplies.
+// flight, one less with four token tiles: step k + 4's (k + 3's) loads go out
+// before step k multiplies.
 // One v_permlane32_swap per dword pair turns the operand's halves into those
 // of the two blocks' int8 MFMAs (lane group g then holds slice sigma(g) of the
 // block: (0, 2, 1, 3) for q8_0, g for q4_0), and the activations are laid out
@@ -421,7 +422,7 @@ size_t mm_few_bytes(int M, int64_t ncols) {
 
 // The pair steps run as straight-line chunks of FEW_CHUNK steps (then one
 // chunk each of 8, 4, 2, 1 for the rest, so no step is wasted), FEW_AHEAD
-// steps of loads in flight (MT + 3 loads per step, within the 63 the memory
+// steps of loads in flight (at most MT + 3 loads per step, within the 63 the memory
 // counter tracks).  Straight-line code keeps the compiler's memory-counter
 // waits exact: a register ring carried around a loop is undone (InstCombine
 // folds the phi of loads into one load at the loop head, buffer loads sink to
@@ -437,8 +438,9 @@ size_t mm_few_bytes(int M, int64_t ncols) {
 // operands straight from memory (same calls, us): q8_0 4096x4096 at 16 / 64
 // tokens 10.7 / 14.6 -> 9.2 / 13.6; q4_0 20480x2560 at 16 / 32 / 64 tokens 22.5
 // / 26.1 / 32.4 -> 15.8 / 18.6 / 24.9; q4_0 2560x10240 19.2 (16) / 27.7 (64) ->
-// 13.8 / 22.4.  At 64 tokens the VALU issue of the epilogues (10.5 us) and the
-// matrix cores (5.3 us) bound the q4_0 20480x2560 call next.
+// 13.8 / 22.4.  At 64 tokens the q4_0 20480x2560 call needs 10.5 us of VALU issue
+// for the epilogues and 5.3 us of the matrix cores (counted from the
+// instructions), at three waves per SIMD.
 constexpr int FEW_CHUNK = 16, FEW_AHEAD = 4;
 
 template <int WT, int MT, bool SV>

@@ -31,7 +31,9 @@
 // 18.8 / 125, tq2_0 24.2 / 147 / 1149 -> 12.4 / 15.0 / 94.5 (486 TOPS).  What
 // bounds it at 509 tokens: the VALU, with four units' conversions and fmas per
 // superblock and output (the GEMV's roundings) and the scale products, at two
-// waves per SIMD (four accumulator tiles, 165 to 256 registers).
+// waves per SIMD (four accumulator tiles, 165 to 256 registers; q5_K's form of
+// 16 classes spills 4 of them, 20 bytes of scratch, and its form of 4 classes
+// takes 276, one wave per SIMD).
 #include <algorithm>
 #include <cstdio>
 

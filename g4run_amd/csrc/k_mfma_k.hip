@@ -297,7 +297,7 @@ __global__ __launch_bounds__(64 * MMK_NW) void k_mmk(g4h_tensor W, const uint8_t
 // (us, k_mmk / this): q4_K at 9 / 64 / 128 / 509 tokens 20.4 / 25.8 / 45.4 /
 // 165 -> 15.8 / 18.3 / 25.1 / 82.8 (554 TOPS); q6_K at 9 / 64 / 509 tokens 30.3
 // / 38.5 / 250 -> 21.6 / 23.2 / 112; q6_K 2048 x 6144 at 64 26.9 -> 14.3.  What
-// bounds it at 509 tokens: 1.0 GB of operands from L2 and 45 us of VALU issue
+// bounds it at 509 tokens: 1.0 GB of operands from L2 and 38 us of VALU issue
 // (the scale multiply-adds), partly overlapped.
 // The waves split the superblocks as k_mmk's do, each superblock's integers
 // and scale products are the same, and the partial tiles are added in the same

@@ -17,7 +17,8 @@
 // Stages, in the reference's order, with its arithmetic:
 //   bans -> -inf, no-repeat-ngram hits -> -inf           (sampler.c:78-101)
 //   repeat / frequency / presence penalties, each distinct id of the window
-//   once; the window is sorted in LDS so a run gives the count (104-137)
+//   once; its entries are counted from the window sorted in LDS (small rows) or
+//   by id (large rows)                                      (104-137)
 //   greedy: first index of the maximum                     (140-144)
 //   top-k (k = top_k in 1..511, else 512, at most n_vocab)  (147-176)
 //   top-p over the fp32 softmax, double sums               (179-194)
@@ -29,12 +30,13 @@
 // its result is fixed by the values alone: the k largest, in descending order.
 // The fast path finds them with a 16-ary search over the order-preserving
 // 32-bit keys for a threshold with between k+1 and 1024 elements at or above
-// it (the row held in registers when it has at most 32 values per thread,
-// else read in batches of 8 per thread), gathers those, bitonic-sorts them one
+// it (small rows are held in registers, at most 16 values per thread; large
+// ones are searched by their group maxima, and read in batches of 8 per thread
+// only where those don't settle it), gathers those, bitonic-sorts them one
 // per thread (lane shuffles within a wave, LDS across waves) and checks the
 // condition.
-// Otherwise (ties, NaN, or more than 4096 elements sharing the boundary key)
-// wave 0 replays the reference's heap exactly, skipping 64 ids at a time
+// Otherwise (ties, NaN, or more than 1024 elements sharing the boundary key)
+// wave 0 replays the reference's heap exactly, skipping 1024 or 64 ids at a time
 // whose values cannot enter it, and the heap array is ordered as the
 // insertion sort orders it (a stable sort by value; the literal insertion
 // sort when NaNs are present).

@@ -140,7 +140,9 @@ int    g4h_tensor_info(const g4h_tensor *t, int *type, int64_t *ncols, int64_t *
 int g4h_matmul(const g4h_tensor *W, const float *x_dev, const void *pre_dev, size_t pre_stride,
                float *Y_dev, int nb, void *stream);
 /* Same with an explicit kernel family: 0 = auto (g4h_matmul_path), 1 = the
- * GEMV family (token chunks of <= 8 staged per workgroup), 2 = matrix-core
+ * GEMV family (token chunks of <= 8 staged per workgroup; from 9 fp32 tokens
+ * q5_K / q3_K / q2_K / tq2_0 weights run on the matrix cores in the GEMV's
+ * order of sums, with its bits), 2 = matrix-core
  * tiles: int8 for q8_0 / q4_0 / q4_K / q6_K weights (every per-block or
  * per-superblock integer sum exact, fp32 scaling in a fixed order), f16 / bf16
  * for f16 / bf16 rows of whole 16-column steps (exact products, fp32 sums);
@@ -164,7 +166,8 @@ int    g4h_matmul_noalloc(const g4h_tensor *W, const float *x_dev, const void *p
                           float *Y_dev, int nb, int path, void *stream);
 size_t g4h_matmul_noalloc_max_bytes(void);
 /* Diagnostic (no reference counterpart): the kernel instantiation and launch
- * shape g4h_matmul_ex would use, e.g. "k_gemv<q4_0,nb=1,lpr=32,upl=4> grid=256
+ * shape g4h_matmul_ex would use for nb fp32 tokens (where pre_dev rows take
+ * another kernel or tile, the end of the text names it), e.g. "k_gemv<q4_0,nb=1,lpr=32,upl=4> grid=256
  * block=512", written NUL-terminated into buf (at most len bytes).  Profiles
  * and benchmarks name the kernel they time with it. */
 int g4h_matmul_describe(const g4h_tensor *W, int nb, int path, char *buf, size_t len);
