@@ -237,48 +237,49 @@ __global__ __launch_bounds__(256) void k_amm_scores(AmmArgs c) {
     }
 }
 
-// Values: 8 waves, each with 4 of the tile's rows for the weights and one of up
-// to 8 units of 32 columns for the sums (heads of 512 take two workgroups, grid
-// y).  Chunk statistics, scores (16 bytes per lane) and half of the V rows (in
-// runs of adjacent bytes) are loaded at the start, 20 loads in all (V as 128
-// words per lane took 4.3 us to issue); the other half of V goes out once the
-// statistics' registers are free and is in flight while the weights are formed.
-// Scores of a chunk past the call's last one are not loaded; scores that a
-// loaded chunk holds outside a row's positions are dropped.  A
+// Values: 8 or 16 waves (NW), each with 4 or 2 of the tile's rows for the weights
+// and one unit of 32 columns for the sums (heads of 512 with 8 waves take two
+// workgroups, grid y).  Chunk statistics, scores (16 bytes per lane) and half of
+// the V rows (in runs of adjacent bytes) are loaded at the start, 20 loads in all
+// with 8 waves (V as 128 words per lane took 4.3 us to issue); the other half of
+// V goes out once the statistics' registers are free and is in flight while the
+// weights are formed.  Scores of a chunk past the call's last one are not loaded;
+// scores that a loaded chunk holds outside a row's positions are dropped.  A
 // row's statistics and weights are one wave's, handed over in registers; V
 // passes through LDS of the wave's own 64 positions at a time and is read there
-// transposed (ds_read_b64_tr_b16).  48 KB of LDS and 128 registers: two
-// workgroups per CU.  64 tokens after 4096 positions, 8 q /
-// 4 kv heads of 256: 20.8 -> 15.6 us.
+// transposed (ds_read_b64_tr_b16).  48 or 80 KB of LDS and 128 registers: 16
+// waves per CU.  64 tokens after 4096 positions, 8 q / 4 kv heads of 256: 20.8 ->
+// 15.6 us.
 typedef short am_v4s __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) am_v4s *am_lds4;
 
-template <int HD, int GRP>
-__global__ __launch_bounds__(512, 4) void k_amm_v(AmmArgs c) {
-    constexpr int NU = HD < 256 ? HD / 32 : 8, ST = AMM_NP / 16, VP = 4, HP = AMM_NP / VP;   // column units, steps, V parts and their positions
+template <int HD, int GRP, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void k_amm_v(AmmArgs c) {
+    constexpr int RW = 32 / NW, NU = HD < 32 * NW ? HD / 32 : NW;   // rows per wave, waves with a column unit
+    constexpr int ST = AMM_NP / 16, VP = 4, HP = AMM_NP / VP;       // steps, V parts and their positions
     // fp16 weights of the span, the 16-byte units of row r at unit ^ (r & 7)
     __shared__ __align__(16) uint8_t wsh[32 * AMM_NP * 2];
-    __shared__ __align__(16) uint8_t vsh[8][HP * 64];               // a wave's part of V: rows of 32 columns
+    __shared__ __align__(16) uint8_t vsh[NW][HP * 64];              // a wave's part of V: rows of 32 columns
     amm_view(c);
     int kvh, tt, cv;
     if (!amm_block(c, blockIdx.x, AMM_NP, kvh, cv, tt)) return;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t) >> 6, li = lane & 31, kh = lane >> 5;
-    const int jl0 = cv * AMM_NP, unit = wave + 8 * blockIdx.y;
+    const int jl0 = cv * AMM_NP, unit = wave + NW * blockIdx.y;
     const int jfirst = c.window ? max(0, c.p0 + 1 - c.window) : 0, jlast = c.jb + c.span - 1;
     // 1. per row the global maximum and normaliser over the row's own chunks
-    // (wave w: rows 4 w .. 4 w + 3; lane k: the row's k-th chunk, 64 per round)
+    // (wave w: rows RW w .. RW w + RW - 1; lane k: the row's k-th chunk, 64 per round)
     const int nca = (c.span + AMM_CH - 1) / AMM_CH;                  // >= any row's chunk count
-    int nrc[4], j0r[4], pr[4];
-    size_t base[4];
-    bool rv[4], on[4];
-    float mcv[4];
-    double lcv[4];
-    float4 sv[4];                                                    // the scores of positions 4 lane .. + 3
+    int nrc[RW], j0r[RW], pr[RW];
+    size_t base[RW];
+    bool rv[RW], on[RW];
+    float mcv[RW];
+    double lcv[RW];
+    float4 sv[RW];                                                   // the scores of positions 4 lane .. + 3
     const int jt = jl0 + 4 * lane, jg = c.jb + jt;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < RW; k++) {
         int b, h;
-        amm_rowinfo<GRP>(c, kvh, tt, wave * 4 + k, b, h, j0r[k], pr[k]);
+        amm_rowinfo<GRP>(c, kvh, tt, wave * RW + k, b, h, j0r[k], pr[k]);
         rv[k] = b < c.nb;
         const int clo = rv[k] ? (j0r[k] - c.jb) / AMM_CH : 0;
         nrc[k] = rv[k] ? (pr[k] - c.jb) / AMM_CH - clo + 1 : 0;
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(512, 4) void k_amm_v(AmmArgs c) {
         lcv[k] = on[k] ? c.Lc[base[k] + lane] : 0.0;
     }
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < RW; k++) {
         // whole chunks of scores are stored for the tile's rows; a span's second
         // chunk may lie past the last one
         const bool in = rv[k] && jt < c.nch * AMM_CH;
@@ -311,27 +312,27 @@ __global__ __launch_bounds__(512, 4) void k_amm_v(AmmArgs c) {
         for (int q = 0; q < ST / 2; q++) load_v(q);
     }
     asm volatile("" ::: "memory");
-    float m[4], inv[4];
+    float m[RW], inv[RW];
     {
-        double sum[4];
+        double sum[RW];
 #pragma unroll
-        for (int k = 0; k < 4; k++) m[k] = group_max<64>(mcv[k]);
+        for (int k = 0; k < RW; k++) m[k] = group_max<64>(mcv[k]);
         for (int c1 = 64; c1 < nca; c1 += 64)
 #pragma unroll
-            for (int k = 0; k < 4; k++) m[k] = fmaxf(m[k], group_max<64>(c1 + lane < nrc[k] ? c.Mc[base[k] + c1 + lane] : -INFINITY));
+            for (int k = 0; k < RW; k++) m[k] = fmaxf(m[k], group_max<64>(c1 + lane < nrc[k] ? c.Mc[base[k] + c1 + lane] : -INFINITY));
 #pragma unroll
-        for (int k = 0; k < 4; k++)                                  // rows outside the batch (uniform) skip the exp
+        for (int k = 0; k < RW; k++)                                 // rows outside the batch (uniform) skip the exp
             sum[k] = rv[k] ? group_sum_t<64>(on[k] ? lcv[k] * exp((double)mcv[k] - (double)m[k]) : 0.0) : 1.0;
         for (int c1 = 64; c1 < nca; c1 += 64)
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
+            for (int k = 0; k < RW; k++) {
                 const bool o = c1 + lane < nrc[k];
                 const float mc = o ? c.Mc[base[k] + c1 + lane] : 0.0f;
                 const double lc = o ? c.Lc[base[k] + c1 + lane] : 0.0;
                 sum[k] += group_sum_t<64>(o ? lc * exp((double)mc - (double)m[k]) : 0.0);
             }
 #pragma unroll
-        for (int k = 0; k < 4; k++) inv[k] = (float)(1.0 / sum[k]);
+        for (int k = 0; k < RW; k++) inv[k] = (float)(1.0 / sum[k]);
     }
     asm volatile("" ::: "memory");
     if (wave < NU) {                                                 // the second half, the statistics' registers free
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(512, 4) void k_amm_v(AmmArgs c) {
     asm volatile("" ::: "memory");
     // 2. the weights (0 outside a row's positions)
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < RW; k++) {
         uint2 w = make_uint2(0, 0);
         if (rv[k]) {                                                 // uniform
             const float e[4] = {sv[k].x, sv[k].y, sv[k].z, sv[k].w};
@@ -353,7 +354,7 @@ __global__ __launch_bounds__(512, 4) void k_amm_v(AmmArgs c) {
             }
             w = make_uint2(hw[0] | (hw[1] << 16), hw[2] | (hw[3] << 16));
         }
-        const int r = wave * 4 + k;
+        const int r = wave * RW + k;
         *(uint2 *)(wsh + r * (AMM_NP * 2) + 16 * ((lane >> 1) ^ (r & 7)) + 8 * (lane & 1)) = w;
     }
     lds_barrier();
@@ -443,7 +444,13 @@ bool attn_batch_mm_ok(const QkvArgs &a) {
 template <int HD, int GRP>
 static void amm_go(const AmmArgs &c, hipStream_t s) {
     hipLaunchKernelGGL((k_amm_scores<HD, GRP>), dim3((unsigned)amm_blocks(c, c.nch)), dim3(256), 0, s, c);
-    hipLaunchKernelGGL((k_amm_v<HD, GRP>), dim3((unsigned)amm_blocks(c, c.nchv), HD == 512 ? 2 : 1), dim3(512), 0, s, c);
+    // heads of 512, 16 column units: two workgroups of 8 waves, or from 320 blocks
+    // one of 16, which forms the weights once (us a call, 8 q / 1 kv heads, two / one:
+    // one token at position 1000 16.5 / 17.3, 64 tokens at 4096 44.4 / 45.5, at 8192
+    // 74.9 / 71.3, 256 at 16000 502 / 454; the per-tile launch before both 478)
+    const unsigned blocks = (unsigned)amm_blocks(c, c.nchv);
+    if (HD == 512 && blocks >= 320) hipLaunchKernelGGL((k_amm_v<HD, GRP, HD == 512 ? 16 : 8>), dim3(blocks), dim3(1024), 0, s, c);
+    else hipLaunchKernelGGL((k_amm_v<HD, GRP, 8>), dim3(blocks, HD == 512 ? 2 : 1), dim3(512), 0, s, c);
     hipLaunchKernelGGL(k_amm_combine<HD>, dim3(c.n_head, c.nb), dim3(256), 0, s, c);
 }
 
@@ -483,7 +490,7 @@ hipError_t launch_attn_batch_mm(const float *q, const QkvArgs &a, int npos0, int
     const int grp = a.n_head / a.n_kv;
     c.ntt = (nb + 32 / grp - 1) / (32 / grp);
     const AmmWs w = amm_ws(a.n_head, a.hd, nb, span);
-    if (ws_bytes < w.total || amm_blocks(c, c.nch) > max_grid(256) || amm_blocks(c, c.nchv) > max_grid(512)) return hipErrorInvalidValue;
+    if (ws_bytes < w.total || amm_blocks(c, c.nch) > max_grid(256) || amm_blocks(c, c.nchv) > max_grid(a.hd == 512 ? 1024 : 512)) return hipErrorInvalidValue;
     c.S = (float *)(ws + w.S);
     c.Mc = (float *)(ws + w.Mc);
     c.Lc = (double *)(ws + w.Lc);

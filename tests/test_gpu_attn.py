@@ -576,9 +576,11 @@ def test_prefill_matrix_cores_errors(gpu):
 
 # position blocks x token tiles dealt to the 8 XCDs: fewer than 8 blocks, whole
 # and broken eighths, and calls of 4096 tiles and more (whole rounds of blocks
-# and a rest: scores at the first such case, values too at the second)
+# and a rest: scores at the first such case, values too at the second); heads of
+# 512 from 320 value blocks, where one workgroup takes all columns
 @pytest.mark.parametrize("n_kv,grp,hd,pos0,nb", [(1, 8, 512, 0, 256), (1, 8, 256, 0, 9), (3, 2, 64, 1000, 33), (1, 1, 128, 1030, 70),
-                                                 (4, 8, 64, 1900, 250), (4, 8, 64, 4000, 256)])
+                                                 (4, 8, 64, 1900, 250), (4, 8, 64, 4000, 256),
+                                                 (1, 8, 512, 1000, 256), (1, 2, 512, 2900, 900)])
 def test_prefill_matrix_cores_blocks_and_tiles(gpu, n_kv, grp, hd, pos0, nb):
     """Every (block, tile) pair is taken once: the rows equal those of the same
     tokens in batches of up to 7."""
