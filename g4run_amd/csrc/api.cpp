@@ -473,7 +473,7 @@ extern "C" int g4h_matmul_describe(const g4h_tensor *W, int nb, int path, char *
     if (path == 2) {
         if (!mfma_capable(W)) return fail(G4H_ERR_TYPE, "g4h_matmul_describe: the matrix-core path takes q8_0 / q4_0 / q4_K / q6_K weights and f16 / bf16 rows of whole 16-column steps");
         if (mmk_capable(W->type)) mmk_describe(*W, nb, buf, len);
-        else if (is_float(W->type)) mmf_describe(W->type, W->nrows, nb, buf, len);
+        else if (is_float(W->type)) mmf_describe(W->type, W->nrows, W->ncols, nb, buf, len);
         else mm_describe(*W, nb, buf, len);
         return G4H_OK;
     }

@@ -192,7 +192,8 @@ __device__ __forceinline__ uint32_t mmf_round2(uint32_t x, uint32_t y) {
 
 // ONE: rows of one chunk (up to 256 columns), which is loaded once and takes one
 // buffer; the loop's loads ahead would all be of the last piece again (us, loop /
-// this: f16 65536 x 256 at 9 / 17 / 80 tokens 14.5 / 16.4 / 40.3 -> 8.1 / 10.3 / 37.3).
+// this, the same tiles: f16 65536 x 256 at 9 / 17 / 80 tokens 14.5 / 16.4 / 40.3 ->
+// 8.1 / 10.3 / 37.3).
 // A32: activation rows of fp32 (row stride `as` bytes), rounded on the way to
 // LDS; else f16 rows.  Workgroup b runs on XCD b % 8: the token tiles of one
 // row tile go to one XCD, consecutively, and find its weights in that XCD's L2.
@@ -339,11 +340,16 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
 // 25.3; at 200 tokens 64 x 64 26.4, 64 x 32 38.5; 10240 x 4096 at 9 tokens 16 x 64
 // 18.3, 16 x 32 23.7.  Past one 16 x 64 workgroup per CU, 16 x 32 keeps more loads in
 // flight instead: 20480 x 1040 at 9 tokens 16.1 / 12.3, 65536 x 1040 37.3 / 29.6.
-// Shapes that this never finds best are not built (fp32: fewer rows than tokens).
-static void mmf_tiles(bool a32, int64_t nrows, int M, int &mr, int &nr, int &ntok, int64_t &grid) {
+// Rows of one chunk wait for one round trip and the sums' LDS pass, so small
+// workgroups, many per CU, are best: at most 32 x 32 (f16 20480 x 256 at 48 tokens
+// 64 x 64 10.0, 32 x 32 7.0; 65536 x 256 at 80 37.4 / 19.7).
+// Shapes that this never finds best are not built (fp32: fewer rows than tokens;
+// one chunk: past 32 x 32).
+static void mmf_tiles(bool a32, int64_t nrows, int64_t ncols, int M, int &mr, int &nr, int &ntok, int64_t &grid) {
+    const int most = ncols <= MMF_KC ? 32 : 64;
     int64_t best = INT64_MAX;
-    for (int m = M > 32 ? 64 : M > 16 ? 32 : 16; m >= 16; m >>= 1)
-        for (int n = 64; n >= (a32 ? m : std::max(16, m / 2)); n >>= 1) {
+    for (int m = M > 32 ? most : M > 16 ? 32 : 16; m >= 16; m >>= 1)
+        for (int n = most; n >= (a32 ? m : std::max(16, m / 2)); n >>= 1) {
             if (m == 16 && n == 64 && nrows > 256 * 64) continue;   // 16 x 32 above
             const int64_t cost = ((M + m - 1) / m * ((nrows + n - 1) / n) + 255) / 256 * ((a32 ? 2 : 1) * m + n);
             if (cost < best) best = cost, mr = m, nr = n;
@@ -354,11 +360,11 @@ static void mmf_tiles(bool a32, int64_t nrows, int M, int &mr, int &nr, int &nto
 // token tiles of one launch (all of them, but for outputs of 2^33 values and more)
 static int mmf_tok(int64_t grid, int ntok) { return (int)std::min<int64_t>(ntok, max_grid(64 * MMF_W) / (grid / ntok)); }
 
-void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len) {
+void mmf_describe(int wtype, int64_t nrows, int64_t ncols, int M, char *buf, size_t len) {
     int mr, nr, ntok, pm, pn;
     int64_t grid, pgrid;
-    mmf_tiles(wtype != F16, nrows, M, pm, pn, ntok, pgrid);
-    mmf_tiles(true, nrows, M, mr, nr, ntok, grid);
+    mmf_tiles(wtype != F16, nrows, ncols, M, pm, pn, ntok, pgrid);
+    mmf_tiles(true, nrows, ncols, M, mr, nr, ntok, grid);
     const int nt = mmf_tok(grid, ntok);
     snprintf(buf, len, "k_mm_float<%s,%dx%d> grid=%lld block=%d (x%d launches; matrix cores, %d waves split the columns; given rows %dx%d)",
              wtype == F16 ? "f16" : "bf16", mr, nr, (long long)(grid / ntok * nt), 64 * MMF_W, nt ? (ntok + nt - 1) / nt : 0, MMF_W, pm, pn);
@@ -367,8 +373,10 @@ void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len) {
 template <int WT, bool A32, int MR, int NR>
 static void mmf_run(dim3 g, const uint8_t *W, size_t ws, int64_t nrows, int64_t ncols, const uint8_t *a, size_t ab, int M, float *Y, int ntok,
                     hipStream_t s) {
-    if (ncols <= MMF_KC) hipLaunchKernelGGL((k_mm_float<WT, A32, true, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
-    else hipLaunchKernelGGL((k_mm_float<WT, A32, false, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
+    if (ncols <= MMF_KC) {
+        if constexpr (MR <= 32 && NR <= 32)
+            hipLaunchKernelGGL((k_mm_float<WT, A32, true, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
+    } else hipLaunchKernelGGL((k_mm_float<WT, A32, false, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
 }
 
 template <int WT, bool A32>
@@ -376,7 +384,7 @@ static hipError_t mmf_go(const uint8_t *W, size_t ws, int64_t nrows, int64_t nco
                          hipStream_t s) {
     int mr, nr, ntok;
     int64_t grid;
-    mmf_tiles(A32, nrows, M, mr, nr, ntok, grid);
+    mmf_tiles(A32, nrows, ncols, M, mr, nr, ntok, grid);
     const int nt = mmf_tok(grid, ntok);
     if (nt < 1 || ncols >= MMF_MAX_COLS) return hipErrorInvalidValue;
     for (int64_t m0 = 0; m0 < M; m0 += (int64_t)nt * mr) {          // one launch as a rule

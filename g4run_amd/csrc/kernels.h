@@ -246,7 +246,7 @@ hipError_t launch_mm_few_ready(const g4h_tensor &W, const FewAct &a, int M, floa
 // weights against GGUF q8_K activation rows at `stride` bytes
 bool mmk_capable(int type);
 void mmk_describe(const g4h_tensor &W, int M, char *buf, size_t len);
-void mmf_describe(int wtype, int64_t nrows, int M, char *buf, size_t len);
+void mmf_describe(int wtype, int64_t nrows, int64_t ncols, int M, char *buf, size_t len);
 // workgroups of one launch: HIP takes gridDim * blockDim below 2^32
 inline int64_t max_grid(int threads) { return 0xffffffffll / threads; }
 // columns of k_mm_float (32-bit byte offsets within a row); longer f16 / bf16 rows
