@@ -444,7 +444,7 @@ static bool x_fused(const g4h_tensor &W, int nb) {
 
 // f16 / bf16 rows need whole 16-column steps (k_mm_float)
 static bool mfma_capable(const g4h_tensor *W) {
-    return W && (W->type == Q8_0 || W->type == Q4_0 || mmk_capable(W->type) || (is_float(W->type) && W->ncols % 16 == 0 && W->ncols < MMF_MAX_COLS));
+    return W && (W->type == Q8_0 || W->type == Q4_0 || mmk_capable(W->type) || (is_float(W->type) && W->ncols % 16 == 0));
 }
 
 extern "C" int g4h_matmul_path(const g4h_tensor *W, int nb) {

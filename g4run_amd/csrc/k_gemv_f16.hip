@@ -9,7 +9,9 @@
 // lanes.  The fp32 order differs from the CPU's 8-lane AVX2 order (within the
 // path's fp32 tolerance) but does not depend on the token count, so a batch
 // gives every token the single-token bits.
+#include <algorithm>
 #include <cstdio>
+#include <type_traits>
 
 #include "common.h"
 #include "kernels.h"
@@ -176,6 +178,9 @@ typedef uint32_t mf_v4u __attribute__((ext_vector_type(4)));
 
 constexpr int MMF_W = 8;              // waves per workgroup
 constexpr int MMF_KC = 256;           // columns per chunk: two steps per wave
+// rows of many chunks, of one, and past 32-bit byte offsets (16 x 16 tiles only)
+enum { MMF_LOOP, MMF_ONE, MMF_LONG };
+static bool mmf_long(int64_t ncols) { return ncols >= (int64_t)1 << 29; }
 
 // two fp32 activations rounded with k_act_float's arithmetic by the packed
 // conversion instructions (round to nearest even; bf16-rounded rows keep their
@@ -190,14 +195,14 @@ __device__ __forceinline__ uint32_t mmf_round2(uint32_t x, uint32_t y) {
     else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2bf));
 }
 
-// ONE: rows of one chunk (up to 256 columns), which is loaded once and takes one
-// buffer; the loop's loads ahead would all be of the last piece again (us, loop /
+// FORM MMF_ONE: rows of one chunk (up to 256 columns), which is loaded once and takes
+// one buffer; the loop's loads ahead would all be of the last piece again (us, loop /
 // this, the same tiles: f16 65536 x 256 at 9 / 17 / 80 tokens 14.5 / 16.4 / 40.3 ->
 // 8.1 / 10.3 / 37.3).
 // A32: activation rows of fp32 (row stride `as` bytes), rounded on the way to
 // LDS; else f16 rows.  Workgroup b runs on XCD b % 8: the token tiles of one
 // row tile go to one XCD, consecutively, and find its weights in that XCD's L2.
-template <int WT, bool A32, bool ONE, int MR, int NR>
+template <int WT, bool A32, int FORM, int MR, int NR>
 __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restrict__ W, size_t ws, int64_t nrows, int64_t ncols,
                                                          const uint8_t *__restrict__ act, size_t as, int M, float *__restrict__ Y,
                                                          int ntok) {
@@ -205,6 +210,7 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
     constexpr int AU = A32 ? 64 : 32, AL = MR * AU / NTH, WL = NR * 32 / NTH;   // 16-byte pieces per row, loads per thread
     static_assert(MR * AU % NTH == 0 && NR * 32 % NTH == 0, "whole loads");
     constexpr int BUF = (MR + NR) * RB, PART = MMF_W * MT * NT * 4096;
+    constexpr bool ONE = FORM == MMF_ONE;
     constexpr int STAGED = ONE ? BUF : 2 * BUF;
     __shared__ __align__(16) uint8_t lds[STAGED > PART ? STAGED : PART];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t) >> 6;
@@ -221,7 +227,8 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
 #pragma unroll
     for (int q = 0; q < AL; q++) ap[q] = act + (size_t)min(m0 + AQ * q + ar, M - 1) * as;
     const int ns = (int)(ncols >> 4), nc = (ns + 15) >> 4;          // steps, chunks
-    const uint32_t wlast = (uint32_t)ncols * 2 - 16, alast = (uint32_t)ncols * (A32 ? 4 : 2) - 16;
+    using Off = std::conditional_t<FORM == MMF_LONG, uint64_t, uint32_t>;
+    const Off wlast = (Off)ncols * 2 - 16, alast = (Off)ncols * (A32 ? 4 : 2) - 16;
     struct Stage {
         mf_v4u w[WL], a[AL];
     };
@@ -230,7 +237,7 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
     constexpr int D = ONE || AL + WL >= 12 ? 1 : AL + WL >= 8 ? 2 : 4;
     Stage st[D];
     auto load = [&](Stage &S, int c) __attribute__((always_inline)) {   // past the row's end its last piece again, never used
-        const uint32_t wo = min((uint32_t)c * RB + 16 * wc, wlast), ao = min((uint32_t)c * (A32 ? 2 * RB : RB) + 16 * ac, alast);
+        const Off wo = std::min((Off)c * RB + 16 * wc, wlast), ao = std::min((Off)c * (A32 ? 2 * RB : RB) + 16 * ac, alast);
 #pragma unroll
         for (int q = 0; q < WL; q++) S.w[q] = *(const mf_v4u *)(wp[q] + wo);
 #pragma unroll
@@ -346,9 +353,9 @@ __global__ __launch_bounds__(64 * MMF_W) void k_mm_float(const uint8_t *__restri
 // Shapes that this never finds best are not built (fp32: fewer rows than tokens;
 // one chunk: past 32 x 32).
 static void mmf_tiles(bool a32, int64_t nrows, int64_t ncols, int M, int &mr, int &nr, int &ntok, int64_t &grid) {
-    const int most = ncols <= MMF_KC ? 32 : 64;
+    const int most = mmf_long(ncols) ? 16 : ncols <= MMF_KC ? 32 : 64;
     int64_t best = INT64_MAX;
-    for (int m = M > 32 ? most : M > 16 ? 32 : 16; m >= 16; m >>= 1)
+    for (int m = std::min(most, M > 32 ? 64 : M > 16 ? 32 : 16); m >= 16; m >>= 1)
         for (int n = most; n >= (a32 ? m : std::max(16, m / 2)); n >>= 1) {
             if (m == 16 && n == 64 && nrows > 256 * 64) continue;   // 16 x 32 above
             const int64_t cost = ((M + m - 1) / m * ((nrows + n - 1) / n) + 255) / 256 * ((a32 ? 2 : 1) * m + n);
@@ -375,8 +382,11 @@ static void mmf_run(dim3 g, const uint8_t *W, size_t ws, int64_t nrows, int64_t 
                     hipStream_t s) {
     if (ncols <= MMF_KC) {
         if constexpr (MR <= 32 && NR <= 32)
-            hipLaunchKernelGGL((k_mm_float<WT, A32, true, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
-    } else hipLaunchKernelGGL((k_mm_float<WT, A32, false, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
+            hipLaunchKernelGGL((k_mm_float<WT, A32, MMF_ONE, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
+    } else if (mmf_long(ncols)) {
+        if constexpr (MR == 16 && NR == 16)
+            hipLaunchKernelGGL((k_mm_float<WT, A32, MMF_LONG, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
+    } else hipLaunchKernelGGL((k_mm_float<WT, A32, MMF_LOOP, MR, NR>), g, dim3(64 * MMF_W), 0, s, W, ws, nrows, ncols, a, ab, M, Y, ntok);
 }
 
 template <int WT, bool A32>
@@ -386,7 +396,7 @@ static hipError_t mmf_go(const uint8_t *W, size_t ws, int64_t nrows, int64_t nco
     int64_t grid;
     mmf_tiles(A32, nrows, ncols, M, mr, nr, ntok, grid);
     const int nt = mmf_tok(grid, ntok);
-    if (nt < 1 || ncols >= MMF_MAX_COLS) return hipErrorInvalidValue;
+    if (nt < 1) return hipErrorInvalidValue;
     for (int64_t m0 = 0; m0 < M; m0 += (int64_t)nt * mr) {          // one launch as a rule
         const int m = (int)std::min<int64_t>(M - m0, (int64_t)nt * mr), n = (m + mr - 1) / mr;
         const dim3 g((unsigned)(grid / ntok * n));

@@ -249,9 +249,6 @@ void mmk_describe(const g4h_tensor &W, int M, char *buf, size_t len);
 void mmf_describe(int wtype, int64_t nrows, int64_t ncols, int M, char *buf, size_t len);
 // workgroups of one launch: HIP takes gridDim * blockDim below 2^32
 inline int64_t max_grid(int threads) { return 0xffffffffll / threads; }
-// columns of k_mm_float (32-bit byte offsets within a row); longer f16 / bf16 rows
-// take the GEMV family
-constexpr int64_t MMF_MAX_COLS = (int64_t)1 << 29;
 // x fp32 (quantized here into k_mmk_tile's layout, ws: M rows of 292 bytes per
 // superblock, 64-byte aligned): the bits of quantizing to q8_K rows first
 hipError_t launch_matmul_mfma_kx(const g4h_tensor &W, const float *x, size_t xs, int M, float *Y, uint8_t *ws, hipStream_t s);

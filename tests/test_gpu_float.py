@@ -246,3 +246,21 @@ def test_one_chunk_rows_cost_less_than_two(gpu):
         us.append(best)
         t.free()
     assert us[0] < 0.4 * us[1], us
+
+
+def test_rows_past_32_bit_offsets(gpu):
+    """A row of 2^29 + 16 columns: 1 GB of f16 weights, 2 GB of fp32 activations;
+    one value in the first piece and one in each of the last two."""
+    cols = (1 << 29) + 16
+    t = gpu.Tensor(1, cols, 1)
+    rows, x, y = gpu.Buffer(cols * 2), gpu.Buffer(cols * 4), gpu.Buffer(4)
+    w_at, x_at = {0: 1.5, cols - 20: 2.0, cols - 1: -3.0}, {0: 2.0, cols - 20: 5.0, cols - 1: 7.0}
+    rows.zero()
+    x.zero()
+    for i in w_at:
+        for b, v in ((rows, np.float16(w_at[i])), (x, np.float32(x_at[i]))):
+            a = np.array([v])
+            gpu.check(gpu.lib().g4h_memcpy_h2d(b.ptr + i * a.nbytes, a.ctypes.data, a.nbytes, None))
+    t.load_device(rows)
+    gpu.matmul(t, y, nb=1, x=x, path=2)
+    assert y.download(np.float32, (1,))[0] == 1.5 * 2.0 + 2.0 * 5.0 - 3.0 * 7.0
