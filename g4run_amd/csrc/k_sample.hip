@@ -355,46 +355,49 @@ __global__ __launch_bounds__(256) void k_sample_groups(SamplerDev *S, float *L, 
     else
         for (int q = 0; q < 4; q++) v[q] = i0 + q < nv ? L[i0 + q] : -INFINITY;
     const int m = ngram >= 2 && rn >= ngram ? (ngram - 1 < 64 ? ngram - 1 : 64) : 0;   // uniform
-    *(int4 *)&cnt[4 * t] = make_int4(0, 0, 0, 0);
-    if (t < 32) out[t] = 0;
-    if (t < m) suf[t] = ring_at(S, rn - m + t);
-    __syncthreads();
-    // f(i, id) for every i < n whose id lies in the slice
-    auto walk = [&](int n, auto &&id_at, auto &&f) {
-        for (int j0 = t; j0 < n; j0 += 8 * 256) {
-            int id[8];
+    const int nban = S->n_ban, nw = (rp != 1.0f || fp != 0 || pp != 0) && rln > 0 ? min(rln, rn) : 0;
+    if (nban || m || nw) {                                           // uniform
+        *(int4 *)&cnt[4 * t] = make_int4(0, 0, 0, 0);
+        if (t < 32) out[t] = 0;
+        if (t < m) suf[t] = ring_at(S, rn - m + t);
+        __syncthreads();
+        // f(i, id) for every i < n whose id lies in the slice
+        auto walk = [&](int n, auto &&id_at, auto &&f) {
+            for (int j0 = t; j0 < n; j0 += 8 * 256) {
+                int id[8];
 #pragma unroll
-            for (int q = 0; q < 8; q++) id[q] = j0 + 256 * q < n ? id_at(j0 + 256 * q) : -1;
+                for (int q = 0; q < 8; q++) id[q] = j0 + 256 * q < n ? id_at(j0 + 256 * q) : -1;
 #pragma unroll
-            for (int q = 0; q < 8; q++)
-                if (id[q] >= lo && id[q] < hi) f(j0 + 256 * q, id[q] - lo);
+                for (int q = 0; q < 8; q++)
+                    if (id[q] >= lo && id[q] < hi) f(j0 + 256 * q, id[q] - lo);
+            }
+        };
+        const int *ban = sampler_bans(S);
+        walk(nban, [&](int j) { return ban[j]; }, [&](int, int e) { atomicOr(&out[e >> 5], 1u << (e & 31)); });
+        if (m)
+            walk(rn - m, [&](int p) { return ring_at(S, p + m); }, [&](int p, int e) {
+                bool hit = true;
+                for (int j = 0; j < m && hit; j++) hit = ring_at(S, p + j) == suf[j];
+                if (hit) atomicOr(&out[e >> 5], 1u << (e & 31));
+            });
+        if (nw)
+            walk(nw, [&](int i) { return ring_at(S, rn - 1 - i); }, [&](int, int e) { atomicAdd(&cnt[e], 1); });
+        __syncthreads();
+        const uint32_t bits = out[t >> 3] >> (4 * (t & 7));
+        const int4 c4 = *(const int4 *)&cnt[4 * t];
+        const int c[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            if (bits >> q & 1) v[q] = -INFINITY;
+            if (c[q] > 0) {
+                float l = v[q];
+                if (rp != 1.0f) l = l <= 0 ? l * rp : l / rp;
+                const float fterm = (float)c[q] * fp;
+                l -= fterm + pp;
+                v[q] = l;
+            }
+            if ((bits >> q & 1) || c[q] > 0) L[i0 + q] = v[q];
         }
-    };
-    const int *ban = sampler_bans(S);
-    walk(S->n_ban, [&](int j) { return ban[j]; }, [&](int, int e) { atomicOr(&out[e >> 5], 1u << (e & 31)); });
-    if (m)
-        walk(rn - m, [&](int p) { return ring_at(S, p + m); }, [&](int p, int e) {
-            bool hit = true;
-            for (int j = 0; j < m && hit; j++) hit = ring_at(S, p + j) == suf[j];
-            if (hit) atomicOr(&out[e >> 5], 1u << (e & 31));
-        });
-    if ((rp != 1.0f || fp != 0 || pp != 0) && rln > 0)
-        walk(min(rln, rn), [&](int i) { return ring_at(S, rn - 1 - i); }, [&](int, int e) { atomicAdd(&cnt[e], 1); });
-    __syncthreads();
-    const uint32_t bits = out[t >> 3] >> (4 * (t & 7));
-    const int4 c4 = *(const int4 *)&cnt[4 * t];
-    const int c[4] = {c4.x, c4.y, c4.z, c4.w};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (bits >> q & 1) v[q] = -INFINITY;
-        if (c[q] > 0) {
-            float l = v[q];
-            if (rp != 1.0f) l = l <= 0 ? l * rp : l / rp;
-            const float fterm = (float)c[q] * fp;
-            l -= fterm + pp;
-            v[q] = l;
-        }
-        if ((bits >> q & 1) || c[q] > 0) L[i0 + q] = v[q];
     }
     uint32_t k = 0;
     bool nan = false;
@@ -511,37 +514,46 @@ __device__ bool gather_from_groups(const float *L, int nv, int ng, const uint32_
     __syncthreads();
     constexpr int LG = GS / 4;                                       // loads of 4 per group
     const int units = sh.gn * LG;                                    // uniform
-    int above = 0;
-    for (int u0 = 0; u0 < units; u0 += 4 * NT) {
-        float v[4][4];
-        int at[4];
+    // f(key, id, in the row) over the listed groups' elements, every lane of a
+    // wave in each call
+    auto each = [&](auto &&f) {
+        for (int u0 = 0; u0 < units; u0 += 4 * NT) {
+            float v[4][4];
+            int at[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int u = u0 + q * NT + t;
-            at[q] = u < units ? sh.glist[u / LG] * GS + 4 * (u % LG) : nv;
-            if (at[q] + 3 < nv) f4(*(const float4 *)(L + at[q]), v[q]);
-            else
-                for (int e = 0; e < 4; e++) v[q][e] = at[q] + e < nv ? L[at[q] + e] : 0.0f;
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t kk = okey(v[q][e]);
-                const bool keep = at[q] + e < nv && kk >= lo;
-                const uint64_t m = __ballot(keep);
-                if (m == 0) continue;                                // uniform
-                above += __builtin_popcountll(__ballot(keep && kk > lo));
-                int base = 0;
-                if (lane == 0) base = atomicAdd(&sh.gathered, __builtin_popcountll(m));
-                base = __shfl(base, 0, 64);
-                const int slot = base + __builtin_popcountll(m & ((1ull << lane) - 1));
-                if (keep && slot < GT) sh.keys[slot] = ((uint64_t)kk << 32) | (uint32_t)~(uint32_t)(at[q] + e);
+            for (int q = 0; q < 4; q++) {
+                const int u = u0 + q * NT + t;
+                at[q] = u < units ? sh.glist[u / LG] * GS + 4 * (u % LG) : nv;
+                if (at[q] + 3 < nv) f4(*(const float4 *)(L + at[q]), v[q]);
+                else
+                    for (int e = 0; e < 4; e++) v[q][e] = at[q] + e < nv ? L[at[q] + e] : 0.0f;
             }
-    }
-    if (lane == 0 && above) atomicAdd(&sh.above, above);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) f(okey(v[q][e]), at[q] + e, at[q] + e < nv);
+        }
+    };
+    each([&](uint32_t kk, int i, bool in) {
+        const bool keep = in && kk >= lo;
+        const uint64_t m = __ballot(keep);
+        if (m == 0) return;                                          // uniform
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&sh.gathered, __builtin_popcountll(m));
+        base = __shfl(base, 0, 64);
+        const int slot = base + __builtin_popcountll(m & ((1ull << lane) - 1));
+        if (keep && slot < GT) sh.keys[slot] = ((uint64_t)kk << 32) | (uint32_t)~(uint32_t)i;
+    });
     __syncthreads();
-    slow = tied ? sh.gathered < K1 : sh.gathered > GT && sh.above < K1;
+    if (tied) {
+        slow = sh.gathered < K1;
+    } else if (sh.gathered > GT) {                                   // uniform
+        int above = 0;
+        each([&](uint32_t kk, int, bool in) { above += __builtin_popcountll(__ballot(in && kk > lo)); });
+        if (lane == 0 && above) atomicAdd(&sh.above, above);
+        __syncthreads();
+        slow = sh.above < K1;
+    }
     return sh.gathered <= GT;
 }
 
